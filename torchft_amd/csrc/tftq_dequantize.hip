@@ -475,10 +475,99 @@ DEV void dequantize_small(const Seg &s, const KParams &p, int blk, int tid, uint
     }
 }
 
+// K_TILE: tensors whose columns are contiguous in memory (a transposed matrix).  A workgroup takes
+// a tile of 64 rows and 256 columns: the codes come in along the packed rows, 256 bytes each, wait
+// in LDS (rows of 65 dwords: neither the writes along a row nor the reads down a column share a
+// bank) and leave along the columns, 64 rows at a time (128 bytes of a 16-bit tensor).  A lane
+// reads one dword of codes of each of 8 (fp32: 4) rows and so holds 16 bytes of four columns.
+// Bound by memory: transposed [4096, 14336] and [4096, 4096] bf16, 227 MB, one element per lane and
+// access 443 us, this kernel 44.7 us (5.1 TB/s).
+template <typename T, bool POST>
+DEV void dequantize_tile(const Seg &s, const KParams &p, int blk, int tid, uint8_t *stage, float (*coef)[3])
+{
+    constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, RS = TFTQ_TILE_COLS / 4 + 1, G = TFTQ_TILE_ROWS / EPV;
+    static_assert(TFTQ_TILE_ROWS * RS * 4 <= TFTQ_D_STAGE, "a tile fits the stage");
+    LDS_AS u32 *codes = (LDS_AS u32 *)(LDS_AS uint8_t *)stage;
+    const int across = (s.n + TFTQ_TILE_COLS - 1) / TFTQ_TILE_COLS;
+    const int rb = blk / across, cb = blk - rb * across;
+    const int row0 = rb * TFTQ_TILE_ROWS, ndw = (s.row_bytes >> 2) - 1;
+    const int d0 = cb * (TFTQ_TILE_COLS / 4), nd = min(TFTQ_TILE_COLS / 4, ndw - d0);
+    const float inv = 1.0f / (float)s.slice_rows;
+    {
+        const int q = tid & 15;
+        const int dd = min(d0 + 4 * q, ndw - 4);  // the row's last vector is moved back to end with it (ndw > 4)
+        u32x4 w[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int row = min(row0 + 16 * t + (tid >> 4), s.m - 1);
+            w[t] = *((GLOBAL const u32x4_a4 *)(as_global<const u32>(p.packed + row_addr_fast(s, p.slot_size, row, inv)) + 1 + dd));
+        }
+        if (tid < TFTQ_TILE_ROWS) {
+            const int row = min(row0 + tid, s.m - 1);
+            const DivCoef c = make_div(as_f(*as_global<const u32>(p.packed + row_addr_fast(s, p.slot_size, row, inv))));
+            coef[tid][0] = c.r;
+            coef[tid][1] = c.r_lo;
+            coef[tid][2] = c.s;
+        }
+        if (4 * q < nd) {
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (dd - d0 + e >= 0) codes[(16 * t + (tid >> 4)) * RS + dd - d0 + e] = w[t][e];
+        }
+    }
+    __syncthreads();
+    // whole 64-byte blocks leave with streaming stores, others are put together in the L2
+    const bool fill = ((s.ptr | (uint64_t)(s.col_stride * ESZ)) & 63u) == 0;
+    const int g = tid & (G - 1);
+    const int r0 = row0 + g * EPV;
+    if (r0 >= s.m) return;
+    float r[EPV], r_lo[EPV];
+    bool fast = true;
+#pragma unroll
+    for (int i = 0; i < EPV; i++) {
+        r[i] = coef[g * EPV + i][0];
+        r_lo[i] = coef[g * EPV + i][1];
+        fast = fast && scale_is_fast(coef[g * EPV + i][2]);
+    }
+#pragma nounroll
+    for (int k = tid / G; k < nd; k += TFTQ_WG / G) {
+        float o[4][EPV];
+#pragma unroll
+        for (int i = 0; i < EPV; i++) {
+            float f[4];
+            unpack_fp8x4(codes[(g * EPV + i) * RS + k], f);
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e][i] = fin<T, POST>(div_fast_signed(f[e], r[i], r_lo[i]), p);
+            if (!fast) {
+                const float sc = coef[g * EPV + i][2];
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e][i] = fin<T, POST>(f[e] / sc, p);  // :250-252
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t c = 4 * (d0 + k) + e;
+            if (c >= s.n) break;
+            const uint64_t at = s.ptr + (uint64_t)((r0 + c * s.col_stride) * ESZ);
+            if (r0 + EPV <= s.m) {
+                if (fill) STORE_STREAM(Elem<T>::pack(o[e]), as_global<u32x4_a2>(at));
+                else *as_global<u32x4_a2>(at) = Elem<T>::pack(o[e]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < EPV; i++)
+                    if (r0 + i < s.m) Elem<T>::store(at, i, o[e][i]);
+            }
+        }
+    }
+}
+
 template <typename T, bool INLINE, bool POST>
 __global__ __launch_bounds__(TFTQ_WG) void k_dequantize(const KParams p, const InlineTable inl)
 {
     __shared__ __align__(16) uint8_t stage[TFTQ_D_STAGE];  // see copy_out_span
+    __shared__ float coef[TFTQ_TILE_ROWS][3];
     Seg s;
     int vb;
     if (!locate<INLINE, ST_D>(p, inl, s, vb)) return;
@@ -500,6 +589,7 @@ __global__ __launch_bounds__(TFTQ_WG) void k_dequantize(const KParams p, const I
         if (s.m > 0) dequantize_col1<T, POST>(s, p, blk * tftq_col1_rows_per_wg(ST_D), tid);
         break;
     case K_VECS: dequantize_small<T, POST>(s, p, blk, tid, stage); break;
+    case K_TILE: dequantize_tile<T, POST>(s, p, blk, tid, stage, coef); break;
     default: break;
     }
 }

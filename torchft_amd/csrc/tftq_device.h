@@ -327,6 +327,18 @@ template <> struct Elem<f16_tag> {
     }
 };
 
+// The elements in one dword of a tensor: one (fp32) or two.
+template <typename T>
+DEV void unpack_dword(u32 w, float (&f)[4 / Elem<T>::ESZ])
+{
+    if constexpr (std::is_same<T, float>::value) f[0] = as_f(w);
+    else if constexpr (std::is_same<T, f16_tag>::value) Elem<T>::unpack2(w, f[0], f[1]);
+    else {
+        f[0] = as_f(w << 16);
+        f[1] = as_f(w & 0xFFFF0000u);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // workgroup -> (segment, first row)
 // ---------------------------------------------------------------------------
@@ -553,10 +565,10 @@ __attribute__((visibility("hidden"))) int tftq_static_table_setup(void);
 // One kernel launch with the launch's own error (not whatever an earlier call left behind).
 template <typename K>
 static inline int launch_kernel(K kernel, unsigned grid, unsigned lds_bytes, hipStream_t st, const KParams &kp,
-                                const InlineTable &inl)
+                                const InlineTable &inl, int threads = TFTQ_WG)
 {
     void *args[2] = {(void *)&kp, (void *)&inl};
-    return (int)hipLaunchKernel((const void *)kernel, dim3(grid), dim3(TFTQ_WG), args, lds_bytes, st);
+    return (int)hipLaunchKernel((const void *)kernel, dim3(grid), dim3(threads), args, lds_bytes, st);
 }
 
 // Kernel parameters of one call.  tensors: host array of the tensors' device addresses (null

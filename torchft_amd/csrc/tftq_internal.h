@@ -8,8 +8,10 @@
 
 #include "../../include/tftq.h"
 
-// Stages of the path, used to index per-stage fields of a segment.
-enum : int { ST_Q = 0, ST_R = 1, ST_D = 2 };
+// Stages of the path, used to index per-stage fields of a segment.  ST_QC: the second launch of
+// quantize, for the tensors stored column by column (K_COLS); a tensor belongs to one of the two
+// launches, so it is numbered by wg_begin[ST_Q] and kind[ST_Q] in either.
+enum : int { ST_Q = 0, ST_R = 1, ST_D = 2, ST_QC = 3, N_LAUNCHES = 4 };
 
 // How the rows of one tensor are mapped onto lanes.  "Team" = the lanes that
 // cooperate on one row.  VEC kinds (quantize, dequantize) need rows that are
@@ -34,6 +36,8 @@ enum : uint8_t {
     K_GEN64 = 6,   // one wavefront per row
     K_GEN256 = 7,  // one workgroup per row (reduce only)
     K_COL1 = 8,    // rows of a single column (1-D tensors): 4 rows per lane, 1024 per workgroup
+    K_COLS = 17,   // columns contiguous in memory (row stride 1: a transposed matrix), quantize: a workgroup of 512 lanes per 16 (fp32: 8) rows
+    K_TILE = 18,   // the same in dequantize: a workgroup per tile of 64 rows and 256 columns
 };
 
 // Helpers shared by the planner (host compiler) and the kernels (hipcc).
@@ -59,7 +63,15 @@ TFTQ_HD static inline int tftq_team_of(uint8_t kind)
     }
 }
 
-constexpr int TFTQ_WG = 256;       // threads per workgroup, all kernels
+constexpr int TFTQ_WG = 256;       // threads per workgroup, all kernels but k_quantize_cols
+
+// K_COLS (k_quantize_cols): TFTQ_QC_WG lanes hold TFTQ_QC_GROUPS groups of rows, 16 bytes of a
+// column each.  The blocks of a tensor start at the slots' first rows, so a block's packed rows
+// are neighbours.
+constexpr int TFTQ_QC_WG = 512, TFTQ_QC_GROUPS = 2;
+TFTQ_HD static inline int tftq_qc_rows(int esz) { return TFTQ_QC_GROUPS * (16 / esz); }
+// K_TILE
+constexpr int TFTQ_TILE_ROWS = 64, TFTQ_TILE_COLS = 256;
 
 // Reduce, teams of 64 or 256 lanes: a lane has 8 loads of 16 bytes in flight
 // when the group has 8 peers.  With fewer peers a team works on 2 or 4
@@ -166,6 +178,8 @@ static_assert(sizeof(Seg) == 64, "Seg must be 64 bytes");
 static inline int tftq_rows_per_wg(const Seg &s, int st, int esz, int ws)
 {
     if (s.kind[st] == K_COL1) return tftq_col1_rows_per_wg(st);
+    if (s.kind[st] == K_COLS) return tftq_qc_rows(esz);
+    if (s.kind[st] == K_TILE) return TFTQ_TILE_ROWS;
     if (s.kind[st] == K_VECS) return tftq_small_rows_per_wg(tftq_small_nvec(s.n, esz), st);
     const int teams = TFTQ_WG / tftq_team_of(s.kind[st]);
     if (st == ST_R) return teams * tftq_reduce_rows_at_once(s.kind[st], s.row_bytes / 4 - 1, ws);
@@ -193,7 +207,9 @@ TFTQ_HD static inline int tftq_d_part_begin(int nvec, int parts, int part)
 static inline int64_t tftq_wgs_of(const Seg &s, int st, int esz, int ws, int64_t rows)
 {
     const int per_wg = tftq_rows_per_wg(s, st, esz, ws);
+    if (s.kind[st] == K_COLS) return (int64_t)ws * ((s.slice_rows + per_wg - 1) / per_wg);
     const int64_t wgs = (rows + per_wg - 1) / per_wg;
+    if (s.kind[st] == K_TILE) return wgs * ((s.n + TFTQ_TILE_COLS - 1) / TFTQ_TILE_COLS);
     return st == ST_D ? wgs * tftq_d_row_parts(s.kind[ST_D], s.n, esz) : wgs;
 }
 
@@ -260,14 +276,15 @@ struct tftq_plan {
     int64_t slot_size;
     int64_t output_size;
     int64_t max_rows;
-    int32_t nwg[3];
+    int32_t nwg[N_LAUNCHES];
     bool wide[3];              // per stage: some row needs the kernel variant with more registers
     bool reduce_long_rows;     // every row of the list runs in a team of 64 or 256 lanes in reduce or has one column (k_reduce's R_LONG)
     int parked;                // quantize: groups of 5 vectors per lane (20 KB of LDS each, up to 3) that the longest row parks in LDS (rows above TFTQ_Q_VECS_WIDE)
-    Dealt dealt[3];            // inline table only
-    int32_t dealt_per_xcd[3];  // inline table only: workgroups of the busiest XCD
-    bool natural[3];           // inline table only: workgroup ids keep their order (see deal_to_xcds)
-    TableIndex index[3];       // device table only
+    int cols_most;             // quantize: columns of the widest K_COLS tensor
+    Dealt dealt[N_LAUNCHES];   // inline table only
+    int32_t dealt_per_xcd[N_LAUNCHES];  // inline table only: workgroups of the busiest XCD
+    bool natural[N_LAUNCHES];  // inline table only: workgroup ids keep their order (see deal_to_xcds)
+    TableIndex index[N_LAUNCHES];  // device table only
     std::vector<Seg> segs;
     std::vector<uint8_t> blob;  // host image of the device table (nseg > TFTQ_N_INLINE)
 };

@@ -83,6 +83,7 @@ static uint8_t pick_io_kind(const Seg &s, int esz)
         return K_VEC256;  // longer than 32 KB: two passes inside the workgroup
     }
     if (s.n <= 16) return K_GEN1;
+    if (s.row_stride == 1 && s.m >= epv) return K_COLS;
     if (s.n <= 128) return K_GEN8;
     return K_GEN64;
 }
@@ -94,6 +95,7 @@ static uint8_t pick_io_kind(const Seg &s, int esz)
 static uint8_t pick_d_kind(const Seg &s, int esz)
 {
     const uint8_t k = pick_io_kind(s, esz);
+    if (k == K_COLS) return K_TILE;
     const int64_t rowb = (int64_t)s.n * esz;
     if (k != K_VEC8 && k != K_VEC16 && k != K_VEC32 && k != K_VEC64 && k != K_VEC256) return k;
     if (s.row_stride != s.n || (rowb & 63) == 0 || rowb > 16384) {
@@ -190,7 +192,7 @@ static void work_order(const tftq_plan *p, int st, std::vector<int32_t> &ord)
 // its heaviest-first order is built on.
 static bool natural_order(const tftq_plan *p, int st)
 {
-    if (st == ST_R) return false;
+    if (st == ST_R || st == ST_QC) return false;
     double whole = 0.0, all = 0.0;
     for (int i = 0; i < p->nseg; i++) {
         const Seg &s = p->segs[(size_t)i];
@@ -208,12 +210,14 @@ static bool natural_order(const tftq_plan *p, int st)
 // dealt round-robin to the 8 XCDs by the hardware; here every XCD takes a
 // contiguous eighth of every segment, so all XCDs see the same mix of row
 // lengths, and works through the segments in work_order().
-static void deal_to_xcds(tftq_plan *p, const int32_t (*wgs)[3])
+static void deal_to_xcds(tftq_plan *p, const int32_t (*wgs)[N_LAUNCHES])
 {
-    for (int st = 0; st < 3; st++) {
+    for (int st = 0; st < N_LAUNCHES; st++) {
+        const int field = st == ST_QC ? ST_Q : st;
         int32_t begin = 0;
         for (int i = 0; i < p->nseg; i++) {  // workgroup numbers in list order
-            p->segs[(size_t)i].wg_begin[st] = begin;
+            if (st == ST_QC && wgs[i][st] == 0) continue;  // numbered for ST_Q
+            p->segs[(size_t)i].wg_begin[field] = begin;
             begin += wgs[i][st];
         }
         std::vector<int32_t> ord;
@@ -235,7 +239,7 @@ static void deal_to_xcds(tftq_plan *p, const int32_t (*wgs)[3])
                 // natural order: every row of the table covers all workgroups of every segment
                 const int64_t lo = p->natural[st] ? 0 : (int64_t)((n * (uint64_t)x) >> 3);
                 const int64_t hi = p->natural[st] ? (int64_t)n : (int64_t)((n * (uint64_t)(x + 1)) >> 3);
-                d.base[x][k] = (int32_t)(p->segs[(size_t)i].wg_begin[st] + lo - cum);
+                d.base[x][k] = (int32_t)(p->segs[(size_t)i].wg_begin[field] + lo - cum);
                 d.seg[x][k] = i;
                 cum += hi - lo;
                 d.cum_end[x][k] = (int32_t)cum;
@@ -247,12 +251,13 @@ static void deal_to_xcds(tftq_plan *p, const int32_t (*wgs)[3])
 }
 
 // Many segments: the image of the device table (layout in tftq_internal.h).
-static int build_table(tftq_plan *p, const int32_t (*wgs)[3])
+static int build_table(tftq_plan *p, const int32_t (*wgs)[N_LAUNCHES])
 {
     const size_t nseg = (size_t)p->nseg;
-    std::vector<SortEnt> sorted[3];
-    std::vector<MapEnt> map[3];
-    for (int st = 0; st < 3; st++) {
+    std::vector<SortEnt> sorted[N_LAUNCHES];
+    std::vector<MapEnt> map[N_LAUNCHES];
+    const int launches = p->nwg[ST_QC] ? N_LAUNCHES : 3;  // no index for a launch that no tensor needs
+    for (int st = 0; st < launches; st++) {
         std::vector<int32_t> ord;
         work_order(p, st, ord);
         sorted[st].resize(nseg);
@@ -264,7 +269,8 @@ static int build_table(tftq_plan *p, const int32_t (*wgs)[3])
             const Seg &sg = p->segs[(size_t)i];
             if (pieces && tftq_reduce_kind_has_barriers(sg.kind[st])) begin = (begin + 3) & ~(int64_t)3;
             if (begin > INT32_MAX - 4096) return TFTQ_E_SHAPE;
-            p->segs[(size_t)i].wg_begin[st] = (int32_t)begin;
+            if (st != ST_QC) p->segs[(size_t)i].wg_begin[st] = (int32_t)begin;
+            else if (wgs[i][st]) p->segs[(size_t)i].wg_begin[ST_Q] = (int32_t)begin;
             sorted[st][k] = SortEnt{(int32_t)begin, i};
             begin += pieces ? tftq_reduce_pieces(sg, p->esz, p->ws, wgs[i][st]) : wgs[i][st];
         }
@@ -295,17 +301,17 @@ static int build_table(tftq_plan *p, const int32_t (*wgs)[3])
         p->index[st].per_xcd = (int32_t)(turns << cs);
     }
     size_t bytes = nseg * sizeof(Seg);
-    for (int st = 0; st < 3; st++) {
+    for (int st = 0; st < launches; st++) {
         p->index[st].sorted_off = (int64_t)bytes;
         bytes += nseg * sizeof(SortEnt);
     }
-    for (int st = 0; st < 3; st++) {
+    for (int st = 0; st < launches; st++) {
         p->index[st].map_off = (int64_t)bytes;
         bytes += map[st].size() * sizeof(MapEnt);
     }
     p->blob.resize(bytes);
     memcpy(p->blob.data(), p->segs.data(), nseg * sizeof(Seg));
-    for (int st = 0; st < 3; st++) {
+    for (int st = 0; st < launches; st++) {
         memcpy(p->blob.data() + p->index[st].sorted_off, sorted[st].data(), nseg * sizeof(SortEnt));
         memcpy(p->blob.data() + p->index[st].map_off, map[st].data(), map[st].size() * sizeof(MapEnt));
     }
@@ -332,7 +338,7 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
     try {  // nothing may throw across the C ABI
         p->segs.resize((size_t)n_tensors);
         offs.resize((size_t)n_tensors);
-        wgs_flat.resize((size_t)n_tensors * 3);
+        wgs_flat.resize((size_t)n_tensors * N_LAUNCHES);
     } catch (...) {
         delete p;
         return TFTQ_E_NOMEM;
@@ -342,8 +348,8 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         delete p;
         return rc;
     }
-    int64_t wg[3] = {0, 0, 0};
-    int32_t (*wgs)[3] = (int32_t (*)[3])wgs_flat.data();  // workgroups per segment and stage
+    int64_t wg[N_LAUNCHES] = {0, 0, 0, 0};
+    int32_t (*wgs)[N_LAUNCHES] = (int32_t (*)[N_LAUNCHES])wgs_flat.data();  // workgroups per segment and launch
     for (int i = 0; i < n_tensors; i++) {
         Seg &s = p->segs[(size_t)i];
         memset(&s, 0, sizeof(s));
@@ -364,18 +370,20 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         const int64_t rows[3] = {m_pad, s.slice_rows, s.m};
         for (int st = 0; st < 3; st++) {
             const int64_t n = tftq_wgs_of(s, st, p->esz, ws, rows[st]);
-            wgs[i][st] = (int32_t)n;
-            wg[st] += n;
-            if (wg[st] > INT32_MAX - 4096) {
+            const int launch = s.kind[st] == K_COLS ? ST_QC : st;
+            wgs[i][st] = 0;
+            wgs[i][launch] = (int32_t)n;
+            wg[launch] += n;
+            if (wg[launch] > INT32_MAX - 4096) {
                 delete p;
                 return TFTQ_E_SHAPE;
             }
         }
+        if (s.kind[ST_Q] == K_COLS) p->cols_most = std::max(p->cols_most, s.n);
     }
-    for (int st = 0; st < 3; st++) p->nwg[st] = (int32_t)wg[st];
+    for (int st = 0; st < N_LAUNCHES; st++) p->nwg[st] = (int32_t)wg[st];
     p->wide[ST_Q] = p->wide[ST_R] = p->wide[ST_D] = false;
     p->parked = 0;
-    p->natural[ST_Q] = p->natural[ST_R] = p->natural[ST_D] = false;
     p->reduce_long_rows = true;
     for (int i = 0; i < n_tensors; i++) {
         const Seg &s = p->segs[(size_t)i];
@@ -400,9 +408,9 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         return TFTQ_E_NOMEM;
     }
     // a grid has fewer than 2^32 threads
-    for (int st = 0; st < 3; st++) {
+    for (int st = 0; st < N_LAUNCHES; st++) {
         const int64_t per_xcd = p->nseg <= TFTQ_N_INLINE ? p->dealt_per_xcd[st] : p->index[st].per_xcd;
-        if (8 * per_xcd * TFTQ_WG > (int64_t)UINT32_MAX) {
+        if (8 * per_xcd * (st == ST_QC ? TFTQ_QC_WG : TFTQ_WG) > (int64_t)UINT32_MAX) {
             delete p;
             return TFTQ_E_SHAPE;
         }

@@ -609,6 +609,168 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize(const KParam
     }
 }
 
+// ---------------------------------------------------------------------------
+// quantize, tensors whose columns are contiguous in memory (K_COLS)
+// ---------------------------------------------------------------------------
+// A transposed matrix: a row's elements are a whole column length apart, a column's lie side by
+// side.  A lane takes 16 bytes of a column, 8 (fp32: 4) rows, of four neighbouring columns: it then
+// holds one dword of codes of each of these rows, and the 32 lanes that share its rows write 128
+// neighbouring bytes of a packed row with one store, with no exchange between lanes.  Only the row
+// maxima go through LDS.  A block of 16 (fp32: 8) rows stays in the registers of a workgroup of 512
+// lanes, up to NS steps of 1024 columns, so that the tensor is read once; what a row has beyond
+// that is read twice.  Bound by the L1's requests in flight, which are 32 bytes each here (HBM
+// traffic is the algorithmic 1.0 times): transposed [4096, 14336] and [4096, 4096] bf16, 227 MB,
+// one element per lane and access and two passes 486 us, this kernel 79 us.  Alone, [4096, 14336]
+// 65.7 us: with blocks of 32 rows 101 (half the compute units idle), workgroups of 256 lanes 89
+// (half of the row read twice), of 1024 lanes 72, streaming loads 77 (neighbouring blocks share
+// lines); a launch for the maxima and one for tiles of 64 rows 82 us.
+template <typename T, int NS>
+DEV void quantize_cols(const Seg &s, const KParams &p, int blk, int tid, float *part, float *scale)
+{
+    constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, G = TFTQ_QC_GROUPS, K = 64 / G, RB = G * EPV;
+    constexpr int WAVES = TFTQ_QC_WG / 64, STEP = 4 * K * WAVES;  // columns per step
+    constexpr int RPD = 4 / ESZ;                                  // rows per dword of a column
+    const int per_slot = (s.slice_rows + RB - 1) / RB;
+    const int slot = blk / per_slot;
+    const int j0 = (blk - slot * per_slot) * RB;
+    const int srow = slot * s.slice_rows;  // the slot's first row
+    const int real = min(max(s.m - srow, 0), s.slice_rows);
+    GLOBAL uint8_t *g0 = as_global<uint8_t>(p.packed + (int64_t)slot * p.slot_size + s.slot_off + (int64_t)j0 * s.row_bytes);
+    {   // padding rows: zero (:93-95 on a zero-filled buffer)
+        const int z0 = max(real - j0, 0), z1 = min(RB, s.slice_rows - j0);
+        for (int z = z0; z < z1; z++)
+            for (int d = tid; d < (s.row_bytes >> 2); d += TFTQ_QC_WG) ((GLOBAL u32 *)(g0 + (int64_t)z * s.row_bytes))[d] = 0;
+    }
+    if (j0 >= real) return;  // the whole workgroup
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+    const int g = l & (G - 1), k = l / G;
+    const int ndw = (s.row_bytes >> 2) - 1;
+    // the lane's rows; the last group of the tensor is moved back to end with it (its rows are
+    // another lane's too: both write the same bytes)
+    const int first = min(srow + j0 + g * EPV, s.m - EPV);
+    const int jf = first - srow - j0, jstop = min(RB, real - j0);  // rows jf + i in [0, jstop) are written
+    const uint64_t col0 = s.ptr + (uint64_t)((int64_t)first * ESZ);
+    const int64_t cs = s.col_stride * ESZ;
+    const int c0 = 4 * (wave * K + k);
+    auto load = [&](u32x4 (&v)[4], int base) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)  // columns past the last one re-read it
+            v[e] = *as_global<const u32x4_a2>(col0 + (uint64_t)((int64_t)min(base + c0 + e, s.n - 1) * cs));
+    };
+    float amax[EPV];
+#pragma unroll
+    for (int i = 0; i < EPV; i++) amax[i] = 0.0f;
+    auto maxima = [&](const u32x4 (&v)[4]) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float f[EPV];
+            Elem<T>::unpack(v[e], f);
+#pragma unroll
+            for (int i = 0; i < EPV; i++) amax[i] = fmaxf(amax[i], __builtin_fabsf(f[i]));
+        }
+    };
+    u32x4 v[NS][4];
+#pragma unroll
+    for (int t = 0; t < NS; t++) load(v[t], t * STEP);
+#pragma unroll
+    for (int t = 0; t < NS; t++) maxima(v[t]);
+#pragma nounroll
+    for (int base = NS * STEP; base < s.n; base += STEP) {  // first pass over the rest
+        u32x4 x[4];
+        load(x, base);
+        maxima(x);
+    }
+#pragma unroll
+    for (int i = 0; i < EPV; i++) {  // over the lanes of the same parity in a row of 16
+        amax[i] = fmaxf(amax[i], dpp_mov<0x128>(amax[i]));  // row_ror:8
+        amax[i] = fmaxf(amax[i], dpp_mov<0x124>(amax[i]));  // row_ror:4
+        amax[i] = fmaxf(amax[i], dpp_mov<0x122>(amax[i]));  // row_ror:2
+        if ((l & 15) < G) part[(wave * 4 + (l >> 4)) * RB + g * EPV + i] = amax[i];
+    }
+    static_assert(G == 2, "the rotations above");
+    __syncthreads();
+    if (tid < RB) {
+        float a = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4 * WAVES; w++) a = fmaxf(a, part[w * RB + tid]);
+        const float sc = calc_scale(a);
+        scale[tid] = sc;
+        const int j = min(srow + j0 + tid / EPV * EPV, s.m - EPV) - srow - j0 + tid % EPV;
+        if (j >= 0 && j < jstop) *(GLOBAL u32 *)(g0 + (int64_t)j * s.row_bytes) = as_u(sc);
+    }
+    __syncthreads();
+    float sc[EPV];
+#pragma unroll
+    for (int i = 0; i < EPV; i++) sc[i] = scale[g * EPV + i];
+    GLOBAL uint8_t *out = g0 + (int64_t)jf * s.row_bytes + 4;
+    auto store = [&](const u32x4 (&v)[4], int base) {
+        const int d = (base + c0) >> 2;  // the lane's dword of the payload
+        if (d >= ndw) return;
+        const int over = 4 * d + 4 - s.n;  // columns of the dword past the last one
+        const u32 mask = over > 0 ? 0xFFFFFFFFu >> (8 * over) : 0xFFFFFFFFu;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {  // dword w of the four vectors: rows RPD * w ...
+            float f[4][RPD];
+#pragma unroll
+            for (int e = 0; e < 4; e++) unpack_dword<T>(v[e][w], f[e]);
+#pragma unroll
+            for (int h = 0; h < RPD; h++) {
+                const int i = RPD * w + h;
+                const u32 o = pack_fp8x4(f[0][h] * sc[i], f[1][h] * sc[i], f[2][h] * sc[i], f[3][h] * sc[i]) & mask;
+                // plain stores: a packed row starts anywhere in its line, the L2 puts the runs together
+                if (jf + i >= 0 && jf + i < jstop) ((GLOBAL u32 *)(out + (int64_t)i * s.row_bytes))[d] = o;
+            }
+        }
+    };
+#pragma unroll
+    for (int t = 0; t < NS; t++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) asm volatile("" : "+v"(v[t][e].x), "+v"(v[t][e].y), "+v"(v[t][e].z), "+v"(v[t][e].w));
+    }
+#pragma unroll
+    for (int t = 0; t < NS; t++) store(v[t], t * STEP);
+#pragma nounroll
+    for (int base = NS * STEP; base < s.n; base += STEP) {  // second pass over the rest
+        u32x4 x[4];
+        load(x, base);
+        store(x, base);
+    }
+}
+
+// Steps that stay in registers: 12 for lists with rows of more than 4096 columns (250 registers, two
+// wavefronts per SIMD; 14 spill), else 4 (114 registers, four).
+constexpr int QC_MOST = 12;
+constexpr int QC_STEP = 4 * (64 / TFTQ_QC_GROUPS) * (TFTQ_QC_WG / 64);
+template <typename T, bool INLINE, int NSMAX>
+__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols(const KParams p, const InlineTable inl)
+{
+    __shared__ float part[4 * TFTQ_QC_WG / 64 * TFTQ_QC_GROUPS * Elem<T>::EPV];
+    __shared__ float scale[TFTQ_QC_GROUPS * Elem<T>::EPV];
+    Seg s;
+    int vb;
+    if (!locate<INLINE, ST_Q>(p, inl, s, vb)) return;
+    const int blk = vb - s.wg_begin[ST_Q];
+    const int tid = threadIdx.x;
+    const int steps = (s.n + QC_STEP - 1) / QC_STEP;  // same for the whole workgroup
+    if (steps <= 1) quantize_cols<T, 1>(s, p, blk, tid, part, scale);
+    else if (steps <= 2) quantize_cols<T, 2>(s, p, blk, tid, part, scale);
+    else if (NSMAX == 4 || steps <= 4) quantize_cols<T, 4>(s, p, blk, tid, part, scale);
+    else if (steps <= 8) quantize_cols<T, NSMAX == 4 ? 4 : 8>(s, p, blk, tid, part, scale);
+    else quantize_cols<T, NSMAX>(s, p, blk, tid, part, scale);
+}
+
+template <typename T>
+static int launch_qc(const KParams &kp, const InlineTable &inl, bool use_inline, int most, hipStream_t st)
+{
+    const unsigned grid = grid_of(kp);
+    if (most > 4 * QC_STEP) {
+        if (use_inline) return launch_kernel(k_quantize_cols<T, true, QC_MOST>, grid, 0, st, kp, inl, TFTQ_QC_WG);
+        return launch_kernel(k_quantize_cols<T, false, QC_MOST>, grid, 0, st, kp, inl, TFTQ_QC_WG);
+    }
+    if (use_inline) return launch_kernel(k_quantize_cols<T, true, 4>, grid, 0, st, kp, inl, TFTQ_QC_WG);
+    return launch_kernel(k_quantize_cols<T, false, 4>, grid, 0, st, kp, inl, TFTQ_QC_WG);
+}
+
 template <typename T>
 static int launch_q(const KParams &kp, const InlineTable &inl, bool use_inline, bool wide, int parked,
                     hipStream_t st)
@@ -633,13 +795,27 @@ extern "C" int tftq_quantize(const tftq_plan *plan, const void *const *tensors, 
     hipStream_t st = (hipStream_t)stream;
     DeviceScope scope(device);
     if (scope.err != hipSuccess) return (int)scope.err;
-    int rc = fill_params(plan, ST_Q, tensors, table, pointers, packed, packed_bytes, st, &kp, &inl, &use_inline);
+    if (!plan) return TFTQ_E_ARG;
+    const bool only_cols = plan->nwg[ST_Q] == 0 && plan->nwg[ST_QC] != 0;
+    int rc = fill_params(plan, only_cols ? ST_QC : ST_Q, tensors, table, pointers, packed, packed_bytes, st, &kp, &inl,
+                         &use_inline);
     if (rc) return rc;
-    if (kp.nwg == 0) return 0;
+    if (kp.nwg != 0 && !only_cols) {
+        switch (plan->dtype) {
+        case TFTQ_F32: rc = launch_q<float>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st); break;
+        case TFTQ_F16: rc = launch_q<f16_tag>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st); break;
+        case TFTQ_BF16: rc = launch_q<bf16_tag>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st); break;
+        default: return TFTQ_E_DTYPE;
+        }
+        if (rc) return rc;
+    }
+    if (plan->nwg[ST_QC] == 0) return 0;
+    kp.nwg = plan->nwg[ST_QC];
+    work_mapping(plan, ST_QC, &kp);
     switch (plan->dtype) {
-    case TFTQ_F32: return launch_q<float>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st);
-    case TFTQ_F16: return launch_q<f16_tag>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st);
-    case TFTQ_BF16: return launch_q<bf16_tag>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st);
+    case TFTQ_F32: return launch_qc<float>(kp, inl, use_inline, plan->cols_most, st);
+    case TFTQ_F16: return launch_qc<f16_tag>(kp, inl, use_inline, plan->cols_most, st);
+    case TFTQ_BF16: return launch_qc<bf16_tag>(kp, inl, use_inline, plan->cols_most, st);
     default: return TFTQ_E_DTYPE;
     }
 }
