@@ -1,0 +1,118 @@
+"""DiLoCo's bucketised all-reduce with kernels that work on the tensors in place, against the same
+step by way of copies into and out of the flat buffer, by bytes."""
+
+import pytest
+import torch
+from torch.distributed import ReduceOp
+
+from sim_pg import SimGroup
+from test_gpu_collectives import run_ranks
+from torchft_amd import allreduce as ar
+
+
+def refused(kind, t):
+    """`t` as a tensor that only a copy can take, and the piece of a flat buffer it belongs to"""
+    piece = torch.zeros(t.numel()).view_as(t)
+    if kind == "strided":
+        return t.t().contiguous().t(), piece
+    if kind == "dtype":
+        return t.to(torch.bfloat16), piece
+    if kind == "autograd":
+        return t.requires_grad_(), piece
+    if kind == "shape":
+        return t[:1], piece
+    if kind == "subclass":
+        return t.as_subclass(type("Other", (torch.Tensor,), {})), piece
+    if kind == "negated":
+        return torch._neg_view(t), piece
+    return t, piece
+
+
+@pytest.mark.parametrize("kind", ["strided", "dtype", "autograd", "shape", "subclass", "negated", "plain"])
+def test_what_only_a_copy_can_take(kind):
+    plain = torch.ones(3, 4)
+    t, piece = refused(kind, torch.ones(3, 4))
+    got = ar._addresses([plain, t], [torch.zeros(3, 4), piece])
+    assert got == ([plain.data_ptr(), t.data_ptr()] if kind == "plain" else None)
+    with torch.autograd.forward_ad.dual_level():
+        assert ar._addresses([plain], [torch.zeros(3, 4)]) is None
+
+
+def step(peers, ws, dtype, capacity, op, way, monkeypatch):
+    """Two steps on copies of the peers' tensors; what every rank holds after each"""
+    group, seen = SimGroup(ws), [[] for _ in range(ws)]
+    mine = [[t.cuda() for t in tensors] for tensors in peers]
+    if way == "copies":
+        monkeypatch.setattr(ar.BucketizedAllreduce, "_in_place", lambda self, bucket, whole: None)
+    if way == "aliased":  # two tensors of one storage, on both ways the same
+        for tensors in mine:
+            tensors[2] = tensors[3][:tensors[2].numel()].view_as(tensors[2])
+    averaging = [ar.BucketizedAllreduce(tensors, capacity * tensors[0].element_size()) for tensors in mine]
+
+    def rank_fn(r):
+        for _ in range(2):
+            works = averaging[r].allreduce(group.rank(r), ws, reduce_op=op)
+            assert all(w.wait() and w.get_future().value() == [] for w in works)
+            seen[r].append([t.clone() for t in mine[r]])
+            for t in mine[r]:
+                t.data = t * 0.5  # storage of its own for the second step
+
+    run_ranks(ws, rank_fn, group)
+    torch.cuda.synchronize()
+    monkeypatch.undo()
+    return seen, averaging
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", [ReduceOp.SUM, ReduceOp.AVG])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ws,sizes,capacity", [
+    (2, [(64, 48), (1,), (7, 33), (2049,), (0,), (3, 1)], 1 << 20),   # one buffer; odd starts
+    (3, [(2047,), (5, 5), (1, 1), (4096, 3)], 1 << 20),               # padding rows
+    (4, [(6,), (6,), (6,), (6,)], 8),                                 # buffers with a rest that no tensor covers
+    (5, [(k % 7 + 1, 2 * k + 1) for k in range(40)], 1 << 20),        # addresses that travel through device memory
+    (1, [(1025,)], 1 << 20),
+])
+def test_in_place_step_has_the_bytes_of_the_copies(monkeypatch, dtype, ws, sizes, capacity, op):
+    g = torch.Generator().manual_seed(len(sizes))
+    peers = [[(torch.randn(s, generator=g) * 0.1).to(dtype) for s in sizes] for _ in range(ws)]
+    got, averaging = step(peers, ws, dtype, capacity, op, "in place", monkeypatch)
+    assert all(b["piecewise"] for a in averaging for b in a.buckets if b["owners"])
+    want, averaging = step(peers, ws, dtype, capacity, op, "copies", monkeypatch)
+    assert not any(b["piecewise"] for a in averaging for b in a.buckets)
+    for r in range(ws):
+        for k in range(2):
+            for i, (a, b) in enumerate(zip(got[r][k], want[r][k])):
+                assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8)), (r, k, sizes[i])
+
+
+@pytest.mark.gpu
+def test_shared_memory_and_storage_that_moves_in_flight(monkeypatch):
+    g = torch.Generator().manual_seed(3)
+    peers = [[torch.randn(s, generator=g) for s in [(16,), (9, 9), (5, 4), (300,)]] for _ in range(2)]
+    _, averaging = step(peers, 2, torch.float32, 1 << 20, ReduceOp.AVG, "aliased", monkeypatch)
+    # the first step has shared memory and copies; afterwards every tensor has storage of its own
+    assert all(len(a.buckets[0]["piecewise"]) == 1 for a in averaging)
+
+    want, _ = step(peers, 2, torch.float32, 1 << 20, ReduceOp.AVG, "copies", monkeypatch)
+    group = SimGroup(2)
+    mine = [[t.cuda() for t in tensors] for tensors in peers]
+    versions = [[t._version for t in tensors] for tensors in mine]
+    gather = type(group.rank(0)).allgather_into_tensor_coalesced
+
+    def moving(self, *args, **kwargs):
+        mine[self.rank()][1].data = torch.zeros(9, 9, device="cuda")
+        return gather(self, *args, **kwargs)
+
+    monkeypatch.setattr(type(group.rank(0)), "allgather_into_tensor_coalesced", moving)
+    averaging = [ar.BucketizedAllreduce(tensors, 1 << 20) for tensors in mine]
+
+    def rank_fn(r):
+        for w in averaging[r].allreduce(group.rank(r), 2):
+            w.wait()
+
+    run_ranks(2, rank_fn, group)
+    torch.cuda.synchronize()
+    for r in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(mine[r], want[r][0]))
+        assert all(t._version > v for i, (t, v) in enumerate(zip(mine[r], versions[r])) if i != 1)
