@@ -1,0 +1,50 @@
+"""Reduce of short rows in groups of more peers than a team of lanes or its registers hold at
+once, and of one-column tensors of few rows, against the CPU checker, by bytes."""
+
+import pytest
+import torch
+from torch.distributed import ReduceOp
+
+from test_gpu_parity import full_check, q  # noqa: F401 (q is a fixture)
+
+pytestmark = pytest.mark.gpu
+
+# columns on both sides of 1, 2, 3, 4, 8, 12, 16, 32, 64 and 128 dwords of codes
+COLUMNS = [0, 1, 2, 4, 5, 8, 9, 12, 13, 16, 17, 31, 32, 33, 44, 45, 48, 49, 64, 65, 127, 128, 129, 256, 257, 511, 512]
+
+
+@pytest.mark.parametrize("plain_divide", [False, True])
+@pytest.mark.parametrize("long_list", [False, True])
+@pytest.mark.parametrize("ws,op", [(1, ReduceOp.SUM), (2, ReduceOp.AVG), (7, ReduceOp.AVG), (8, ReduceOp.SUM), (9, ReduceOp.AVG),
+                                   (16, ReduceOp.AVG), (17, ReduceOp.SUM), (24, ReduceOp.AVG), (25, ReduceOp.SUM),
+                                   (33, ReduceOp.AVG), (64, ReduceOp.AVG), (65, ReduceOp.SUM), (70, ReduceOp.AVG)])
+def test_short_rows_in_large_groups(q, oracle, ws, op, long_list, plain_divide):  # noqa: F811
+    g = torch.Generator().manual_seed(ws)
+    columns = COLUMNS if long_list else COLUMNS[ws % 2::2]
+    shapes = [((3 * i) % (4 * ws) + 1, n) for i, n in enumerate(columns)]
+    base = []
+    for p in range(min(ws, 3)):
+        ts = [torch.randn(s, generator=g) * (1 + p) for s in shapes]
+        for i, t in enumerate(ts):
+            t[len(t) // 3] = -0.0
+            if plain_divide and p == 1 and i % 2:
+                t[len(t) // 2] *= 1e-30  # a scale outside the range of the fast division
+        base.append([t.to(torch.bfloat16) for t in ts])
+    full_check(q, oracle, [base[p % len(base)] for p in range(ws)], ws, op, sorted({0, ws // 2, ws - 1}))
+
+
+@pytest.mark.parametrize("ws,op", [(1, ReduceOp.SUM), (2, ReduceOp.SUM), (3, ReduceOp.AVG), (4, ReduceOp.AVG),
+                                   (5, ReduceOp.SUM), (16, ReduceOp.AVG), (17, ReduceOp.SUM), (70, ReduceOp.AVG)])
+@pytest.mark.parametrize("long_list", [False, True])
+def test_one_column_of_few_and_many_rows(q, oracle, ws, op, long_list):  # noqa: F811
+    # rows per slot on both sides of a wavefront, a workgroup and four rows per lane
+    per_slot = [1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 1280, 1281]
+    sizes = [n * ws - i % 2 * (ws > 1) for i, n in enumerate(per_slot)] * (2 if long_list else 1)
+    g = torch.Generator().manual_seed(ws)
+    base = []
+    for p in range(min(ws, 3)):
+        ts = [torch.randn(n, generator=g) * 10.0 ** torch.randint(-30, 30, (n,), generator=g).float() for n in sizes]
+        for t in ts:
+            t[::5] = 0.0
+        base.append(ts)
+    full_check(q, oracle, [base[p % len(base)] for p in range(ws)], ws, op, sorted({0, ws - 1}))

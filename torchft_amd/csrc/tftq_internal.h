@@ -279,6 +279,7 @@ struct tftq_plan {
     int32_t nwg[N_LAUNCHES];
     bool wide[3];              // per stage: some row needs the kernel variant with more registers
     bool reduce_long_rows;     // every row of the list runs in a team of 64 or 256 lanes in reduce or has one column (k_reduce's R_LONG)
+    bool reduce_one_column;    // every row of the list has one column (R_ONE)
     int parked;                // quantize: groups of 5 vectors per lane (20 KB of LDS each, up to 3) that the longest row parks in LDS (rows above TFTQ_Q_VECS_WIDE)
     int cols_most;             // quantize: columns of the widest K_COLS tensor
     Dealt dealt[N_LAUNCHES];   // inline table only

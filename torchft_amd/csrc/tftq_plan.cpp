@@ -127,13 +127,15 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
     // 17 to 64 bytes of codes.  A lane per row loads its row with two or four 16-byte loads that
     // lie a row apart from its neighbours'; a pair of lanes (up to 32 bytes) or a team of 4 with
     // one vector each covers 32 or 16 neighbouring rows with one load per wavefront and peer
-    // and has every load of its row in flight at once (groups of up to 16 peers).  218 M bf16
-    // elements, 8 peers, a lane per row against the team: 24 columns 81.1 -> 66.7 us, 28: 89.2
-    // -> 64.4, 32: 65.0 -> 64.4, 44: 92.1 -> 68.7, 60: 95.6 -> 64.7, 64: 70.6 -> 65.0; 48 columns
-    // (three whole vectors: a lane per row wastes nothing, the team idles a lane) 67.3 -> 69.4.
-    if (ndw > 8 && ndw <= 16 && ndw != 12 && ws <= 16) return K_GEN4;
-    if (ndw > 4 && ndw <= 8 && ws <= 16) return K_GEN2;
-    if (ndw <= 16) return K_GEN1;  // a lane per row beats a team with idle lanes
+    // and has every load of its row in flight at once (in groups of more than 16 peers, of 8 peers
+    // and the next 8).  218 M bf16 elements, 8 peers, a lane per row against the team: 24 columns
+    // 81.1 -> 66.7 us, 28: 89.2 -> 64.4, 32: 65.0 -> 64.4, 44: 92.1 -> 68.7, 60: 95.6 -> 64.7, 64:
+    // 70.6 -> 65.0.  45 to 48 columns are three whole vectors, of which a lane alone wastes none:
+    // [2097152, 48], 4, 8 and 16 peers: 33.1 -> 31.0 us, 29.6 -> 28.2, 27.4 -> 29.8; in a tensor of
+    // a few rows the lane alone waits 33 us for its 16 peers, the team 7 us.
+    if (ndw > 8 && ndw <= 16) return K_GEN4;
+    if (ndw > 4 && ndw <= 8) return K_GEN2;
+    if (ndw <= 16) return K_GEN1;
     if (ndw <= 32) return K_GEN8;
     if (ndw <= 64) return K_GEN16;
     // Rows that would leave more than a quarter of the next team idle take three vectors per
@@ -384,12 +386,13 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
     for (int st = 0; st < N_LAUNCHES; st++) p->nwg[st] = (int32_t)wg[st];
     p->wide[ST_Q] = p->wide[ST_R] = p->wide[ST_D] = false;
     p->parked = 0;
-    p->reduce_long_rows = true;
+    p->reduce_long_rows = p->reduce_one_column = true;
     for (int i = 0; i < n_tensors; i++) {
         const Seg &s = p->segs[(size_t)i];
         const int nvec = s.n / (16 / p->esz), ndw = s.row_bytes / 4 - 1;
         if (s.m > 0 && s.kind[ST_R] != K_GEN256 && s.kind[ST_R] != K_GEN64 && s.kind[ST_R] != K_COL1)
             p->reduce_long_rows = false;
+        if (s.m > 0 && s.kind[ST_R] != K_COL1) p->reduce_one_column = false;
         if (s.kind[ST_Q] == K_VEC256 && nvec > TFTQ_Q_VECS && s.m > 0) p->wide[ST_Q] = true;
         if (s.kind[ST_Q] == K_VEC256 && nvec > TFTQ_Q_VECS_WIDE && s.m > 0) p->parked = std::max(p->parked, tftq_q_park_groups(nvec));
         if (s.kind[ST_R] == K_GEN256 && ndw > TFTQ_R_DWORDS && s.m > 0 && ws <= 64)

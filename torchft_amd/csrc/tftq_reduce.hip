@@ -41,27 +41,6 @@ DEV u32x4 load_codes(GLOBAL const u32 *payload, int d0, int ndw, int n)
     return w;
 }
 
-// The same without a branch, for lanes that own a whole short row each whose length is not a
-// whole number of 16-byte vectors (loads under a condition end up one per basic block with a
-// wait in front of each: a row of 3 dwords cost its lane 3 round trips to memory per peer):
-// four dword loads at indices clamped into the row, then dwords past the end are cleared.
-// Plain loads: the rows of neighbouring lanes share cache lines, as do the loads of one lane.
-DEV u32x4 load_codes_clamped(GLOBAL const u32 *payload, int d0, int ndw, int n)
-{
-    u32x4 w;
-    w.x = payload[min(d0, ndw - 1)];
-    w.y = payload[min(d0 + 1, ndw - 1)];
-    w.z = payload[min(d0 + 2, ndw - 1)];
-    w.w = payload[min(d0 + 3, ndw - 1)];
-    const int last = ndw - 1 - d0;  // position of the row's last dword in w
-    const u32 mask = (n & 3) ? (1u << (8 * (n & 3))) - 1u : 0xFFFFFFFFu;
-    w.x = last < 0 ? 0u : last == 0 ? w.x & mask : w.x;
-    w.y = last < 1 ? 0u : last == 1 ? w.y & mask : w.y;
-    w.z = last < 2 ? 0u : last == 2 ? w.z & mask : w.z;
-    w.w = last < 3 ? 0u : last == 3 ? w.w & mask : w.w;
-    return w;
-}
-
 DEV void store_codes(GLOBAL u32 *payload, int d0, int ndw, const u32x4 w)
 {
     const int rem = ndw - d0;
@@ -431,9 +410,9 @@ DEV void reduce_row_hybrid(const Seg &s, const KParams &p, int j, int tid, float
 }
 
 // Register-resident row: the team holds all accumulators of the row, each peer
-// row is read once.  UNITS = 16-byte vectors of codes per lane and peer.
-// CLAMPED (one lane per row, rows that are not whole 16-byte vectors): loads without branches.
-template <int TEAM, int UNITS, bool GDIV, bool CLAMPED = false>
+// row is read once.  UNITS = 16-byte vectors of codes per lane and peer.  Teams of 64 and 256 lanes
+// in groups of more than 64 peers.
+template <int TEAM, int UNITS, bool GDIV>
 DEV void reduce_row(const Seg &s, const KParams &p, int j, int lane, float *lds)
 {
     constexpr int PB = 8 / UNITS;  // peers whose loads are in flight together
@@ -455,22 +434,14 @@ DEV void reduce_row(const Seg &s, const KParams &p, int j, int lane, float *lds)
         // first, then the codes of the first peers go in flight, and only then
         // are the scales turned into division coefficients.
         float my_scale = 1.0f;
-        if (TEAM >= 64 && kc + wlane < p.ws) my_scale = guarded_scale(peer_row(p, kc + wlane, off));
+        if (kc + wlane < p.ws) my_scale = guarded_scale(peer_row(p, kc + wlane, off));
 
         u32x4 w[PB][UNITS];
-        float sraw[PB];
         auto load_batch = [&](int k0) {
 #pragma unroll
             for (int b = 0; b < PB; b++) {
-                if constexpr (CLAMPED) {
-                    // no branch: a peer past the last one re-reads the last and is ignored below
-                    GLOBAL const u32 *prow = peer_row(p, min(k0 + b, kend - 1), off);
-                    sraw[b] = guarded_scale(prow);
-#pragma unroll
-                    for (int u = 0; u < UNITS; u++) w[b][u] = load_codes_clamped(prow + 1, u * 4, ndw, n);
-                } else if (k0 + b < kend) {
+                if (k0 + b < kend) {
                     GLOBAL const u32 *prow = peer_row(p, k0 + b, off);
-                    if (TEAM < 64) sraw[b] = guarded_scale(prow);
 #pragma unroll
                     for (int u = 0; u < UNITS; u++)
                         w[b][u] = load_codes(prow + 1, (u * TEAM + lane) * 4, ndw, n);
@@ -479,40 +450,17 @@ DEV void reduce_row(const Seg &s, const KParams &p, int j, int lane, float *lds)
         };
         load_batch(kc);
 
-        float cr = 1.0f, cl = 0.0f;
-        if (TEAM >= 64) {
-            const DivCoef c = make_div(my_scale);
-            cr = c.r;
-            cl = c.r_lo;
-            if (__builtin_amdgcn_ballot_w64(!c.fast) != 0) {  // some peer needs the plain divide
-                reduce_row_slow<TEAM, GDIV>(s, p, j, lane, lds);
-                return;
-            }
+        const DivCoef c = make_div(my_scale);
+        if (__builtin_amdgcn_ballot_w64(!c.fast) != 0) {  // some peer needs the plain divide
+            reduce_row_slow<TEAM, GDIV>(s, p, j, lane, lds);
+            return;
         }
         for (int k0 = kc; k0 < kend; k0 += PB) {
             if (k0 != kc) load_batch(k0);
-            if (TEAM < 64) {
-                bool fast = true;
-#pragma unroll
-                for (int b = 0; b < PB; b++)
-                    if (k0 + b < kend) fast = fast && scale_is_fast(sraw[b]);
-                if (!fast) {  // same decision in every lane of the team
-                    reduce_row_slow<TEAM, GDIV>(s, p, j, lane, lds);
-                    return;
-                }
-            }
 #pragma unroll
             for (int b = 0; b < PB; b++) {
                 if (k0 + b < kend) {
-                    float pr, pl;
-                    if (TEAM >= 64) {
-                        pr = bcast_lane(cr, k0 + b - kc);
-                        pl = bcast_lane(cl, k0 + b - kc);
-                    } else {
-                        const DivCoef c = make_div(sraw[b]);
-                        pr = c.r;
-                        pl = c.r_lo;
-                    }
+                    const float pr = bcast_lane(c.r, k0 + b - kc), pl = bcast_lane(c.r_lo, k0 + b - kc);
 #pragma unroll
                     for (int u = 0; u < UNITS; u++) accumulate16(acc[u], w[b][u], pr, pl);
                 }
@@ -734,6 +682,165 @@ DEV void reduce_rows_narrow(const Seg &s, const KParams &p, int j, int lane, flo
     if (valid && lane == 0) orow[0] = as_u(s2);  // :375; all lanes read the old scale before team_max
 }
 
+// Rows of up to 16 * TEAM bytes of codes in groups of more peers than a team (or the registers)
+// holds at once: one vector per lane and peer, R_CHUNK peers at a time, the next chunk's scales
+// and codes in flight while the current one is accumulated.  Lane l of a team fetches the scales
+// of the chunk's peers l, l + TEAM, ...  As everywhere in this file the loads carry no branch.
+// (A load under a condition waits for the one before it: with such loads a row cost its team a
+// trip to memory per peer, and a list whose tensors have a few rows each, so that one wavefront
+// does a whole tensor, waits for exactly that.  10 000 tensors of up to 4096 elements, 16 peers:
+// 60.1 -> 36.1 us, of that reduce_col1_few about half.  24 peers, 60 columns: 32 -> 12.5 us.)
+// `valid` as in reduce_rows.
+constexpr int R_CHUNK = 8;
+template <int TEAM, bool GDIV>
+DEV void reduce_rows_chunks(const Seg &s, const KParams &p, int j, int lane, float *lds, bool valid)
+{
+    constexpr int CH = TEAM == 1 ? R_CHUNK / 2 : R_CHUNK;  // a lane alone holds the coefficients of all of them
+    constexpr int NS = CH > TEAM ? CH / TEAM : 1;  // scales per lane
+    const int ndw = (s.row_bytes >> 2) - 1;  // >= 4 here
+    const int ws = p.ws;
+    const int64_t off = s.slot_off + (int64_t)j * s.row_bytes;
+    const int doff = min(4 * lane, ndw - 4);  // the last vector ends with the row (see reduce_rows)
+    const u32 padmask = (doff == ndw - 4 && (s.n & 3)) ? (1u << (8 * (s.n & 3))) - 1u : 0xFFFFFFFFu;
+
+    struct Chunk {
+        float raw[NS];
+        u32x4 w[CH];
+    };
+    auto issue = [&](Chunk &c, int k0) {
+#pragma unroll
+        for (int i = 0; i < NS; i++) c.raw[i] = as_f(peer_row(p, min(k0 + lane % CH + i * TEAM, ws - 1), off)[0]);
+#pragma unroll
+        for (int k = 0; k < CH; k++)
+            c.w[k] = LOAD_STREAM((GLOBAL const u32x4_a4 *)(peer_row(p, min(k0 + k, ws - 1), off) + 1 + doff));
+        __builtin_amdgcn_sched_barrier(0);  // all loads are issued before anything below
+    };
+    float acc[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+    // false: some peer needs the plain divide (the same for the whole wavefront)
+    auto consume = [&](const Chunk &c, int k0) {
+        DivCoef d[NS];
+        bool fast = true;
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            d[i] = make_div(c.raw[i] == 0.0f ? 1.0f : c.raw[i]);  // padding rows (:419)
+            fast = fast && d[i].fast;
+        }
+        if (__builtin_amdgcn_ballot_w64(!fast) != 0) return false;
+#pragma unroll
+        for (int k = 0; k < CH; k++) {
+            if (k0 + k < ws) {
+                const float pr = team_bcast<TEAM>(d[k / TEAM].r, k % TEAM);
+                const float pl = team_bcast<TEAM>(d[k / TEAM].r_lo, k % TEAM);
+                u32x4 v = c.w[k];
+                v.w &= padmask;
+                accumulate16(acc, v, pr, pl);
+            }
+        }
+        return true;
+    };
+    Chunk A, B;
+    bool fast = true;
+    issue(A, 0);
+#pragma nounroll
+    for (int k0 = 0; k0 < ws; k0 += 2 * CH) {  // A holds the chunk at k0
+        if (k0 + CH < ws) issue(B, k0 + CH);
+        if (!(fast = consume(A, k0))) break;
+        if (k0 + CH < ws) {
+            if (k0 + 2 * CH < ws) issue(A, k0 + 2 * CH);
+            if (!(fast = consume(B, k0 + CH))) break;
+        }
+    }
+    if (!fast) {
+        if (valid) reduce_row_slow<TEAM, GDIV>(s, p, j, lane, lds);
+        return;
+    }
+    float amax = 0.0f;  // duplicates held by lanes past the row's end do not change it
+#pragma unroll
+    for (int e = 0; e < 16; e++) amax = fmaxf(amax, __builtin_fabsf(acc[e]));
+    amax = team_max<TEAM>(amax, lds);
+    const float s2 = calc_scale(amax_div<GDIV>(amax, p));  // :340
+    GLOBAL u32 *orow = as_global<u32>(p.packed + (int64_t)p.rank * p.slot_size + off);
+    const u32x4 o = requant16<GDIV>(acc, s2, p);
+    if (valid && 4 * lane < ndw) STORE_CODES(o, (GLOBAL u32x4_a4 *)(orow + 1 + doff));
+    if (valid && lane == 0) orow[0] = as_u(s2);  // :375; all lanes read the old scale before team_max
+}
+
+// Rows of ND = 1, 2 or 3 payload dwords (2 to 12 columns), a lane per row: the scale and all codes
+// of a row come in with one load of ND + 1 dwords, neighbouring lanes' rows are neighbours in
+// memory, and the next R_CHUNK peers are in flight while the current ones are accumulated.
+// [6291456, 3] bf16 against four clamped dword loads per row and peer: 2 peers 75 -> 35 us,
+// 8 peers 27.5 -> 14.3 us; [4194304, 5]: 54.5 -> 28, 23.1 -> 13.8 us.
+template <int ND, bool GDIV>
+DEV void reduce_rows_tiny(const Seg &s, const KParams &p, int j, float *lds, bool valid)
+{
+    typedef u32 Row __attribute__((ext_vector_type(ND + 1)));
+    typedef Row Row_a4 __attribute__((aligned(4)));
+    const int ws = p.ws;
+    const int64_t off = s.slot_off + (int64_t)j * s.row_bytes;
+    const u32 padmask = (s.n & 3) ? (1u << (8 * (s.n & 3))) - 1u : 0xFFFFFFFFu;
+    struct Chunk {
+        Row w[R_CHUNK];
+    };
+    auto issue = [&](Chunk &c, int k0) {
+#pragma unroll
+        for (int k = 0; k < R_CHUNK; k++) c.w[k] = LOAD_STREAM((GLOBAL const Row_a4 *)peer_row(p, min(k0 + k, ws - 1), off));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float acc[4 * ND];
+#pragma unroll
+    for (int e = 0; e < 4 * ND; e++) acc[e] = 0.0f;
+    auto consume = [&](const Chunk &c, int k0) {
+        bool fast = true;
+#pragma unroll
+        for (int k = 0; k < R_CHUNK; k++) fast = fast && (c.w[k][0] == 0u || scale_is_fast(as_f(c.w[k][0])));
+        if (__builtin_amdgcn_ballot_w64(!fast) != 0) return false;
+#pragma unroll
+        for (int k = 0; k < R_CHUNK; k++) {
+            if (k0 + k < ws) {
+                const float sc = as_f(c.w[k][0]);
+                const DivCoef d = make_div(sc == 0.0f ? 1.0f : sc);  // padding rows (:419)
+#pragma unroll
+                for (int t = 0; t < ND; t++) {
+                    float f[4];
+                    unpack_fp8x4(t == ND - 1 ? c.w[k][1 + t] & padmask : c.w[k][1 + t], f);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[4 * t + e] = acc[4 * t + e] + div_fast(f[e], d.r, d.r_lo);
+                }
+            }
+        }
+        return true;
+    };
+    Chunk A, B;
+    bool fast = true;
+    issue(A, 0);
+#pragma nounroll
+    for (int k0 = 0; k0 < ws; k0 += 2 * R_CHUNK) {
+        if (k0 + R_CHUNK < ws) issue(B, k0 + R_CHUNK);
+        if (!(fast = consume(A, k0))) break;
+        if (k0 + R_CHUNK < ws) {
+            if (k0 + 2 * R_CHUNK < ws) issue(A, k0 + 2 * R_CHUNK);
+            if (!(fast = consume(B, k0 + R_CHUNK))) break;
+        }
+    }
+    if (!fast) {
+        if (valid) reduce_row_slow<1, GDIV>(s, p, j, 0, lds);
+        return;
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4 * ND; e++) amax = fmaxf(amax, __builtin_fabsf(acc[e]));
+    const float s2 = calc_scale(amax_div<GDIV>(amax, p));  // :340
+    Row o;
+    o[0] = as_u(s2);
+#pragma unroll
+    for (int t = 0; t < ND; t++)
+        o[1 + t] = pack_fp8x4(scale_div<GDIV>(acc[4 * t], s2, p), scale_div<GDIV>(acc[4 * t + 1], s2, p),
+                              scale_div<GDIV>(acc[4 * t + 2], s2, p), scale_div<GDIV>(acc[4 * t + 3], s2, p));
+    if (valid) STORE_CODES(o, (GLOBAL Row_a4 *)as_global<u32>(p.packed + (int64_t)p.rank * p.slot_size + off));
+}
+
 // One row per team with UNITS >= 2 vectors per lane and peer, as a rolling window over the
 // peers: as soon as a lane has taken vector u of peer k out of its registers, the load of
 // vector u of peer k + 1 is issued into them, so UNITS loads are in flight all the time at
@@ -929,12 +1036,107 @@ DEV void reduce_rows_at_once(const Seg &s, const KParams &p, int j0, int lane, f
 }
 
 // Rows of one column: 8 bytes per row and peer, one plain divide per peer
-// (coefficients for the fast division would cost two), four rows per lane.
+// (coefficients for the fast division would cost two).
+// a += code / scale of a packed row
+DEV void accumulate_one(float &a, const u32x2 w)
+{
+    float sc = as_f(w.x);
+    sc = sc == 0.0f ? 1.0f : sc;  // padding rows (:419)
+    a = a + __builtin_amdgcn_cvt_f32_fp8((int)w.y, 0) / sc;
+}
+// [scale, code] of a sum
+template <bool GDIV, bool IEEE>
+DEV u32x2 requant_one(const KParams &p, float a)
+{
+    const float s2 = calc_scale(amax_div<GDIV>(fmaxf(0.0f, __builtin_fabsf(a)), p));  // NaN ignored (:331-338)
+    u32x2 o;
+    o.x = as_u(s2);
+    o.y = pack_fp8x4(scale_div<GDIV, IEEE>(a, s2, p), 0.0f, 0.0f, 0.0f) & 0xFFu;
+    return o;
+}
+
+// At most a row per lane left: the loads of PB peers in flight at once.  (A list of short vectors
+// is done when its wavefronts have waited for their peers: 1728 vectors of up to 4096 elements,
+// 16 peers: 25.4 us with a peer at a time, 8.6 us with all of them.)
+template <int PB, bool GDIV, bool IEEE>
+DEV void reduce_col1_few(const Seg &s, const KParams &p, int j, bool valid)
+{
+    const int64_t off = s.slot_off + (int64_t)j * 8;
+    float acc = 0.0f;
+#pragma nounroll
+    for (int k0 = 0; k0 < p.ws; k0 += PB) {
+        u32x2 w[PB];
+#pragma unroll
+        for (int b = 0; b < PB; b++) w[b] = LOAD_STREAM((GLOBAL const u32x2_a4 *)peer_row(p, min(k0 + b, p.ws - 1), off));
+        __builtin_amdgcn_sched_barrier(0);  // all loads are issued before anything below
+#pragma unroll
+        for (int b = 0; b < PB; b++)
+            if (k0 + b < p.ws) accumulate_one(acc, w[b]);
+    }
+    if (!valid) return;
+    const u32x2 o = requant_one<GDIV, IEEE>(p, acc);
+    STORE_STREAM(o, (GLOBAL u32x2_a4 *)as_global<u32>(p.packed + (int64_t)p.rank * p.slot_size + off));
+}
+
+// One or two peers: two pairs of neighbouring rows per lane, a pair with one 16-byte access.
+// (44 M rows, 2 peers: 92 us with four rows per lane and 8-byte accesses, 86 us.)
+template <bool GDIV, bool IEEE>
+DEV void reduce_col1_pairs(const Seg &s, const KParams &p, int j0, int tid)
+{
+    constexpr int PAIRS = 2, PB = 2;
+    float acc[PAIRS][2];
+    int64_t off[PAIRS];
+    u32x4 w[PB][PAIRS];
+#pragma unroll
+    for (int k = 0; k < PAIRS; k++) {
+        acc[k][0] = acc[k][1] = 0.0f;
+        // a row without a neighbour (the last of an odd number) comes in behind the one before it
+        off[k] = s.slot_off + (int64_t)min(j0 + 2 * (k * TFTQ_WG + tid), s.slice_rows - 2) * 8;
+    }
+#pragma unroll
+    for (int b = 0; b < PB; b++)
+#pragma unroll
+        for (int k = 0; k < PAIRS; k++) w[b][k] = LOAD_STREAM((GLOBAL const u32x4_a4 *)peer_row(p, min(b, p.ws - 1), off[k]));
+    __builtin_amdgcn_sched_barrier(0);  // all loads are issued before anything below
+#pragma unroll
+    for (int b = 0; b < PB; b++) {
+        if (b < p.ws) {
+#pragma unroll
+            for (int k = 0; k < PAIRS; k++) {
+                accumulate_one(acc[k][0], u32x2{w[b][k].x, w[b][k].y});
+                accumulate_one(acc[k][1], u32x2{w[b][k].z, w[b][k].w});
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < PAIRS; k++) {
+        const int j = j0 + 2 * (k * TFTQ_WG + tid);
+        if (j >= s.slice_rows) continue;
+        const u32x2 a = requant_one<GDIV, IEEE>(p, acc[k][0]), b = requant_one<GDIV, IEEE>(p, acc[k][1]);
+        GLOBAL u32 *out = as_global<u32>(p.packed + (int64_t)p.rank * p.slot_size + off[k]);
+        // streaming: neighbouring lanes write neighbouring rows, whole lines per wavefront
+        if (j + 1 < s.slice_rows) STORE_STREAM((u32x4{a.x, a.y, b.x, b.y}), (GLOBAL u32x4_a4 *)out);
+        else STORE_STREAM(b, (GLOBAL u32x2_a4 *)(out + 2));  // the row before it is another lane's
+    }
+}
+
+// More peers: four rows per lane, a peer at a time (16-byte accesses and two or four peers at a
+// time are 2 to 8 % slower from 4 peers on: 33.5 M rows, 8 peers 51.9 us, 54 to 55 us).
 template <bool GDIV, bool IEEE = false>
 DEV void reduce_col1(const Seg &s, const KParams &p, int j0, int tid)
 {
+    if (s.slice_rows - j0 > TFTQ_WG && p.ws <= 2) {  // same for the whole workgroup, as is the next
+        reduce_col1_pairs<GDIV, IEEE>(s, p, j0, tid);
+        return;
+    }
     // a wavefront none of whose lanes has a row (rows go up with k) leaves at once
     if (__builtin_amdgcn_ballot_w64(j0 + tid < s.slice_rows) == 0) return;
+    if (s.slice_rows - j0 <= TFTQ_WG) {
+        const int j = min(j0 + tid, s.slice_rows - 1);
+        if (p.ws <= 4) reduce_col1_few<4, GDIV, IEEE>(s, p, j, j0 + tid < s.slice_rows);
+        else reduce_col1_few<16, GDIV, IEEE>(s, p, j, j0 + tid < s.slice_rows);
+        return;
+    }
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     int64_t off[4];
 #pragma unroll
@@ -946,20 +1148,12 @@ DEV void reduce_col1(const Seg &s, const KParams &p, int j0, int tid)
 #pragma unroll
         for (int k = 0; k < 4; k++) w[k] = LOAD_STREAM((GLOBAL const u32x2_a4 *)peer_row(p, kk, off[k]));
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            float sc = as_f(w[k].x);
-            sc = sc == 0.0f ? 1.0f : sc;  // padding rows (:419)
-            acc[k] = acc[k] + __builtin_amdgcn_cvt_f32_fp8((int)w[k].y, 0) / sc;
-        }
+        for (int k = 0; k < 4; k++) accumulate_one(acc[k], w[k]);
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         if (j0 + k * TFTQ_WG + tid < s.slice_rows) {
-            const float s2 = calc_scale(amax_div<GDIV>(fmaxf(0.0f, __builtin_fabsf(acc[k])), p));  // NaN ignored (:331-338)
-            u32x2 o;
-            o.x = as_u(s2);
-            o.y = pack_fp8x4(scale_div<GDIV, IEEE>(acc[k], s2, p), 0.0f, 0.0f, 0.0f) & 0xFFu;
-            // streaming: neighbouring lanes write neighbouring rows, whole lines per wavefront
+            const u32x2 o = requant_one<GDIV, IEEE>(p, acc[k]);
             STORE_STREAM(o, (GLOBAL u32x2_a4 *)as_global<u32>(p.packed + (int64_t)p.rank * p.slot_size + off[k]));
         }
     }
@@ -975,13 +1169,15 @@ DEV void reduce_col1(const Seg &s, const KParams &p, int j0, int tid)
     } while (0)
 
 // reduce_rows_narrow for a team of TEAM lanes, for the smallest of 2, 4, 8 and 16 peers that
-// holds the group (a variant for more peers loads the last peer again in their place)
+// holds the group (a variant for more peers loads the last peer again in their place);
+// larger groups go through it in chunks
 #define TFTQ_REDUCE_NARROW(TEAM, ...)                                             \
     do {                                                                          \
         if (p.ws <= 2) reduce_rows_narrow<TEAM, 2, GDIV>(__VA_ARGS__);            \
         else if (p.ws <= 4) reduce_rows_narrow<TEAM, 4, GDIV>(__VA_ARGS__);       \
         else if (p.ws <= 8) reduce_rows_narrow<TEAM, 8, GDIV>(__VA_ARGS__);       \
-        else reduce_rows_narrow<TEAM, 16, GDIV>(__VA_ARGS__);                     \
+        else if (p.ws <= 16) reduce_rows_narrow<TEAM, 16, GDIV>(__VA_ARGS__);     \
+        else reduce_rows_chunks<TEAM, GDIV>(__VA_ARGS__);                         \
     } while (0)
 
 // FLAVOUR: R_ALL, every kind of row; R_WIDE, for lists with rows of more than 16384 columns:
@@ -991,10 +1187,21 @@ DEV void reduce_col1(const Seg &s, const KParams &p, int j0, int tid)
 // the compiler makes of one kind's code depends on what else the kernel holds (registers
 // kept across the switch, the order of the blocks): with R_LONG the code for the long rows
 // of such lists is compiled on its own and does not move when another kind's code changes.
-enum { R_ALL = 0, R_WIDE = 1, R_LONG = 2 };
-DEV int long_kind(int kind) { return kind == K_GEN64 ? K_GEN64 : kind == K_COL1 ? K_COL1 : K_GEN256; }
+// R_ONE, for lists of one-column tensors (a flat bucket, a list of vectors): few registers, so
+// that a SIMD holds all the wavefronts it can.  From 3 peers on that is too many, each with as many
+// streams as there are peers; dynamic LDS that nobody uses then holds a CU to four workgroups
+// (33.5 M rows, 8 peers: 55.6 us with eight workgroups, 53.0 with six, 52.2 with four, 57.4 with
+// three; 16 peers 52.5, 51.6, 46.6, 53.0; before this variant 51.8 and 48.6).
+constexpr unsigned R_ONE_LDS = 40000;
+enum { R_ALL = 0, R_WIDE = 1, R_LONG = 2, R_ONE = 3 };
+template <int FLAVOUR>
+DEV int kind_of(int kind)
+{
+    if (FLAVOUR == R_LONG) return kind == K_GEN64 ? K_GEN64 : kind == K_COL1 ? K_COL1 : K_GEN256;
+    return FLAVOUR == R_ONE ? (int)K_COL1 : kind;
+}
 template <bool INLINE, bool GDIV, int FLAVOUR>
-__global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : 4) void k_reduce(const KParams p, const InlineTable inl)
+__global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : FLAVOUR == R_ONE ? 8 : 4) void k_reduce(const KParams p, const InlineTable inl)
 {
     constexpr bool WIDE = FLAVOUR == R_WIDE;
     __shared__ float lds[16];
@@ -1014,7 +1221,7 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : 4) void k_reduce(c
     if (GDIV && p.div_mode == 3) {
         // averages over 1024 peers or more, not a power of two: the untuned path with plain divides
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        switch (FLAVOUR == R_LONG ? long_kind(s.kind[ST_R]) : s.kind[ST_R]) {
+        switch (kind_of<FLAVOUR>(s.kind[ST_R])) {
         case K_GEN256: reduce_row_slow<256, true, true>(s, p, blk, tid, lds); break;
         case K_GEN64:
             if (blk * 4 + wave < s.slice_rows) reduce_row_slow<64, true, true>(s, p, blk * 4 + wave, tid & 63, lds);
@@ -1042,8 +1249,8 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : 4) void k_reduce(c
         }
         return;
     }
-    // (R_LONG: one of the three kinds that it is launched for, whatever the table says)
-    switch (FLAVOUR == R_LONG ? long_kind(s.kind[ST_R]) : s.kind[ST_R]) {
+    // (R_LONG, R_ONE: a kind that they are launched for, whatever the table says)
+    switch (kind_of<FLAVOUR>(s.kind[ST_R])) {
     case K_GEN256: {  // one workgroup per row, or per 2 or 4 rows when the group is small
         const int rows = tftq_reduce_rows_at_once(K_GEN256, ndw, p.ws);
         const int j = blk * rows;
@@ -1122,8 +1329,10 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : 4) void k_reduce(c
                 else if (j < s.slice_rows) reduce_row_slow<TEAM, GDIV>(s, p, j, tid % TEAM, lds);
             } else if (p.ws <= TEAM) {
                 TFTQ_REDUCE_ROWS(TEAM, 1, s, p, min(j, s.slice_rows - 1), tid % TEAM, lds, j < s.slice_rows);
+            } else if (TEAM == 8 && p.ws <= 16) {
+                reduce_rows_narrow<TEAM, 16, GDIV>(s, p, min(j, s.slice_rows - 1), tid % TEAM, lds, j < s.slice_rows);
             } else {
-                reduce_row<TEAM, 1, GDIV>(s, p, j, tid % TEAM, lds);
+                reduce_rows_chunks<TEAM, GDIV>(s, p, min(j, s.slice_rows - 1), tid % TEAM, lds, j < s.slice_rows);
             }
         };
         if (s.kind[ST_R] == K_GEN32) small(std::integral_constant<int, 32>());
@@ -1131,30 +1340,26 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : 4) void k_reduce(c
         else small(std::integral_constant<int, 8>());
         break;
     }
-    case K_GEN4: {  // one row per team of 4 lanes, groups of up to 16 peers
+    case K_GEN4: {  // one row per team of 4 lanes
         const int j = blk * 64 + (tid >> 2);
         TFTQ_REDUCE_NARROW(4, s, p, min(j, s.slice_rows - 1), tid & 3, lds, j < s.slice_rows);
         break;
     }
-    case K_GEN2: {  // one row per pair of lanes, groups of up to 16 peers
+    case K_GEN2: {  // one row per pair of lanes
         const int j = blk * 128 + (tid >> 1);
         TFTQ_REDUCE_NARROW(2, s, p, min(j, s.slice_rows - 1), tid & 1, lds, j < s.slice_rows);
         break;
     }
-    case K_GEN1:  // one lane per row: 1, 2 or 4 vectors of codes per peer
-        if (ndw == 4 && p.ws <= 16) {  // one whole vector, all peers in flight at once
-            const int j = blk * 256 + tid;
-            TFTQ_REDUCE_NARROW(1, s, p, min(j, s.slice_rows - 1), 0, lds, j < s.slice_rows);
-        } else if (ndw & 3) {  // not whole 16-byte vectors
-            if (ndw <= 4) reduce_row<1, 1, GDIV, true>(s, p, blk * 256 + tid, 0, lds);
-            else if (ndw <= 8) reduce_row<1, 2, GDIV, true>(s, p, blk * 256 + tid, 0, lds);
-            else reduce_row<1, 4, GDIV, true>(s, p, blk * 256 + tid, 0, lds);
-        } else {
-            if (ndw <= 4) reduce_row<1, 1, GDIV>(s, p, blk * 256 + tid, 0, lds);
-            else if (ndw <= 8) reduce_row<1, 2, GDIV>(s, p, blk * 256 + tid, 0, lds);
-            else reduce_row<1, 4, GDIV>(s, p, blk * 256 + tid, 0, lds);
-        }
+    case K_GEN1: {  // one lane per row
+        const int j = blk * 256 + tid, jc = min(j, s.slice_rows - 1);
+        const bool valid = j < s.slice_rows;
+        if (ndw == 4) TFTQ_REDUCE_NARROW(1, s, p, jc, 0, lds, valid);
+        else if (ndw == 3) reduce_rows_tiny<3, GDIV>(s, p, jc, lds, valid);
+        else if (ndw == 2) reduce_rows_tiny<2, GDIV>(s, p, jc, lds, valid);
+        else if (ndw == 1) reduce_rows_tiny<1, GDIV>(s, p, jc, lds, valid);
+        else if (valid) reduce_row_slow<1, GDIV>(s, p, j, 0, lds);  // no columns: a scale
         break;
+    }
     case K_COL1: reduce_col1<GDIV>(s, p, blk * tftq_col1_rows_per_wg(ST_R), tid); break;
     default: break;
     }
@@ -1190,13 +1395,14 @@ static int reduce_launch(const tftq_plan *plan, const void *table, void *packed,
     if (kp.nwg == 0) return 0;
     const unsigned grid = grid_of(kp);
     const bool gdiv = kp.div_mode >= 2;
-#define TFTQ_LAUNCH_R(I, G, F) return launch_kernel(k_reduce<I, G, F>, grid, 0, st, kp, inl)
+#define TFTQ_LAUNCH_R(I, G, F) return launch_kernel(k_reduce<I, G, F>, grid, F == R_ONE && plan->ws > 2 ? R_ONE_LDS : 0, st, kp, inl)
 #define TFTQ_LAUNCH_R_FLAVOUR(F)                                                                        \
     do {                                                                                                \
         if (gdiv) { if (use_inline) TFTQ_LAUNCH_R(true, true, F); else TFTQ_LAUNCH_R(false, true, F); } \
         else { if (use_inline) TFTQ_LAUNCH_R(true, false, F); else TFTQ_LAUNCH_R(false, false, F); }    \
     } while (0)
     if (plan->wide[ST_R]) TFTQ_LAUNCH_R_FLAVOUR(R_WIDE);
+    else if (plan->reduce_one_column) TFTQ_LAUNCH_R_FLAVOUR(R_ONE);
     else if (plan->reduce_long_rows) TFTQ_LAUNCH_R_FLAVOUR(R_LONG);
     else TFTQ_LAUNCH_R_FLAVOUR(R_ALL);
 #undef TFTQ_LAUNCH_R_FLAVOUR
