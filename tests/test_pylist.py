@@ -100,3 +100,26 @@ def test_named_functions_fall_back_without_a_gpu():
     assert q._match_long_list(ts, 2, True) is None
     with pytest.raises(RuntimeError, match="no CPU path"):
         q.fused_quantize_into_fp8(ts, 2)
+
+
+def test_describe_tells_short_lists_apart(pylist):
+    def said(*ts, most=16):
+        return pylist.describe(list(ts), most)
+
+    a, b = torch.empty(3, 4), torch.empty(5, 2).t()
+    key, device, ptrs = said(a, b)
+    assert device == -1 and list((ctypes.c_uint64 * 2).from_buffer_copy(ptrs)) == [a.data_ptr(), b.data_ptr()]
+    assert said(torch.nn.Parameter(torch.empty(3, 4)), torch.empty(5, 2).t())[0] == key   # other tensors of the same form
+    others = [(a,), (b, a), (a, torch.empty(2, 5)), (torch.empty(4, 3).t(), b), (a[:2], b), (a, b, a),
+              (a.bfloat16(), b.bfloat16()), (a.half(), b.half()), (torch.empty(3, 9)[:, :4], b)]
+    keys = [said(*ts)[0] for ts in others]
+    assert len(set(keys + [key])) == len(others) + 1
+
+
+@pytest.mark.parametrize("what", ["1-D", "3-D", "dtype", "mixed dtypes", "mixed devices", "subclass", "none", "empty", "long", "tuple"])
+def test_describe_leaves_the_rest_to_python(pylist, what):
+    a = torch.empty(3, 4)
+    ts = {"1-D": [a, a[0]], "3-D": [a.unsqueeze(0)], "dtype": [a.double()], "mixed dtypes": [a, a.half()],
+          "mixed devices": [a, torch.empty(3, 4, device="meta")], "subclass": [_Wrapper(a)], "none": [a, None],
+          "empty": [], "long": [a] * 17, "tuple": (a,)}[what]
+    assert pylist.describe(ts, 16) is None

@@ -13,6 +13,7 @@
 // (torchft_amd/_build.py).  Not part of libtftq.so, whose C ABI has no Python or torch
 // types.
 
+#define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <torch/csrc/autograd/python_variable.h>
@@ -20,6 +21,31 @@
 #include <ATen/core/Tensor.h>
 
 namespace {
+
+// A tensor is three objects one behind the other (the Python object, the tensor, its storage), and a
+// walk that asks for each when it needs it waits for memory three times per tensor.  The objects of
+// the tensors ahead are asked for before their turn.
+constexpr Py_ssize_t AHEAD = 8;
+inline void fetch_ahead(PyObject *list, Py_ssize_t i, Py_ssize_t n, bool storages)
+{
+    if (i + 3 * AHEAD < n) __builtin_prefetch(PyList_GET_ITEM(list, i + 3 * AHEAD));
+    if (i + 2 * AHEAD < n) {
+        PyObject *o = PyList_GET_ITEM(list, i + 2 * AHEAD);
+        if (THPVariable_CheckExact(o)) {
+            const char *impl = reinterpret_cast<const char *>(THPVariable_Unpack(o).unsafeGetTensorImpl());
+            __builtin_prefetch(impl);
+            __builtin_prefetch(impl + 64);
+            __builtin_prefetch(impl + 128);
+        }
+    }
+    if (storages && i + AHEAD < n) {
+        PyObject *o = PyList_GET_ITEM(list, i + AHEAD);
+        if (THPVariable_CheckExact(o)) {
+            const at::Tensor &t = THPVariable_Unpack(o);
+            if (t.defined()) __builtin_prefetch(t.unsafeGetTensorImpl()->unsafe_storage().unsafeGetStorageImpl());
+        }
+    }
+}
 
 // scan(tensors, dtype, device, shapes, strides, pointers, n) -> int
 //   tensors   a list
@@ -51,6 +77,7 @@ PyObject *scan(PyObject *, PyObject *args)
     Py_ssize_t i = 0;
     try {
         for (; i < n; i++) {
+            fetch_ahead(list, i, n, pointers != nullptr);
             PyObject *o = PyList_GET_ITEM(list, i);
             if (!THPVariable_CheckExact(o) && !THPVariable_Check(o)) break;
             const at::Tensor &t = THPVariable_Unpack(o);
@@ -73,7 +100,56 @@ PyObject *scan(PyObject *, PyObject *args)
     return PyLong_FromSsize_t(i);
 }
 
+// describe(tensors, most) -> (key, device, pointers) or None
+// For a list of 1 to `most` (at most 64) plain 2-D tensors of one of the three dtypes on one device:
+// bytes that differ for lists of other lengths, dtypes, devices, sizes or strides, the device's
+// ordinal (-1: host memory) and the tensors' addresses as the bytes of an array of uint64.  None
+// for anything else.
+PyObject *describe(PyObject *, PyObject *args)
+{
+    constexpr Py_ssize_t MOST = 64;
+    PyObject *list = nullptr;
+    Py_ssize_t most = 0;
+    if (!PyArg_ParseTuple(args, "On", &list, &most)) return nullptr;
+    if (most > MOST) most = MOST;
+    const Py_ssize_t n = PyList_CheckExact(list) ? PyList_GET_SIZE(list) : 0;
+    if (n < 1 || n > most) Py_RETURN_NONE;
+    int64_t key[2 + 4 * MOST];
+    uint64_t pointers[MOST];
+    int64_t device = 0;
+    try {
+        for (Py_ssize_t i = 0; i < n; i++) {
+            PyObject *o = PyList_GET_ITEM(list, i);
+            if (!THPVariable_CheckExact(o)) Py_RETURN_NONE;
+            const at::Tensor &t = THPVariable_Unpack(o);
+            if (!t.defined() || t.unsafeGetTensorImpl()->is_python_dispatch() || t.dim() != 2) Py_RETURN_NONE;
+            const c10::Device d = t.device();
+            if (!d.is_cuda() && !d.is_cpu()) Py_RETURN_NONE;
+            const int64_t dtype = static_cast<int64_t>(t.scalar_type()), at_device = d.is_cuda() ? d.index() : -1;
+            if (i == 0) {
+                if (t.scalar_type() != at::kFloat && t.scalar_type() != at::kHalf && t.scalar_type() != at::kBFloat16) Py_RETURN_NONE;
+                key[0] = dtype;
+                key[1] = device = at_device;
+            }
+            if (dtype != key[0] || at_device != device) Py_RETURN_NONE;
+            const c10::IntArrayRef sz = t.sizes(), st = t.strides();
+            int64_t *k = key + 2 + 4 * i;
+            k[0] = sz[0];
+            k[1] = sz[1];
+            k[2] = st[0];
+            k[3] = st[1];
+            pointers[i] = static_cast<uint64_t>(reinterpret_cast<uintptr_t>(t.data_ptr()));
+        }
+    } catch (...) {
+        Py_RETURN_NONE;  // whatever this tensor is, the Python walk will say it in the reference's words
+    }
+    return Py_BuildValue("(y#iy#)", reinterpret_cast<const char *>(key), static_cast<Py_ssize_t>((2 + 4 * n) * 8),
+                         static_cast<int>(device), reinterpret_cast<const char *>(pointers), static_cast<Py_ssize_t>(n * 8));
+}
+
 PyMethodDef methods[] = {
+    {"describe", describe, METH_VARARGS,
+     "describe(tensors, most): (bytes that tell lists apart, device, addresses) of a short list of 2-D tensors, or None"},
     {"scan", scan, METH_VARARGS,
      "scan(tensors, dtype, device, shapes, strides, pointers, n): check a list of tensors against a plan's "
      "arrays and collect their addresses; returns n, the index of the first mismatch, or -1"},

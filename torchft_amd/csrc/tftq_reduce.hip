@@ -1122,16 +1122,17 @@ DEV void reduce_col1_pairs(const Seg &s, const KParams &p, int j0, int tid)
 
 // More peers: four rows per lane, a peer at a time (16-byte accesses and two or four peers at a
 // time are 2 to 8 % slower from 4 peers on: 33.5 M rows, 8 peers 51.9 us, 54 to 55 us).
-template <bool GDIV, bool IEEE = false>
+// PLAIN: always so (the vectors beside matrices in a layer bucket).
+template <bool GDIV, bool IEEE, bool PLAIN>
 DEV void reduce_col1(const Seg &s, const KParams &p, int j0, int tid)
 {
-    if (s.slice_rows - j0 > TFTQ_WG && p.ws <= 2) {  // same for the whole workgroup, as is the next
+    if (!PLAIN && s.slice_rows - j0 > TFTQ_WG && p.ws <= 2) {  // same for the whole workgroup, as is the next
         reduce_col1_pairs<GDIV, IEEE>(s, p, j0, tid);
         return;
     }
     // a wavefront none of whose lanes has a row (rows go up with k) leaves at once
     if (__builtin_amdgcn_ballot_w64(j0 + tid < s.slice_rows) == 0) return;
-    if (s.slice_rows - j0 <= TFTQ_WG) {
+    if (!PLAIN && s.slice_rows - j0 <= TFTQ_WG) {
         const int j = min(j0 + tid, s.slice_rows - 1);
         if (p.ws <= 4) reduce_col1_few<4, GDIV, IEEE>(s, p, j, j0 + tid < s.slice_rows);
         else reduce_col1_few<16, GDIV, IEEE>(s, p, j, j0 + tid < s.slice_rows);
@@ -1244,7 +1245,7 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : FLAVOUR == R_ONE ?
         case K_GEN1:
             if (blk * 256 + tid < s.slice_rows) reduce_row_slow<1, true, true>(s, p, blk * 256 + tid, 0, lds);
             break;
-        case K_COL1: reduce_col1<true, true>(s, p, blk * tftq_col1_rows_per_wg(ST_R), tid); break;
+        case K_COL1: reduce_col1<true, true, FLAVOUR == R_LONG>(s, p, blk * tftq_col1_rows_per_wg(ST_R), tid); break;
         default: break;
         }
         return;
@@ -1360,7 +1361,7 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : FLAVOUR == R_ONE ?
         else if (valid) reduce_row_slow<1, GDIV>(s, p, j, 0, lds);  // no columns: a scale
         break;
     }
-    case K_COL1: reduce_col1<GDIV>(s, p, blk * tftq_col1_rows_per_wg(ST_R), tid); break;
+    case K_COL1: reduce_col1<GDIV, false, FLAVOUR == R_LONG>(s, p, blk * tftq_col1_rows_per_wg(ST_R), tid); break;
     default: break;
     }
 }
