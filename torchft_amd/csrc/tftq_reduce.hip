@@ -450,17 +450,22 @@ DEV void reduce_row(const Seg &s, const KParams &p, int j, int lane, float *lds)
         };
         load_batch(kc);
 
-        const DivCoef c = make_div(my_scale);
-        if (__builtin_amdgcn_ballot_w64(!c.fast) != 0) {  // some peer needs the plain divide
-            reduce_row_slow<TEAM, GDIV>(s, p, j, lane, lds);
-            return;
+        float cr = 1.0f, cl = 0.0f;
+        {
+            const DivCoef c = make_div(my_scale);
+            cr = c.r;
+            cl = c.r_lo;
+            if (__builtin_amdgcn_ballot_w64(!c.fast) != 0) {  // some peer needs the plain divide
+                reduce_row_slow<TEAM, GDIV>(s, p, j, lane, lds);
+                return;
+            }
         }
         for (int k0 = kc; k0 < kend; k0 += PB) {
             if (k0 != kc) load_batch(k0);
 #pragma unroll
             for (int b = 0; b < PB; b++) {
                 if (k0 + b < kend) {
-                    const float pr = bcast_lane(c.r, k0 + b - kc), pl = bcast_lane(c.r_lo, k0 + b - kc);
+                    const float pr = bcast_lane(cr, k0 + b - kc), pl = bcast_lane(cl, k0 + b - kc);
 #pragma unroll
                     for (int u = 0; u < UNITS; u++) accumulate16(acc[u], w[b][u], pr, pl);
                 }
