@@ -48,3 +48,24 @@ def test_one_column_of_few_and_many_rows(q, oracle, ws, op, long_list):  # noqa:
             t[::5] = 0.0
         base.append(ts)
     full_check(q, oracle, [base[p % len(base)] for p in range(ws)], ws, op, sorted({0, ws - 1}))
+
+
+@pytest.mark.parametrize("plain_divide", [False, True])
+@pytest.mark.parametrize("long_list", [False, True])
+@pytest.mark.parametrize("ws,op", [(1, ReduceOp.SUM), (2, ReduceOp.AVG), (3, ReduceOp.AVG), (4, ReduceOp.SUM)])
+def test_rows_side_by_side_in_small_groups(q, oracle, ws, op, long_list, plain_divide):  # noqa: F811
+    # rows per slot on both sides of 256 workgroups of teams of 1, 2, 4, 8, 16 and 32 lanes, and
+    # remainders of a wavefront's rows
+    shapes = [(65535 * ws, 13), (65537 * ws, 14), (65536 * ws, 16), (32771 * ws, 19), (16383 * ws, 48), (16384 * ws, 46),
+              (16389 * ws, 60), (8193 * ws, 65), (8195 * ws, 128), (4101 * ws - ws // 2, 130), (2048 * ws, 511), (2055 * ws, 257)]
+    shapes = shapes + [(3, 40)] * 8 if long_list else shapes[ws % 2::2]
+    g = torch.Generator().manual_seed(ws)
+    peers = []
+    for p in range(ws):
+        ts = [torch.randn(s, generator=g) * (1 + p) for s in shapes]
+        for t in ts:
+            t[len(t) // 3] = -0.0
+            if plain_divide:
+                t[len(t) // 2] *= 1e-30
+        peers.append([t.to(torch.bfloat16) for t in ts])
+    full_check(q, oracle, peers, ws, op, sorted({0, ws - 1}))

@@ -86,6 +86,20 @@ TFTQ_HD static inline int tftq_reduce_rows_at_once(uint8_t kind, int ndw, int ws
     return 1;
 }
 
+// Reduce, teams of 2 to 32 lanes with one vector per lane and peer: in groups of up to 2 peers a team
+// takes 4 rows at once, so that a lane has 8 loads in flight and not 2 (reduce_rows_side).  Only
+// tensors with work for 256 workgroups without that: a smaller one keeps all its teams.  2 peers,
+// [524288, 200] 49.5 -> 36.5 us, [262144, 400] 48.0 -> 33.1, [2097152, 60] 49.6 -> 44.7; not for a lane
+// per row ([4194304, 14] 27.8 -> 30.4) and not two rows for 4 peers ([2097152, 60] 37.2 -> 40.0).
+constexpr int TFTQ_R_SIDE_ROWS = 4;
+TFTQ_HD static inline int tftq_reduce_rows_side(uint8_t kind, int ndw, int slice_rows, int ws)
+{
+    if (kind != K_GEN32 && kind != K_GEN16 && kind != K_GEN8 && kind != K_GEN4 && kind != K_GEN2) return 1;
+    const int team = tftq_team_of(kind);
+    const bool side = ws <= 2 && ndw <= 4 * team && (int64_t)slice_rows * team >= 256 * TFTQ_WG;
+    return side ? TFTQ_R_SIDE_ROWS : 1;
+}
+
 // K_VECS: a row of nvec (1..32) 16-byte vectors is owned by a team of 2^lt lanes (the
 // smallest of 1, 2, 4, 8, 16 that holds it with one vector per lane; 16 lanes with two
 // vectors each for 17 to 24 vectors, 32 lanes for 25 to 32), every lane holds c (1 or 2)
@@ -182,7 +196,9 @@ static inline int tftq_rows_per_wg(const Seg &s, int st, int esz, int ws)
     if (s.kind[st] == K_TILE) return TFTQ_TILE_ROWS;
     if (s.kind[st] == K_VECS) return tftq_small_rows_per_wg(tftq_small_nvec(s.n, esz), st);
     const int teams = TFTQ_WG / tftq_team_of(s.kind[st]);
-    if (st == ST_R) return teams * tftq_reduce_rows_at_once(s.kind[st], s.row_bytes / 4 - 1, ws);
+    if (st == ST_R)
+        return teams * tftq_reduce_rows_at_once(s.kind[st], s.row_bytes / 4 - 1, ws) *
+               tftq_reduce_rows_side(s.kind[st], s.row_bytes / 4 - 1, s.slice_rows, ws);
     return teams;
 }
 

@@ -131,8 +131,8 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
     // and the next 8).  218 M bf16 elements, 8 peers, a lane per row against the team: 24 columns
     // 81.1 -> 66.7 us, 28: 89.2 -> 64.4, 32: 65.0 -> 64.4, 44: 92.1 -> 68.7, 60: 95.6 -> 64.7, 64:
     // 70.6 -> 65.0.  45 to 48 columns are three whole vectors, of which a lane alone wastes none:
-    // [2097152, 48], 4, 8 and 16 peers: 33.1 -> 31.0 us, 29.6 -> 28.2, 27.4 -> 29.8; in a tensor of
-    // a few rows the lane alone waits 33 us for its 16 peers, the team 7 us.
+    // [2097152, 48], 2, 4, 8 and 16 peers: 41.1 -> 38.6 us, 33.1 -> 31.2, 29.6 -> 28.2, 27.7 -> 30; in a
+    // tensor of a few rows the lane alone waits 33 us for its 16 peers, the team 7 us.
     if (ndw > 8 && ndw <= 16) return K_GEN4;
     if (ndw > 4 && ndw <= 8) return K_GEN2;
     if (ndw <= 16) return K_GEN1;

@@ -687,6 +687,90 @@ DEV void reduce_rows_narrow(const Seg &s, const KParams &p, int j, int lane, flo
     if (valid && lane == 0) orow[0] = as_u(s2);  // :375; all lanes read the old scale before team_max
 }
 
+// One or two peers: four rows of a team at once (tftq_reduce_rows_side), one vector per lane and
+// peer, the loads of all rows issued together: 8 per lane, where a row alone has 2.
+// Rows j0, j0 + step, ...: neighbouring teams' rows are neighbours.  The sums of one row at a time
+// are in registers.  Rows past the end of the tensor are given the last row and store nothing.
+template <int TEAM, bool GDIV>
+DEV void reduce_rows_side(const Seg &s, const KParams &p, int j0, int step, int lane, float *lds)
+{
+    constexpr int ROWS = TFTQ_R_SIDE_ROWS, PEERS = 2, N = ROWS * PEERS, NS = N > TEAM ? N / TEAM : 1;  // scales per lane
+    const int ndw = (s.row_bytes >> 2) - 1;  // >= 4 here
+    const int ws = p.ws;
+    const int doff = min(4 * lane, ndw - 4);  // the last vector ends with the row (see reduce_rows)
+    const u32 padmask = (doff == ndw - 4 && (s.n & 3)) ? (1u << (8 * (s.n & 3))) - 1u : 0xFFFFFFFFu;
+    auto row_off = [&](int r) { return s.slot_off + (int64_t)min(j0 + r * step, s.slice_rows - 1) * s.row_bytes; };
+
+    float raw[NS];  // scale number r * PEERS + k, of row r and peer k, in lane (number % TEAM)
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        const int i = lane % N + q * TEAM;
+        raw[q] = as_f(peer_row(p, min(i % PEERS, ws - 1), row_off(i / PEERS))[0]);
+    }
+    u32x4 w[ROWS][PEERS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        const int64_t off = row_off(r);
+#pragma unroll
+        for (int k = 0; k < PEERS; k++)
+            w[r][k] = LOAD_STREAM((GLOBAL const u32x4_a4 *)(peer_row(p, min(k, ws - 1), off) + 1 + doff));
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all loads are issued before anything below
+
+    DivCoef c[NS];
+    bool fast = true;
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        c[q] = make_div(raw[q] == 0.0f ? 1.0f : raw[q]);  // padding rows (:419)
+        fast = fast && c[q].fast;
+    }
+    if (__builtin_amdgcn_ballot_w64(!fast) != 0) {  // some peer of some row needs the plain divide
+#pragma nounroll
+        for (int r = 0; r < ROWS; r++)
+            if (j0 + r * step < s.slice_rows) reduce_row_slow<TEAM, GDIV>(s, p, j0 + r * step, lane, lds);
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        float acc[16];  // set by the first peer
+#pragma unroll
+        for (int k = 0; k < PEERS; k++) {
+            if (k < ws) {
+                const int i = r * PEERS + k;
+                const float pr = team_bcast<TEAM>(c[i / TEAM].r, i % TEAM), pl = team_bcast<TEAM>(c[i / TEAM].r_lo, i % TEAM);
+                u32x4 v = w[r][k];
+                v.w &= padmask;
+                if (k == 0) accumulate16<true>(acc, v, pr, pl);
+                else accumulate16<false>(acc, v, pr, pl);
+            }
+        }
+        float amax = 0.0f;  // duplicates held by lanes past the row's end do not change it
+#pragma unroll
+        for (int e = 0; e < 16; e++) amax = fmaxf(amax, __builtin_fabsf(acc[e]));
+        amax = team_max<TEAM>(amax, lds);
+        const float s2 = calc_scale(amax_div<GDIV>(amax, p));  // :340
+        const bool valid = j0 + r * step < s.slice_rows;
+        GLOBAL u32 *orow = as_global<u32>(p.packed + (int64_t)p.rank * p.slot_size + row_off(r));
+        const u32x4 o = requant16<GDIV>(acc, s2, p);
+        if (valid && 4 * lane < ndw) STORE_CODES(o, (GLOBAL u32x4_a4 *)(orow + 1 + doff));
+        if (valid && lane == 0) orow[0] = as_u(s2);  // :375; all loads of the row came before
+    }
+}
+
+// The rows of a wavefront's teams, side by side; false when the tensor's rows go one at a time.
+template <int TEAM, bool GDIV>
+DEV bool reduce_side(const Seg &s, const KParams &p, int blk, int tid, float *lds)
+{
+    constexpr int TW = 64 / TEAM;  // teams per wavefront
+    const int rows = tftq_reduce_rows_side(s.kind[ST_R], (s.row_bytes >> 2) - 1, s.slice_rows, p.ws);  // same for all
+    if (rows == 1) return false;
+    const int first = (blk * 4 + __builtin_amdgcn_readfirstlane(tid >> 6)) * TW * rows;
+    if (first >= s.slice_rows) return true;  // the whole wavefront leaves
+    const int j0 = first + (tid & 63) / TEAM;
+    reduce_rows_side<TEAM, GDIV>(s, p, j0, TW, tid % TEAM, lds);
+    return true;
+}
+
 // Rows of up to 16 * TEAM bytes of codes in groups of more peers than a team (or the registers)
 // holds at once: one vector per lane and peer, R_CHUNK peers at a time, the next chunk's scales
 // and codes in flight while the current one is accumulated.  Lane l of a team fetches the scales
@@ -1333,6 +1417,7 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : FLAVOUR == R_ONE ?
             if (ndw > 4 * TEAM) {  // three vectors per lane (see pick_reduce_kind)
                 if (p.ws <= TEAM) reduce_rows_roll<TEAM, 3, GDIV>(s, p, min(j, s.slice_rows - 1), tid % TEAM, lds, j < s.slice_rows);
                 else if (j < s.slice_rows) reduce_row_slow<TEAM, GDIV>(s, p, j, tid % TEAM, lds);
+            } else if (reduce_side<TEAM, GDIV>(s, p, blk, tid, lds)) {
             } else if (p.ws <= TEAM) {
                 TFTQ_REDUCE_ROWS(TEAM, 1, s, p, min(j, s.slice_rows - 1), tid % TEAM, lds, j < s.slice_rows);
             } else if (TEAM == 8 && p.ws <= 16) {
@@ -1348,11 +1433,13 @@ __global__ __launch_bounds__(TFTQ_WG, FLAVOUR == R_WIDE ? 2 : FLAVOUR == R_ONE ?
     }
     case K_GEN4: {  // one row per team of 4 lanes
         const int j = blk * 64 + (tid >> 2);
+        if (reduce_side<4, GDIV>(s, p, blk, tid, lds)) break;
         TFTQ_REDUCE_NARROW(4, s, p, min(j, s.slice_rows - 1), tid & 3, lds, j < s.slice_rows);
         break;
     }
     case K_GEN2: {  // one row per pair of lanes
         const int j = blk * 128 + (tid >> 1);
+        if (reduce_side<2, GDIV>(s, p, blk, tid, lds)) break;
         TFTQ_REDUCE_NARROW(2, s, p, min(j, s.slice_rows - 1), tid & 1, lds, j < s.slice_rows);
         break;
     }
