@@ -50,3 +50,32 @@ def test_transposed_matrices(q, oracle, dtype, ws, long_list):  # noqa: F811
     q.fused_dequantize_from_fp8(list(gpu), packed.cuda(), ws, divide_by=3)
     for v, c, s in zip(gpu_views, views, shapes):  # (torch drops the sign of some fp16 zeros: compared as numbers)
         assert torch.equal(v, c.cuda() / 3), f"dequantize and divide {s}"
+
+
+def test_reduce_static_takes_2800_transposed_tensors():
+    """The index of quantize's second launch, which reduce does not read, is not part of what has to
+    fit the library's fixed array: a list whose whole table does not."""
+    import ctypes
+
+    from torchft_amd import _lib
+    L = _lib.load()
+    T, m, n, ws, rank = 2800, 1000, 400, 2, 1
+    shapes = (ctypes.c_int64 * (2 * T))(*([m, n] * T))
+    strides = (ctypes.c_int64 * (2 * T))(*([1, m] * T))
+    h = ctypes.c_void_p()
+    assert L.tftq_plan_create(2, T, shapes, strides, ws, ctypes.byref(h)) == 0
+    size, nbytes = L.tftq_plan_output_size(h), L.tftq_plan_table_bytes(h)
+    assert nbytes > 512 * 1024
+    x = (torch.randn(n, m, generator=torch.Generator().manual_seed(1)) * 0.1).to(torch.bfloat16).cuda()
+    host = (ctypes.c_uint8 * nbytes).from_address(L.tftq_plan_table_host(h))
+    table = torch.frombuffer(host, dtype=torch.uint8).cuda()
+    pointers = torch.full((T,), x.data_ptr(), dtype=torch.int64, device="cuda")  # one matrix 2800 times
+    a = torch.empty(size, dtype=torch.uint8, device="cuda")
+    stream, dev = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), torch.cuda.current_device()
+    assert L.tftq_quantize(h, None, table.data_ptr(), pointers.data_ptr(), a.data_ptr(), size, dev, stream) == 0
+    b = a.clone()
+    assert L.tftq_reduce(h, table.data_ptr(), a.data_ptr(), size, rank, 1, dev, stream) == 0
+    assert L.tftq_reduce_static(h, b.data_ptr(), size, rank, 1, dev, stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+    L.tftq_plan_destroy(h)

@@ -304,6 +304,7 @@ struct tftq_plan {
     TableIndex index[N_LAUNCHES];  // device table only
     std::vector<Seg> segs;
     std::vector<uint8_t> blob;  // host image of the device table (nseg > TFTQ_N_INLINE)
+    size_t static_bytes;        // what tftq_reduce_static writes of it: all but the index of quantize's second launch
 };
 
 // Kernel parameters common to the three stages.

@@ -303,14 +303,19 @@ static int build_table(tftq_plan *p, const int32_t (*wgs)[N_LAUNCHES])
         p->index[st].per_xcd = (int32_t)(turns << cs);
     }
     size_t bytes = nseg * sizeof(Seg);
-    for (int st = 0; st < launches; st++) {
-        p->index[st].sorted_off = (int64_t)bytes;
-        bytes += nseg * sizeof(SortEnt);
-    }
-    for (int st = 0; st < launches; st++) {
-        p->index[st].map_off = (int64_t)bytes;
-        bytes += map[st].size() * sizeof(MapEnt);
-    }
+    auto place = [&](int begin, int end) {
+        for (int st = begin; st < end; st++) {
+            p->index[st].sorted_off = (int64_t)bytes;
+            bytes += nseg * sizeof(SortEnt);
+        }
+        for (int st = begin; st < end; st++) {
+            p->index[st].map_off = (int64_t)bytes;
+            bytes += map[st].size() * sizeof(MapEnt);
+        }
+    };
+    place(0, 3);
+    p->static_bytes = bytes;
+    place(3, launches);  // quantize's second launch, last: tftq_reduce_static leaves it out
     p->blob.resize(bytes);
     memcpy(p->blob.data(), p->segs.data(), nseg * sizeof(Seg));
     for (int st = 0; st < launches; st++) {

@@ -1576,7 +1576,7 @@ extern "C" int tftq_reduce_static(const tftq_plan *plan, void *packed, int64_t p
     hipStream_t st = (hipStream_t)stream;
     if (plan->nseg <= TFTQ_N_INLINE || plan->nwg[ST_R] == 0)  // descriptors in the kernel arguments: no scratch
         return reduce_launch(plan, nullptr, packed, packed_bytes, rank, is_avg, st);
-    if (plan->blob.size() > (size_t)TFTQ_STATIC_TABLE_BYTES) return TFTQ_E_TOOBIG;
+    if (plan->static_bytes > (size_t)TFTQ_STATIC_TABLE_BYTES) return TFTQ_E_TOOBIG;
     if (packed_bytes != plan->output_size) return TFTQ_E_SIZE;  // before anything is queued
     if (rank < 0 || rank >= plan->ws || (!packed && plan->output_size != 0) || ((uintptr_t)packed & 3) != 0)
         return TFTQ_E_ARG;
@@ -1593,8 +1593,8 @@ extern "C" int tftq_reduce_static(const tftq_plan *plan, void *packed, int64_t p
         if (e == hipErrorNotReady) return TFTQ_E_BUSY;  // an earlier call's kernel, on another stream, may still read the array
         if (e != hipSuccess) return (int)e;
     }
-    // the whole image every time: the array keeps whatever the last call, of any plan, left there
-    rc = tftq_put_bytes(t->ptr, plan->blob.data(), plan->blob.size(), st);
+    // the image anew every time: the array keeps whatever the last call, of any plan, left there
+    rc = tftq_put_bytes(t->ptr, plan->blob.data(), plan->static_bytes, st);
     if (rc) return rc;
     rc = reduce_launch(plan, t->ptr, packed, packed_bytes, rank, is_avg, st);
     if (!captured) {
