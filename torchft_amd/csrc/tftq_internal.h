@@ -35,7 +35,7 @@ enum : uint8_t {
     K_GEN32 = 10,  // 32 lanes per row (reduce only)
     K_GEN64 = 6,   // one wavefront per row
     K_GEN256 = 7,  // one workgroup per row (reduce only)
-    K_COL1 = 8,    // rows of a single column (1-D tensors): 4 rows per lane, 1024 per workgroup
+    K_COL1 = 8,    // rows of a single column (1-D tensors); reduce: 4 rows per lane, 1024 per workgroup
     K_COLS = 17,   // columns contiguous in memory (row stride 1: a transposed matrix), quantize: a workgroup of 512 lanes per 16 (fp32: 8) rows
     K_TILE = 18,   // the same in dequantize: a workgroup per tile of 64 rows and 256 columns
 };
@@ -271,6 +271,7 @@ struct Dealt {
 //   Seg      segs[nseg]                    in list order
 //   SortEnt  sorted[3][nseg]               per stage, in workgroup order
 //   MapEnt   map[3][...]                   per stage: bucket of 2^shift workgroups -> position
+//   (and, for a list with K_COLS tensors, sorted[] and map[] of quantize's second launch)
 // and a workgroup finds its segment with one load of map[b], map[b+1] and, only
 // if those differ, a binary search of sorted[] between the two positions.
 struct SortEnt { int32_t begin, seg; };  // first workgroup of the segment, index into segs[]
