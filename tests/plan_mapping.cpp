@@ -181,8 +181,10 @@ static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype)
                 const int64_t blk = (int64_t)vb - p->segs[(size_t)sg].wg_begin[st];
                 if (pieces && blk >= (int64_t)seen[(size_t)sg].size()) {
                     // padding in front of a tensor whose kind needs whole workgroups: it must
-                    // fall to a kind whose wavefronts simply find no row
-                    if (blk >= 0 && !tftq_reduce_kind_has_barriers(p->segs[(size_t)sg].kind[st]) && blk < (int64_t)seen[(size_t)sg].size() + 3)
+                    // fall to a kind whose wavefronts simply find no row, of a tensor that has
+                    // rows (a lane without a row of its own reads the tensor's last one)
+                    if (blk >= 0 && !tftq_reduce_kind_has_barriers(p->segs[(size_t)sg].kind[st]) && blk < (int64_t)seen[(size_t)sg].size() + 3 &&
+                        p->segs[(size_t)sg].slice_rows > 0)
                         continue;
                 }
                 if (blk < 0 || blk >= (int64_t)seen[(size_t)sg].size() || seen[(size_t)sg][(size_t)blk]) {
@@ -237,6 +239,15 @@ int main()
         s.push_back(0);
         s.push_back(5);
         if (check_plan(s, 16, TFTQ_BF16)) return 1;
+        plans++;
+    }
+    {   // an empty tensor whose place by weight is right before a row that needs a whole workgroup
+        std::vector<int64_t> s = {0, 12, 5, 13, 5, 2100};
+        for (int i = 0; i < 15; i++) {
+            s.push_back(5);
+            s.push_back(4);
+        }
+        if (check_plan(s, 8, TFTQ_BF16)) return 1;
         plans++;
     }
     // random lists on both sides of the inline limit

@@ -6,6 +6,7 @@
 // the reference keeps them in int32 (:514-515).
 
 #include <limits.h>
+#include <math.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -168,7 +169,10 @@ static double wg_weight(const Seg &s, int st, int esz, int ws)
 // The order in which a stage works through the segments.  Reduce: by workgroup
 // weight, heaviest first (equal weights keep the list order), so that the last
 // workgroups to finish are light; its weights differ by orders of magnitude
-// within one list.  Quantize and dequantize keep the list order: their
+// within one list.  Empty tensors come before all others: the pieces that pad the numbering up to a
+// whole workgroup (build_table) belong to the tensor in front of them, whose lanes without a row of
+// their own read its last row, so it must have one.
+// Quantize and dequantize keep the list order: their
 // workgroups are all of similar weight, and sorting them measured slower.
 static void work_order(const tftq_plan *p, int st, std::vector<int32_t> &ord)
 {
@@ -176,7 +180,8 @@ static void work_order(const tftq_plan *p, int st, std::vector<int32_t> &ord)
     ord.resize((size_t)p->nseg);
     for (int i = 0; i < p->nseg; i++) {
         ord[(size_t)i] = i;
-        w[(size_t)i] = wg_weight(p->segs[(size_t)i], st, p->esz, p->ws);
+        const Seg &s = p->segs[(size_t)i];
+        w[(size_t)i] = s.m > 0 ? wg_weight(s, st, p->esz, p->ws) : HUGE_VAL;
     }
     if (st != ST_R) return;
     std::stable_sort(ord.begin(), ord.end(), [&](int32_t a, int32_t b) { return w[(size_t)a] > w[(size_t)b]; });
