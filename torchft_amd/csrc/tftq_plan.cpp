@@ -157,13 +157,10 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
     return K_GEN256;
 }
 
-// Bytes one workgroup of segment s moves in a stage.
-static double wg_weight(const Seg &s, int st, int esz, int ws)
+// Bytes one workgroup of segment s moves in reduce.
+static double reduce_weight(const Seg &s, int esz, int ws)
 {
-    double rows = (double)tftq_rows_per_wg(s, st, esz, ws);
-    if (st == ST_D) rows /= tftq_d_row_parts(s.kind[ST_D], s.n, esz);
-    if (st == ST_R) return rows * (double)s.row_bytes * (ws + 1);
-    return rows * ((double)s.n * esz + (double)s.row_bytes);
+    return (double)tftq_rows_per_wg(s, ST_R, esz, ws) * (double)s.row_bytes * (ws + 1);
 }
 
 // The order in which a stage works through the segments.  Reduce: by workgroup
@@ -176,14 +173,14 @@ static double wg_weight(const Seg &s, int st, int esz, int ws)
 // workgroups are all of similar weight, and sorting them measured slower.
 static void work_order(const tftq_plan *p, int st, std::vector<int32_t> &ord)
 {
-    std::vector<double> w((size_t)p->nseg);
     ord.resize((size_t)p->nseg);
-    for (int i = 0; i < p->nseg; i++) {
-        ord[(size_t)i] = i;
-        const Seg &s = p->segs[(size_t)i];
-        w[(size_t)i] = s.m > 0 ? wg_weight(s, st, p->esz, p->ws) : HUGE_VAL;
-    }
+    for (int i = 0; i < p->nseg; i++) ord[(size_t)i] = i;
     if (st != ST_R) return;
+    std::vector<double> w((size_t)p->nseg);
+    for (int i = 0; i < p->nseg; i++) {
+        const Seg &s = p->segs[(size_t)i];
+        w[(size_t)i] = s.m > 0 ? reduce_weight(s, p->esz, p->ws) : HUGE_VAL;
+    }
     std::stable_sort(ord.begin(), ord.end(), [&](int32_t a, int32_t b) { return w[(size_t)a] > w[(size_t)b]; });
 }
 
