@@ -5,6 +5,7 @@ import pytest
 import torch
 from torch.distributed import ReduceOp
 
+import sim_pg
 from sim_pg import SimGroup
 from test_gpu_collectives import run_ranks
 from torchft_amd import allreduce as ar
@@ -116,3 +117,106 @@ def test_shared_memory_and_storage_that_moves_in_flight(monkeypatch):
     for r in range(2):
         assert all(torch.equal(a, b) for a, b in zip(mine[r], want[r][0]))
         assert all(t._version > v for i, (t, v) in enumerate(zip(mine[r], versions[r])) if i != 1)
+
+
+class Whole:
+    """Stands for the prepared bucket of the flat buffer."""
+    ws = 2
+
+
+@pytest.mark.parametrize("count,capacity", [(16, 64), (15, 61), (16, 61), (17, 68), (40, 1 << 10)])
+def test_no_table_is_made_under_a_capture(monkeypatch, count, capacity):
+    # capacity 64 + or - 3 of tensors of 4 elements: with or without a rest that no tensor covers
+    tensors = [torch.ones(4) for _ in range(count)]
+    averaging = ar.BucketizedAllreduce(tensors, 4 * capacity)
+    bucket = averaging.buckets[0]
+    parts = len(bucket["owners"]) + (bucket["used"] < bucket["flat"].numel())
+    capturing = [True]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(ar._q, "prepare", lambda tensors, ws: type("Prepared", (), {"list": tensors})())
+    made = averaging._in_place(bucket, Whole)
+    assert (made is None) == (parts > 16)
+    if made is not None:
+        assert len(made._parts.list) == parts and bucket["captured"] == [made]
+        return
+    assert not bucket["piecewise"] and not bucket["captured"]
+    capturing[0] = False
+    made = averaging._in_place(bucket, Whole)   # an eager step makes the table ...
+    assert len(made._parts.list) == parts and not bucket["captured"]
+    capturing[0] = True
+    assert averaging._in_place(bucket, Whole) is made and bucket["captured"] == [made]   # ... for captures after it
+    bucket["owners"][3].data = torch.ones(4)
+    assert averaging._in_place(bucket, Whole) is None
+
+
+class OneRank:
+    """Rank 0 of a group whose other ranks send what `others` holds."""
+
+    def __init__(self, others):
+        self.others = others
+
+    def rank(self):
+        return 0
+
+    def size(self):
+        return len(self.others)
+
+    def alltoall_base(self, output, input, output_splits, input_splits, opts=None):
+        output.copy_(self.others)
+        output[0].copy_(input[0])
+        return sim_pg._DoneWork()
+
+    def allgather_into_tensor_coalesced(self, outputs, inputs, opts=None):
+        outputs[0].copy_(self.others)
+        outputs[0][:1].copy_(inputs[0])
+        return sim_pg._DoneWork()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [9, 40])
+@pytest.mark.parametrize("warm", [False, True])
+def test_a_step_under_a_capture(count, warm):
+    """The graph replayed between eager steps, each against the same step by way of the copies."""
+    g = torch.Generator().manual_seed(count)
+    start = [torch.randn(3 * i % 50 + 1, 5, generator=g) for i in range(count)]
+    total = sum(t.numel() for t in start)
+    peer = ar._q.fused_quantize_into_fp8([torch.randn(total, generator=g).cuda()], 2).view(2, -1)
+    want = [t.cuda() for t in start]
+    copies = ar.BucketizedAllreduce(want, 4 * total)
+    copies._in_place = lambda bucket, whole: None
+    mine = [t.cuda() for t in start]
+    averaging = ar.BucketizedAllreduce(mine, 4 * total)
+
+    def step(averaging):
+        for w in averaging.allreduce(OneRank(peer), 2):
+            w.wait()
+
+    def check(what):
+        torch.cuda.synchronize()
+        for a, b in zip(mine, want):
+            assert torch.equal(a, b), what
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        if warm:
+            step(averaging)
+            step(copies)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            step(averaging)
+        assert bool(averaging.buckets[0]["captured"]) == (warm or count <= 16)
+        check("the capture itself")
+        step(averaging)   # eager, on the stream of the capture, before the first replay
+        step(copies)
+        check("eager step behind the capture")
+        for k in range(3):
+            for t, w in zip(mine, want):
+                t.mul_(1.5)
+                w.mul_(1.5)
+            graph.replay()
+            step(copies)
+            check(f"replay {k}")
+            step(averaging)
+            step(copies)
+            check(f"eager step {k}")
