@@ -131,7 +131,7 @@ class _Plan:
                 if entry is None:
                     host = (ctypes.c_uint8 * self.table_bytes).from_address(
                         self._lib.tftq_plan_table_host(self.handle))
-                    staged = torch.empty(self.table_bytes, dtype=torch.uint8, pin_memory=True)
+                    staged = torch.empty(self.table_bytes, dtype=torch.uint8, device="cpu", pin_memory=True)
                     staged.copy_(torch.frombuffer(host, dtype=torch.uint8))
                     with torch.cuda.device(device):
                         table = torch.empty(self.table_bytes, dtype=torch.uint8, device=device)
@@ -274,7 +274,8 @@ class _StreamPointers:
     __slots__ = ("dev", "held", "lock")
 
     def __init__(self, plan: _Plan, device: torch.device, table: torch.Tensor) -> None:
-        with torch.cuda.device(device):
+        # (written again by later calls, in whatever mode they come: no inference tensor)
+        with torch.cuda.device(device), torch.inference_mode(False):
             stream = torch.cuda.current_stream(device)
             self.dev = torch.empty(plan.n_tensors, dtype=torch.int64, device=device)
             # both are read by kernels on this stream, which need not be the one they were allocated on
@@ -299,7 +300,7 @@ def _upload(plan: _Plan, ptrs, dev: torch.Tensor, raw_stream: int, capturing: bo
         _check(plan._lib.tftq_upload_pointers(plan.handle, ptrs, dev.data_ptr(), dev.device.index, raw_stream),
                "tftq_upload_pointers")
         return
-    staged = torch.empty(n, dtype=torch.int64, pin_memory=True)
+    staged = torch.empty(n, dtype=torch.int64, device="cpu", pin_memory=True)  # whatever the default device
     ctypes.memmove(staged.data_ptr(), ptrs, 8 * n)
     dev.copy_(staged, non_blocking=True)  # the pinned allocator keeps `staged` until then
 
@@ -417,7 +418,7 @@ class PreparedBucket:
             table, ready = plan.table_on(device)
             self._table = table
             self._table_ready = ready
-            with torch.cuda.device(device):
+            with torch.cuda.device(device), torch.inference_mode(False):  # written by the first call
                 self._ptrs_dev = torch.empty(plan.n_tensors, dtype=torch.int64, device=device)
 
     # -- properties of the layout ------------------------------------------------------
