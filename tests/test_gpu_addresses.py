@@ -2,6 +2,7 @@
 pinned memory: new addresses on every call, on several streams, named functions and buckets."""
 
 import contextlib
+import threading
 
 import pytest
 import torch
@@ -56,3 +57,58 @@ def test_addresses_in_other_modes(n, way, first, then):
             else:
                 got = q.fused_quantize_into_fp8(lists[k], 1)
         assert torch.equal(got, want[k]), (k, mode)
+
+
+@pytest.mark.parametrize("side", [False, True])
+@pytest.mark.parametrize("n", [q._COPY_FROM - 1, q._COPY_FROM, 9000])
+def test_new_addresses_while_another_thread_captures(n, side):
+    """A capture in global mode, and calls of this thread meanwhile with new addresses every time,
+    more of them than the pinned allocator has memory of that size for."""
+    g = torch.Generator().manual_seed(n)
+    lists = [[torch.randn(2, 5, generator=g).cuda() for _ in range(n)] for _ in range(6)]
+    want = [q.fused_quantize_into_fp8([torch.cat(ts)], 1) for ts in lists]
+    stream = torch.cuda.Stream() if side else torch.cuda.current_stream()
+    with torch.cuda.stream(stream):
+        q.fused_quantize_into_fp8(lists[0], 1)   # the plan's table and this stream's buffer
+        buckets = [q.prepare(ts, 1) for ts in lists]
+        outs = [torch.empty_like(w) for w in want]
+        # what the calls below allocate: torch may not ask for more then, and gives back whole segments before
+        spare = [torch.empty_like(w) for w in want for _ in range(3)]
+        del spare[::2]
+    torch.cuda.synchronize()
+    x = torch.arange(1024, device="cuda", dtype=torch.float32)
+    y = torch.zeros_like(x)
+    torch.cuda.synchronize()
+    graph, began, finish, failed = torch.cuda.CUDAGraph(), threading.Event(), threading.Event(), []
+
+    def capture():
+        try:
+            with torch.cuda.graph(graph, capture_error_mode="global"):
+                y.copy_(x * 2)
+                began.set()
+                finish.wait(60)
+                y.add_(1)
+        except Exception as e:  # reported below
+            failed.append(e)
+            began.set()
+
+    thread = threading.Thread(target=capture)
+    thread.start()
+    began.wait(60)
+    got = []
+    try:
+        with torch.cuda.stream(stream):
+            for ts, bucket, out in zip(lists, buckets, outs):
+                got.append(q.fused_quantize_into_fp8(ts, 1))
+                got.append(bucket.quantize(out))
+    finally:
+        finish.set()
+        thread.join()
+    assert not failed, failed
+    torch.cuda.synchronize()
+    assert all(torch.equal(packed, want[k // 2]) for k, packed in enumerate(got))
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, x * 2 + 1)

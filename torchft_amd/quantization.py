@@ -290,6 +290,7 @@ class _StreamPointers:
 # 448 of them (new addresses on every call, host time of quantize: 500 tensors 20.5 us by launches, 21.5
 # by a copy; 1000: 34.6, 27.3; 3682: 65, 46; 10 000: 159, 90).
 _COPY_FROM = 2 * 448 + 1
+_CAPTURE_RELAXED = 2  # hipStreamCaptureModeRelaxed
 
 
 def _upload(plan: _Plan, ptrs, dev: torch.Tensor, raw_stream: int, capturing: bool) -> None:
@@ -300,9 +301,19 @@ def _upload(plan: _Plan, ptrs, dev: torch.Tensor, raw_stream: int, capturing: bo
         _check(plan._lib.tftq_upload_pointers(plan.handle, ptrs, dev.data_ptr(), dev.device.index, raw_stream),
                "tftq_upload_pointers")
         return
-    staged = torch.empty(n, dtype=torch.int64, device="cpu", pin_memory=True)  # whatever the default device
-    ctypes.memmove(staged.data_ptr(), ptrs, 8 * n)
-    dev.copy_(staged, non_blocking=True)  # the pinned allocator keeps `staged` until then
+    # The pinned allocator may allocate and ask events for their state, which a stream capture of any
+    # other thread forbids this one (and breaks at) unless this thread's own capture mode is relaxed.
+    # Nothing of it touches the captured work: the memory and the events are this call's.
+    exchange = plan._lib.hipThreadExchangeStreamCaptureMode  # of the HIP runtime that the library is linked to
+    mode = ctypes.c_int(_CAPTURE_RELAXED)
+    _check(exchange(ctypes.byref(mode)), "hipThreadExchangeStreamCaptureMode")
+    try:
+        staged = torch.empty(n, dtype=torch.int64, device="cpu", pin_memory=True)  # whatever the default device
+        ctypes.memmove(staged.data_ptr(), ptrs, 8 * n)
+        dev.copy_(staged, non_blocking=True)  # the pinned allocator keeps its memory until then
+        del staged
+    finally:
+        exchange(ctypes.byref(mode))
 
 
 _memcmp = ctypes.CDLL(None).memcmp
