@@ -3,6 +3,9 @@ restatement of torchft/local_sgd.py:499-556, on the CPU with a stand-in
 all-reduce (no GPU, no process group), and the argument checks of the managed
 all-reduce (manager.py:422-429)."""
 
+import ctypes
+import threading
+
 import pytest
 import torch
 from torch.distributed import ReduceOp
@@ -124,3 +127,45 @@ def test_average_and_participation():
         lambda f: order.append("b"))
     w.wait()
     assert order == [("a", 1.0), "b"]
+
+
+def test_capture_is_asked_of_the_tensors_device(monkeypatch):
+    """The current device is 0 and its stream is captured; the current stream of device 1 is not."""
+    from torchft_amd import quantization as q
+    current = [0]
+
+    class Guard:
+        def __init__(self, device):
+            self.index = device.index
+
+        def __enter__(self):
+            self.before, current[0] = current[0], self.index
+
+        def __exit__(self, *exc):
+            current[0] = self.before
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    monkeypatch.setattr(torch.cuda, "device", Guard)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: current[0] == 0)
+    assert q._capturing(torch.device("cuda", 0)) and not q._capturing(torch.device("cuda", 1))
+    assert current == [0]
+
+    # addresses of a list on device 1: not taken for captured ones, which the next call would send again
+    sent = []
+    monkeypatch.setattr(q, "_upload", lambda plan, ptrs, dev, raw, capturing: sent.append(capturing))
+
+    class Memory:
+        def data_ptr(self):
+            return 256
+
+    class Plan:
+        n_tensors = 17
+        streams = {(1, 7): type("Kept", (), {"held": None, "dev": Memory(), "lock": threading.Lock()})()}
+
+        def table_on(self, device):
+            return Memory(), type("Done", (), {"event": None})()
+
+    ptrs = (ctypes.c_void_p * 17)()
+    for _ in range(2):
+        q._long_list_args(Plan(), torch.device("cuda", 1), 7, ptrs)[2].release()
+    assert sent == [False]

@@ -132,7 +132,7 @@ def test_no_table_is_made_under_a_capture(monkeypatch, count, capacity):
     bucket = averaging.buckets[0]
     parts = len(bucket["owners"]) + (bucket["used"] < bucket["flat"].numel())
     capturing = [True]
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(ar._q, "_capturing", lambda device: capturing[0])
     monkeypatch.setattr(ar._q, "prepare", lambda tensors, ws: type("Prepared", (), {"list": tensors})())
     made = averaging._in_place(bucket, Whole)
     assert (made is None) == (parts > 16)

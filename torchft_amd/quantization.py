@@ -68,6 +68,14 @@ _PLAN_CACHE_SIZE = 4096
 _PLAN_CACHE_TENSORS = 1 << 18
 
 
+def _capturing(device: torch.device) -> bool:
+    """Whether the current stream of `device`, which need not be the current device, is being captured."""
+    if torch.cuda.current_device() == device.index:
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class _Ready:
     """An upload that kernels on other streams must wait for until it has completed."""
 
@@ -82,7 +90,7 @@ class _Ready:
         ev = self.event
         if ev is None or raw_stream == self.stream_id:  # done, or ordered by the stream itself
             return
-        if torch.cuda.is_current_stream_capturing():
+        if _capturing(stream.device):
             stream.wait_event(ev)  # a capture may wait for an outside event, but not ask about it
         elif ev.query():
             self.event = None
@@ -370,7 +378,7 @@ def _long_list_args(plan: _Plan, device: torch.device, raw_stream: int, ptrs):
         return table.data_ptr(), None, None
     sp.lock.acquire()
     try:
-        capturing = torch.cuda.is_current_stream_capturing()
+        capturing = _capturing(device)
         if capturing or sp.held is None or _memcmp(sp.held, ptrs, 8 * plan.n_tensors) != 0:
             _upload(plan, ptrs, sp.dev, raw_stream, capturing)
             # an upload that a stream capture records has not run: the next call uploads again
@@ -486,7 +494,7 @@ class PreparedBucket:
                 ready = self._ptrs_ready
                 if ready is None:
                     # the first call on this bucket writes the addresses; later calls reuse them
-                    capturing = torch.cuda.is_current_stream_capturing()
+                    capturing = _capturing(self.device)
                     _upload(self.plan, self._ptrs, self._ptrs_dev, raw_stream, capturing)
                     # Under a stream capture the upload has only been recorded (it runs with the
                     # graph, before the kernel recorded behind it): nothing is ready, and the
