@@ -104,7 +104,7 @@ class _Plan:
 
     __slots__ = ("handle", "output_size", "slot_size", "max_rows", "n_tensors", "table_bytes",
                  "tables", "_lib", "_lock", "dtype_code", "ws", "shapes", "strides", "a_shapes",
-                 "a_strides", "streams")
+                 "a_strides", "streams", "used", "cached", "short_keys")
 
     def __init__(self, lib, handle, n_tensors, dtype_code, ws, shapes, strides):
         self._lib = lib
@@ -124,6 +124,9 @@ class _Plan:
         self.max_rows = lib.tftq_plan_max_rows(handle)
         self.table_bytes = lib.tftq_plan_table_bytes(handle)
         self.tables: dict = {}  # device index -> (device tensor, _Ready)
+        self.used = False       # found by a short list since the cache last looked for a plan to let go
+        self.cached = False     # one of _plan_cache
+        self.short_keys: list = []  # its entries in _short_plans
         self._lock = threading.Lock()
 
     def table_on(self, device: torch.device):
@@ -214,26 +217,38 @@ def _plan_for(dtype: torch.dtype, ws: int, sizes_key: tuple, strides_key: tuple)
         old = _plan_cache.pop(key, None)  # another thread may have built the same plan
         if old is not None:
             _plan_cache_tensors -= old.n_tensors
-            _forget_long_plan(old)
+            _forget_plan(old)
         _plan_cache[key] = plan
+        plan.cached = True
         _plan_cache_tensors += T
         if T > _N_INLINE:
             _long_plans.setdefault((T, ws), []).insert(0, plan)
         while len(_plan_cache) > 1 and (len(_plan_cache) > _PLAN_CACHE_SIZE
                                         or _plan_cache_tensors > _PLAN_CACHE_TENSORS):
-            _, gone = _plan_cache.popitem(last=False)
+            gone_key, gone = _plan_cache.popitem(last=False)
+            if gone is plan or gone.used:  # short lists do not move what they find to the end: a second chance
+                gone.used = False
+                _plan_cache[gone_key] = gone
+                continue
             _plan_cache_tensors -= gone.n_tensors
-            _forget_long_plan(gone)
-            _short_plans.clear()
+            _forget_plan(gone)
     return plan
+
+
+def _forget_plan(plan: _Plan) -> None:  # called with _cache_lock held
+    plan.cached = False
+    for key in plan.short_keys:
+        _short_plans.pop(key, None)
+    plan.short_keys.clear()
+    _forget_long_plan(plan)
 
 
 # ---------------------------------------------------------------------------------------------
 # short lists through the three named functions
 # ---------------------------------------------------------------------------------------------
 # What _pylist.describe says of a list of up to 16 two-dimensional tensors, with the group size ->
-# the plan of an earlier call.  Every entry's plan is one of _plan_cache: emptied when that lets a
-# plan go.  One C++ walk and one look-up per call instead of the Python walk of prepare(): 2.1 to
+# the plan of an earlier call.  Every entry's plan is one of _plan_cache and goes with it; a hit marks
+# the plan as used, which keeps it there.  One C++ walk and one look-up per call instead of the Python walk of prepare(): 2.1 to
 # 2.7 us of a call's 7.4 us of host time on one tensor of 4096 elements.
 _short_plans: "dict[tuple, _Plan]" = {}
 
@@ -252,7 +267,12 @@ def _match_short_list(inputs, ws: int):
     plan = _short_plans.get(key)
     if plan is None:
         plan = prepare(inputs, ws).plan
-        _short_plans[key] = plan
+        with _cache_lock:
+            if plan.cached:  # another thread may have made the cache let go of it
+                _short_plans[key] = plan
+                plan.short_keys.append(key)
+    else:
+        plan.used = True
     return plan, device, said[2]
 
 
