@@ -6,7 +6,7 @@
 // per-XCD dealt rows; device tables: chunk dealing, bucket map, binary search,
 // and for reduce the quarters of workgroups that its wavefronts take one each)
 // and checks that every block of every tensor is visited exactly once, in all
-// three stages.  Prints "ok <plans> plans" on success.
+// three stages and in quantize's second launch.  Prints "ok <plans> plans" on success.
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -83,13 +83,15 @@ static bool locate_table(const tftq_plan *p, int st, uint32_t b, int wave, int *
     return true;
 }
 
-static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype)
+// by_columns: 0: contiguous rows, 1: every tensor stored column by column, 2: every other one
+static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype, int by_columns = 0)
 {
     const int n = (int)shapes.size() / 2;
     std::vector<int64_t> strides((size_t)n * 2);
     for (int i = 0; i < n; i++) {
-        strides[2 * (size_t)i] = shapes[2 * (size_t)i + 1];
-        strides[2 * (size_t)i + 1] = 1;
+        const bool cols = by_columns == 1 || (by_columns == 2 && i % 2);
+        strides[2 * (size_t)i] = cols ? 1 : shapes[2 * (size_t)i + 1];
+        strides[2 * (size_t)i + 1] = cols ? shapes[2 * (size_t)i] : 1;
     }
     tftq_plan *p = nullptr;
     const int rc = tftq_plan_create(dtype, n, shapes.data(), strides.data(), ws, &p);
@@ -105,7 +107,9 @@ static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype)
             return 1;
         }
     }
-    for (int st = 0; st < 3; st++) {
+    for (int st = 0; st < N_LAUNCHES; st++) {
+        if (st == ST_QC && p->nwg[st] == 0) continue;
+        const int field = st == ST_QC ? ST_Q : st;
         // blocks each segment must receive: workgroups, or quarters of workgroups (pieces)
         const bool pieces = !inl && p->index[st].pieces > 0;
         if (pieces != (!inl && st == ST_R)) {
@@ -117,9 +121,11 @@ static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype)
         for (int i = 0; i < n; i++) {
             const Seg &s = p->segs[(size_t)i];
             const int64_t m_pad = (int64_t)s.slice_rows * ws;
-            const int64_t rows = st == ST_Q ? m_pad : st == ST_R ? s.slice_rows : s.m;
-            const int per_wg = tftq_rows_per_wg(s, st, dtype == TFTQ_F32 ? 4 : 2, ws);
+            const int64_t rows = field == ST_Q ? m_pad : st == ST_R ? s.slice_rows : s.m;
+            const int per_wg = tftq_rows_per_wg(s, field, dtype == TFTQ_F32 ? 4 : 2, ws);
             int64_t blocks = (rows + per_wg - 1) / per_wg;
+            if (field == ST_Q && (s.kind[ST_Q] == K_COLS) != (st == ST_QC)) blocks = 0;  // the other launch's
+            else if (st == ST_QC) blocks = (int64_t)ws * ((s.slice_rows + per_wg - 1) / per_wg);
             if (st == ST_D) {  // long rows of dequantize are dealt to several workgroups
                 const int epv = dtype == TFTQ_F32 ? 4 : 8;
                 const int nvec = s.n / epv;
@@ -134,7 +140,7 @@ static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype)
                     printf("segment %d: %d parts for %d vectors\n", i, parts, nvec);
                     return 1;
                 }
-                blocks *= parts;
+                blocks *= s.kind[ST_D] == K_TILE ? (s.n + TFTQ_TILE_COLS - 1) / TFTQ_TILE_COLS : parts;
             }
             if (pieces) {
                 blocks = tftq_reduce_pieces(s, dtype == TFTQ_F32 ? 4 : 2, ws, blocks);
@@ -178,7 +184,7 @@ static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype)
                     printf("stage %d id %lld: segment %d\n", st, (long long)b, sg);
                     return 1;
                 }
-                const int64_t blk = (int64_t)vb - p->segs[(size_t)sg].wg_begin[st];
+                const int64_t blk = (int64_t)vb - p->segs[(size_t)sg].wg_begin[field];
                 if (pieces && blk >= (int64_t)seen[(size_t)sg].size()) {
                     // padding in front of a tensor whose kind needs whole workgroups: it must
                     // fall to a kind whose wavefronts simply find no row, of a tensor that has
@@ -213,9 +219,44 @@ static int check_plan(const std::vector<int64_t> &shapes, int ws, int dtype)
     return 0;
 }
 
+// The kinds that quantize and dequantize give `count` tensors of m rows and n columns stored column by
+// column, behind one [4096, 4096] stored by rows if `others`.
+static int check_kinds(int count, int64_t m, int64_t n, int dtype, int ws, bool others, bool cols, bool tile)
+{
+    std::vector<int64_t> shapes, strides;
+    if (others) {
+        shapes = {4096, 4096};
+        strides = {4096, 1};
+    }
+    for (int i = 0; i < count; i++) {
+        shapes.insert(shapes.end(), {m, n});
+        strides.insert(strides.end(), {1, m});
+    }
+    tftq_plan *p = nullptr;
+    if (tftq_plan_create(dtype, count + others, shapes.data(), strides.data(), ws, &p)) {
+        printf("plan_create failed\n");
+        return 1;
+    }
+    const Seg &s = p->segs.back();
+    const bool ok = (s.kind[ST_Q] == K_COLS) == cols && (s.kind[ST_D] == K_TILE) == tile && (p->nwg[ST_QC] > 0) == cols;
+    if (!ok)
+        printf("%d x [%d, %d] dtype %d ws %d others %d: kinds %d and %d\n", count, (int)m, (int)n, dtype, ws, others, s.kind[ST_Q], s.kind[ST_D]);
+    tftq_plan_destroy(p);
+    return !ok;
+}
+
 int main()
 {
     int plans = 0;
+    // which transposed tensors are worth blocks of columns: the faster side of measured pairs
+    if (check_kinds(1, 4096, 14336, TFTQ_BF16, 8, false, true, true) || check_kinds(1, 1024, 4096, TFTQ_BF16, 8, false, true, true) ||
+        check_kinds(1, 256, 8192, TFTQ_BF16, 16, true, true, true) || check_kinds(1, 4096, 4096, TFTQ_F32, 64, true, true, true) ||
+        check_kinds(1, 1024, 128, TFTQ_BF16, 8, false, true, true) || check_kinds(100, 1024, 256, TFTQ_F32, 16, false, true, true) ||
+        check_kinds(10000, 32, 32, TFTQ_BF16, 16, false, false, false) || check_kinds(10000, 32, 32, TFTQ_F32, 2, false, false, false) ||
+        check_kinds(1, 100000, 32, TFTQ_F32, 8, false, false, true) || check_kinds(1000, 128, 128, TFTQ_BF16, 64, false, false, true) ||
+        check_kinds(1000, 64, 256, TFTQ_BF16, 64, false, false, true) || check_kinds(1, 64, 64, TFTQ_BF16, 8, true, false, false) ||
+        check_kinds(1, 256, 256, TFTQ_BF16, 8, false, false, false) || check_kinds(512, 16, 1024, TFTQ_F32, 64, true, false, true))
+        return 1;
     // hand-picked lists: the Llama-3-8B layer bucket, empty tensors, one huge and many tiny
     const int64_t llama[] = {4096, 4096, 1024, 4096, 1024, 4096, 4096, 4096, 14336, 4096,
                              14336, 4096, 4096, 14336, 4096, 1, 4096, 1};
@@ -250,6 +291,16 @@ int main()
         if (check_plan(s, 8, TFTQ_BF16)) return 1;
         plans++;
     }
+    for (int n = 1; n <= 40; n += 13) {  // quantize's second launch alone: nothing but transposed tensors, some empty
+        std::vector<int64_t> s;
+        for (int i = 0; i < n; i++) {
+            s.push_back(i % 5 == 3 ? 0 : 300 + 37 * i);
+            s.push_back(700 + 131 * i);
+        }
+        for (int ws = 1; ws <= 16; ws += 5)
+            if (check_plan(s, ws, n % 3, 1)) return 1;
+        plans++;
+    }
     // random lists on both sides of the inline limit
     for (int it = 0; it < 300; it++) {
         const int n = 1 + (int)(rnd() % (it % 3 == 0 ? 16 : it % 3 == 1 ? 64 : 700));
@@ -265,11 +316,13 @@ int main()
             s.push_back(m);
             s.push_back(c);
         }
-        if (check_plan(s, ws, (int)(rnd() % 3))) {
-            printf("failed at random list %d (n=%d ws=%d)\n", it, n, ws);
-            return 1;
+        for (int by_columns = 0; by_columns < 3; by_columns++) {
+            if (check_plan(s, ws, (int)(rnd() % 3), by_columns)) {
+                printf("failed at random list %d (n=%d ws=%d by columns %d)\n", it, n, ws, by_columns);
+                return 1;
+            }
+            plans++;
         }
-        plans++;
     }
     printf("ok %d plans\n", plans);
     return 0;

@@ -84,7 +84,6 @@ static uint8_t pick_io_kind(const Seg &s, int esz)
         return K_VEC256;  // longer than 32 KB: two passes inside the workgroup
     }
     if (s.n <= 16) return K_GEN1;
-    if (s.row_stride == 1 && s.m >= epv) return K_COLS;
     if (s.n <= 128) return K_GEN8;
     return K_GEN64;
 }
@@ -96,7 +95,6 @@ static uint8_t pick_io_kind(const Seg &s, int esz)
 static uint8_t pick_d_kind(const Seg &s, int esz)
 {
     const uint8_t k = pick_io_kind(s, esz);
-    if (k == K_COLS) return K_TILE;
     const int64_t rowb = (int64_t)s.n * esz;
     if (k != K_VEC8 && k != K_VEC16 && k != K_VEC32 && k != K_VEC64 && k != K_VEC256) return k;
     if (s.row_stride != s.n || (rowb & 63) == 0 || rowb > 16384) {
@@ -155,6 +153,102 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
     if (ndw <= 512) return K_GEN64;
     if (ndw <= 768 && ws <= 64 && many) return K_GEN64;
     return K_GEN256;
+}
+
+// Tensors whose columns are contiguous in memory (transposed matrices).  Their rows have two kernels
+// each way: teams of 8 or 64 lanes with an element per lane and access (K_GEN8 up to 128 columns,
+// K_GEN64), or blocks of 16 (fp32: 8) rows in quantize (K_COLS, a launch of its own) and tiles of 64
+// rows and 256 columns in dequantize (K_TILE).  The blocks and tiles read and write whole pieces of
+// columns, but cost the same however many rows and columns of them the tensor has (a block never
+// crosses a slot), so they lose on narrow tensors and where a slot has few rows of one.
+//
+// What either costs, in us: a kernel takes the longest of its workgroups' latencies, or BASE and the
+// work of all its tensors, whichever is more.  Fitted to kernels back to back in a graph, 2248 lists in
+// quantize and 562 in dequantize: one tensor and lists of up to 10000, 16 to 65536 rows, 17 to 16384
+// columns, 1 to 64 slots, both sizes of element.  On all but a few percent of them the choice takes
+// the faster kernel or one within 5 % or 0.3 us of it.  Teams against blocks in quantize, bf16:
+// [4096, 14336] 267 against 41 us, [256, 8192] 41 against 12.3, [1024, 128] 7.0 against 4.4,
+// [100000, 32] 9.7 against 35, 10000 [32, 32] in 16 slots 26 against 644; teams against tiles in
+// dequantize: [4096, 14336] 290 against 28, [256, 256] 4.0 against 5.8, 10000 [32, 32] 18 against 22.
+struct Cost {
+    double latency, work;
+};
+constexpr double COST_BASE = 3.5;
+constexpr double COST_HIDDEN = 4.2;  // of a latency, beside other tensors in the same launch
+// What a second launch of quantize, behind one for other tensors, saves of its own: [4096, 4096] by
+// rows and one transposed [64, 64], 9.6 us in one launch and 12.6 in two; [1024, 1024], 15.8 and 13.4.
+constexpr double COST_OVERLAP = 0.8;
+
+static Cost cost_of(const Seg &s, uint8_t kind, int st, int esz, int ws)
+{
+    const double m = s.m, n = s.n, padded = (double)s.slice_rows * ws;
+    const bool half = esz == 2;
+    if (kind == K_COLS) {
+        const int rows = tftq_qc_rows(esz);
+        const double block = half ? 4.3e-3 + 3.6e-6 * n : 3.6e-3 + 3.0e-6 * n;
+        return {(half ? 4.1 : 3.8) + 0.0009 * n, (double)ws * ((s.slice_rows + rows - 1) / rows) * (block + 5e-10 * n * n)};
+    }
+    if (kind == K_TILE) {
+        const double tiles = (double)((s.m + TFTQ_TILE_ROWS - 1) / TFTQ_TILE_ROWS) * ((s.n + TFTQ_TILE_COLS - 1) / TFTQ_TILE_COLS);
+        return {4.3 + 0.006 * std::min(n, 256.0), tiles * 1.45e-3 + m * n * esz * 1.35e-7};
+    }
+    if (st == ST_Q)
+        return kind == K_GEN64 ? Cost{3.0 + 0.0045 * n, padded * n * (half ? 4.5e-6 : 6.0e-6)}
+                               : Cost{3.0 + (half ? 0.032 : 0.026) * n, padded * (n * 2.1e-6 + 1.2e-5)};
+    return kind == K_GEN64 ? Cost{2.9 + 0.0044 * n, m * n * 4.0e-6}
+                           : Cost{3.0 + 0.021 * n, m * (n * 1.0e-6 + (half ? 1.4e-5 : 2.0e-5))};
+}
+
+// Chooses for a stage between the teams that the tensors have been given and `blocks` (K_COLS or
+// K_TILE): for none of them, for those that it makes less work, or for all (a few tensors that the
+// machine takes at once, where only the latency counts).
+static void pick_column_kinds(tftq_plan *p, int st, uint8_t blocks)
+{
+    auto stored_by_columns = [&](const Seg &s) {
+        return s.row_stride == 1 && s.m >= 16 / p->esz && s.m < INT32_MAX - 4096 &&  // the blocks round up
+               (s.kind[st] == K_GEN8 || s.kind[st] == K_GEN64);
+    };
+    enum { NONE, LESS_WORK, ALL, N_WAYS };
+    // per way: what is left to the teams, what goes to the blocks
+    Cost teams[N_WAYS] = {}, taken[N_WAYS] = {};
+    bool any[N_WAYS] = {}, others = false;
+    for (const Seg &s : p->segs) {
+        if (!stored_by_columns(s)) {
+            others = others || s.m > 0;
+            continue;
+        }
+        const Cost t = cost_of(s, s.kind[st], st, p->esz, p->ws), b = cost_of(s, blocks, st, p->esz, p->ws);
+        for (int way = NONE; way < N_WAYS; way++) {
+            const bool take = way == ALL || (way == LESS_WORK && b.work < t.work);
+            Cost &sum = take ? taken[way] : teams[way];
+            sum.latency = std::max(sum.latency, take ? b.latency : t.latency);
+            sum.work += take ? b.work : t.work;
+            any[way] = any[way] || take;
+        }
+    }
+    int best = NONE;
+    double least = HUGE_VAL;
+    for (int way = NONE; way < N_WAYS; way++) {
+        auto launch = [&](double latency, double work) {
+            return others ? std::max(latency - COST_HIDDEN, work) : latency > 0.0 ? std::max(latency, COST_BASE + work) : 0.0;
+        };
+        double t;
+        if (st == ST_D) {
+            t = launch(std::max(teams[way].latency, taken[way].latency), teams[way].work + taken[way].work);
+        } else {
+            t = launch(teams[way].latency, teams[way].work);
+            if (any[way]) t += std::max(taken[way].latency, COST_BASE + taken[way].work) - (others ? COST_OVERLAP : 0.0);
+        }
+        if (t < least) {
+            least = t;
+            best = way;
+        }
+    }
+    if (!any[best]) return;
+    for (Seg &s : p->segs)
+        if (stored_by_columns(s) &&
+            (best == ALL || cost_of(s, blocks, st, p->esz, p->ws).work < cost_of(s, s.kind[st], st, p->esz, p->ws).work))
+            s.kind[st] = blocks;
 }
 
 // Bytes one workgroup of segment s moves in reduce.
@@ -376,7 +470,12 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         s.kind[ST_Q] = pick_io_kind(s, p->esz);
         s.kind[ST_D] = pick_d_kind(s, p->esz);
         s.kind[ST_R] = pick_reduce_kind(s, p->ws);
-        const int64_t rows[3] = {m_pad, s.slice_rows, s.m};
+    }
+    pick_column_kinds(p, ST_Q, K_COLS);
+    pick_column_kinds(p, ST_D, K_TILE);
+    for (int i = 0; i < n_tensors; i++) {
+        Seg &s = p->segs[(size_t)i];
+        const int64_t rows[3] = {(int64_t)s.slice_rows * ws, s.slice_rows, s.m};
         for (int st = 0; st < 3; st++) {
             const int64_t n = tftq_wgs_of(s, st, p->esz, ws, rows[st]);
             const int launch = s.kind[st] == K_COLS ? ST_QC : st;
