@@ -248,6 +248,22 @@ static int check_kinds(int count, int64_t m, int64_t n, int dtype, int ws, bool 
 int main()
 {
     int plans = 0;
+    // rows side by side in reduce only where enough workgroups are left
+    const struct { int n, ws; int64_t rows; int at_once; } side[] = {
+        {64, 2, 23000, 1}, {65, 2, 49151, 1}, {65, 2, 49152, 4}, {512, 1, 8191, 1}, {512, 1, 8192, 4}, {512, 2, 4000, 1},
+        {32, 1, 262143, 1}, {32, 1, 262144, 4}, {32, 2, 1 << 22, 1}, {17, 2, 1 << 19, 1}, {17, 2, 1 << 20, 4},
+        {60, 2, 1 << 19, 1}, {60, 2, 1 << 20, 4}, {46, 2, 131071, 1}, {46, 2, 131072, 4}, {65, 3, 1 << 20, 1}, {13, 2, 1 << 22, 1}};
+    for (const auto &c : side) {
+        const int64_t shape[] = {c.rows * c.ws, c.n}, stride[] = {c.n, 1};
+        tftq_plan *p = nullptr;
+        if (tftq_plan_create(TFTQ_BF16, 1, shape, stride, c.ws, &p)) return 1;
+        const int got = p->segs[0].side;
+        tftq_plan_destroy(p);
+        if (got != c.at_once) {
+            printf("%lld rows of %d columns in each of %d slots: %d rows side by side\n", (long long)c.rows, c.n, c.ws, got);
+            return 1;
+        }
+    }
     // which transposed tensors are worth blocks of columns: the faster side of measured pairs
     if (check_kinds(1, 4096, 14336, TFTQ_BF16, 8, false, true, true) || check_kinds(1, 1024, 4096, TFTQ_BF16, 8, false, true, true) ||
         check_kinds(1, 256, 8192, TFTQ_BF16, 16, true, true, true) || check_kinds(1, 4096, 4096, TFTQ_F32, 64, true, true, true) ||

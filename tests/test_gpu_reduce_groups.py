@@ -69,3 +69,24 @@ def test_rows_side_by_side_in_small_groups(q, oracle, ws, op, long_list, plain_d
                 t[len(t) // 2] *= 1e-30
         peers.append([t.to(torch.bfloat16) for t in ts])
     full_check(q, oracle, peers, ws, op, sorted({0, ws - 1}))
+
+
+# (columns, rows per slot from which rows go side by side in groups of 1 and of 2: tftq_reduce_rows_side)
+SIDE = [(17, 262144, 1048576), (32, 262144, None), (46, 131072, 131072), (60, 131072, 1048576), (65, 32768, 49152),
+        (128, 32768, 49152), (130, 16384, 24576), (257, 8192, 12288), (512, 8192, 12288)]
+
+
+@pytest.mark.parametrize("plain_divide", [False, True])
+@pytest.mark.parametrize("ws,op", [(1, ReduceOp.SUM), (2, ReduceOp.AVG)])
+@pytest.mark.parametrize("n,one,two", SIDE)
+def test_rows_side_by_side_where_workgroups_are_left(q, oracle, n, one, two, ws, op, plain_divide):  # noqa: F811
+    least = (one, two)[ws - 1] or 300000
+    g = torch.Generator().manual_seed(n)
+    shapes = [(least * ws, n), ((least - 1) * ws, n), ((least + 3) * ws - ws // 2, n)]
+    for shape in shapes if n < 40 or least < 1 << 20 else shapes[2:]:
+        base = torch.randn(1000, n, generator=g)
+        base[333] = -0.0
+        if plain_divide:
+            base[500] *= 1e-30
+        peers = [[(base * (1 + p)).to(torch.bfloat16).repeat(-(-shape[0] // 1000), 1)[:shape[0]].contiguous()] for p in range(ws)]
+        full_check(q, oracle, peers, ws, op, [ws - 1])

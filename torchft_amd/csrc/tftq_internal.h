@@ -87,17 +87,30 @@ TFTQ_HD static inline int tftq_reduce_rows_at_once(uint8_t kind, int ndw, int ws
 }
 
 // Reduce, teams of 2 to 32 lanes with one vector per lane and peer: in groups of up to 2 peers a team
-// takes 4 rows at once, so that a lane has 8 loads in flight and not 2 (reduce_rows_side).  Only
-// tensors with work for 256 workgroups without that: a smaller one keeps all its teams.  2 peers,
-// [524288, 200] 49.5 -> 36.5 us, [262144, 400] 48.0 -> 33.1, [2097152, 60] 49.6 -> 44.7; not for a lane
-// per row ([4194304, 14] 27.8 -> 30.4) and not two rows for 4 peers ([2097152, 60] 37.2 -> 40.0).
+// takes 4 rows at once, so that a lane has 8 loads in flight and not 2 (reduce_rows_side; Seg::side).
+// That leaves a quarter of the workgroups, so only tensors that keep enough of them.  Packed rows of
+// 65 columns, 1 peer: 2 MB (227 workgroups left) 5.0 -> 4.9 us, 1 MB 4.1 -> 4.7, 4 MB 7.2 -> 5.9; 2 peers:
+// 6 MB (341) 6.5 -> 6.6, 8 MB (455) 7.5 -> 6.8, 48 MB 27.9 -> 21.1; 256 columns, 2 peers: 3 MB 4.3 -> 5.5,
+// 12 MB (378) both 7.1, 200 MB 78 -> 56: from 256 workgroups on, 384 for 2 peers.  Teams of 2 and 4 lanes
+// from 512: 60 columns, 1 peer: 6 MB (384) 6.0 -> 6.3, 8 MB (512) 7.1 -> 6.7.  Rows that fill such a team
+// load well alone: 2 peers, 32 columns: 8 MB 5.2 -> 6.0, 64 MB 21.3 -> 22.7, 200 MB 50.6 -> 54.7: never; 60
+// columns: 48 MB 17.1 -> 18.2, 100 MB 30.4 -> 30.6, 200 MB 55.3 -> 53.5: from 4096; a team of 2 that they
+// don't fill, 24 columns: 24 MB 10.5 -> 11.0, 64 MB 24.4 -> 22.8: from 2048.  Not for a lane per row
+// ([4194304, 14] 27.8 -> 30.4) and not two rows for 4 peers ([2097152, 60] 37.2 -> 40.0).
 constexpr int TFTQ_R_SIDE_ROWS = 4;
-TFTQ_HD static inline int tftq_reduce_rows_side(uint8_t kind, int ndw, int slice_rows, int ws)
+static inline int tftq_reduce_rows_side(uint8_t kind, int ndw, int slice_rows, int ws)
 {
     if (kind != K_GEN32 && kind != K_GEN16 && kind != K_GEN8 && kind != K_GEN4 && kind != K_GEN2) return 1;
     const int team = tftq_team_of(kind);
-    const bool side = ws <= 2 && ndw <= 4 * team && (int64_t)slice_rows * team >= 256 * TFTQ_WG;
-    return side ? TFTQ_R_SIDE_ROWS : 1;
+    if (ws > 2 || ndw > 4 * team) return 1;
+    int least = team <= 4 ? 512 : ws == 1 ? 256 : 384;
+    if (ws == 2 && team == 2) {
+        if (ndw == 8) return 1;
+        least = 2048;
+    } else if (ws == 2 && team == 4 && ndw > 12) {
+        least = 4096;
+    }
+    return (int64_t)slice_rows * team >= (int64_t)least * TFTQ_R_SIDE_ROWS * TFTQ_WG ? TFTQ_R_SIDE_ROWS : 1;
 }
 
 // K_VECS: a row of nvec (1..32) 16-byte vectors is owned by a team of 2^lt lanes (the
@@ -184,7 +197,7 @@ struct Seg {
     int32_t row_bytes;   // 4 + round_up(n, 4)
     int32_t wg_begin[3]; // first workgroup of this segment, per stage
     uint8_t kind[3];     // lane mapping, per stage
-    uint8_t reserved;
+    uint8_t side;        // reduce: rows that a team of 2 to 32 lanes takes at once (tftq_reduce_rows_side)
 };
 static_assert(sizeof(Seg) == 64, "Seg must be 64 bytes");
 
@@ -197,8 +210,7 @@ static inline int tftq_rows_per_wg(const Seg &s, int st, int esz, int ws)
     if (s.kind[st] == K_VECS) return tftq_small_rows_per_wg(tftq_small_nvec(s.n, esz), st);
     const int teams = TFTQ_WG / tftq_team_of(s.kind[st]);
     if (st == ST_R)
-        return teams * tftq_reduce_rows_at_once(s.kind[st], s.row_bytes / 4 - 1, ws) *
-               tftq_reduce_rows_side(s.kind[st], s.row_bytes / 4 - 1, s.slice_rows, ws);
+        return teams * tftq_reduce_rows_at_once(s.kind[st], s.row_bytes / 4 - 1, ws) * s.side;
     return teams;
 }
 

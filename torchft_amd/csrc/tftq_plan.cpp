@@ -470,6 +470,7 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         s.kind[ST_Q] = pick_io_kind(s, p->esz);
         s.kind[ST_D] = pick_d_kind(s, p->esz);
         s.kind[ST_R] = pick_reduce_kind(s, p->ws);
+        s.side = (uint8_t)tftq_reduce_rows_side(s.kind[ST_R], s.row_bytes / 4 - 1, s.slice_rows, p->ws);
     }
     pick_column_kinds(p, ST_Q, K_COLS);
     pick_column_kinds(p, ST_D, K_TILE);

@@ -762,9 +762,8 @@ template <int TEAM, bool GDIV>
 DEV bool reduce_side(const Seg &s, const KParams &p, int blk, int tid, float *lds)
 {
     constexpr int TW = 64 / TEAM;  // teams per wavefront
-    const int rows = tftq_reduce_rows_side(s.kind[ST_R], (s.row_bytes >> 2) - 1, s.slice_rows, p.ws);  // same for all
-    if (rows == 1) return false;
-    const int first = (blk * 4 + __builtin_amdgcn_readfirstlane(tid >> 6)) * TW * rows;
+    if (s.side == 1) return false;  // same for all
+    const int first = (blk * 4 + __builtin_amdgcn_readfirstlane(tid >> 6)) * TW * TFTQ_R_SIDE_ROWS;
     if (first >= s.slice_rows) return true;  // the whole wavefront leaves
     const int j0 = first + (tid & 63) / TEAM;
     reduce_rows_side<TEAM, GDIV>(s, p, j0, TW, tid % TEAM, lds);
