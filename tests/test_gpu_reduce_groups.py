@@ -90,3 +90,11 @@ def test_rows_side_by_side_where_workgroups_are_left(q, oracle, n, one, two, ws,
             base[500] *= 1e-30
         peers = [[(base * (1 + p)).to(torch.bfloat16).repeat(-(-shape[0] // 1000), 1)[:shape[0]].contiguous()] for p in range(ws)]
         full_check(q, oracle, peers, ws, op, [ws - 1])
+
+
+@pytest.mark.parametrize("plain_divide", [False, True])
+@pytest.mark.parametrize("long_list", [False, True])
+@pytest.mark.parametrize("ws,op", [(9, ReduceOp.SUM), (10, ReduceOp.AVG), (11, ReduceOp.SUM), (12, ReduceOp.AVG), (12, ReduceOp.SUM),
+                                   (13, ReduceOp.AVG), (15, ReduceOp.SUM)])
+def test_short_rows_in_groups_of_9_to_15(q, oracle, ws, op, long_list, plain_divide):  # noqa: F811
+    test_short_rows_in_large_groups(q, oracle, ws, op, long_list, plain_divide)

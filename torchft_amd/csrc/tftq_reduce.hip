@@ -626,7 +626,7 @@ DEV void reduce_rows(const Seg &s, const KParams &p, int j, int lane, float *lds
 }
 
 // Rows of up to 16 * TEAM bytes of codes in teams of 1, 2 or 4 lanes: one vector per lane and
-// peer, groups of up to MAXWS (2, 4, 8 or 16) peers, every load of the row in flight at once.  (One
+// peer, groups of up to MAXWS (2, 4, 8, 12 or 16) peers, every load of the row in flight at once.  (One
 // lane per row reads such a row with two or four loads that lie a row apart from its
 // neighbours'; here a load instruction of a wavefront covers 32 or 16 neighbouring rows.)
 // Lane l of a team fetches the scales of peers l, l + TEAM, ...: MAXWS / TEAM of them, ahead
@@ -635,6 +635,7 @@ DEV void reduce_rows(const Seg &s, const KParams &p, int j, int lane, float *lds
 template <int TEAM, int MAXWS, bool GDIV>
 DEV void reduce_rows_narrow(const Seg &s, const KParams &p, int j, int lane, float *lds, bool valid)
 {
+    static_assert(MAXWS <= TEAM || MAXWS % TEAM == 0, "every peer's scale has a lane");
     constexpr int NS = MAXWS > TEAM ? MAXWS / TEAM : 1;  // scales per lane
     const int ndw = (s.row_bytes >> 2) - 1;  // >= 4 here
     const int ws = p.ws;                     // <= MAXWS
@@ -1257,14 +1258,16 @@ DEV void reduce_col1(const Seg &s, const KParams &p, int j0, int tid)
         else reduce_rows<TEAM, UNITS, true, GDIV>(__VA_ARGS__);                                   \
     } while (0)
 
-// reduce_rows_narrow for a team of TEAM lanes, for the smallest of 2, 4, 8 and 16 peers that
-// holds the group (a variant for more peers loads the last peer again in their place);
-// larger groups go through it in chunks
+// reduce_rows_narrow for a team of TEAM lanes, for the smallest of 2, 4, 8, 12 and 16 peers that
+// holds the group (a variant for more peers loads the last peer again in their place: averages over 9
+// and 12 peers, [2097152, 60], with the variant for 16 33.0 and 31.3 us, for 12 29.7 and 28.9);
+// larger groups go through the rows in chunks
 #define TFTQ_REDUCE_NARROW(TEAM, ...)                                             \
     do {                                                                          \
         if (p.ws <= 2) reduce_rows_narrow<TEAM, 2, GDIV>(__VA_ARGS__);            \
         else if (p.ws <= 4) reduce_rows_narrow<TEAM, 4, GDIV>(__VA_ARGS__);       \
         else if (p.ws <= 8) reduce_rows_narrow<TEAM, 8, GDIV>(__VA_ARGS__);       \
+        else if (p.ws <= 12) reduce_rows_narrow<TEAM, 12, GDIV>(__VA_ARGS__);     \
         else if (p.ws <= 16) reduce_rows_narrow<TEAM, 16, GDIV>(__VA_ARGS__);     \
         else reduce_rows_chunks<TEAM, GDIV>(__VA_ARGS__);                         \
     } while (0)
