@@ -16,6 +16,10 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <algorithm>
+#include <utility>
+#include <vector>
+
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/core/Tensor.h>
@@ -147,7 +151,78 @@ PyObject *describe(PyObject *, PyObject *args)
                          static_cast<int>(device), reinterpret_cast<const char *>(pointers), static_cast<Py_ssize_t>(n * 8));
 }
 
+// Tensors that stand for others.
+constexpr c10::DispatchKeySet WRAPPERS({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                        c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::BatchedNestedTensor,
+                                        c10::DispatchKey::Functionalize});
+
+// in_place(owners, pieces, known) -> addresses, or None
+// The owners' addresses as a list of ints, if a kernel may read and write the owners, all at once, as
+// the elements of `pieces` (as many plain contiguous tensors), and `known` itself if they are the
+// addresses that this list holds.  None where only a copy does that: tensors of another type, dtype,
+// device or shape than their piece, that are not contiguous, that autograd or functorch follows, that
+// were made in inference mode, that have their sign in a flag or no memory, and owners that share
+// memory.
+PyObject *in_place(PyObject *, PyObject *args)
+{
+    PyObject *owners = nullptr, *pieces = nullptr, *known = nullptr;
+    if (!PyArg_ParseTuple(args, "O!O!O", &PyList_Type, &owners, &PyList_Type, &pieces, &known)) return nullptr;
+    const Py_ssize_t n = PyList_GET_SIZE(owners);
+    if (PyList_GET_SIZE(pieces) != n) Py_RETURN_NONE;
+    bool same = PyList_CheckExact(known) && PyList_GET_SIZE(known) == n;
+    std::vector<std::pair<uintptr_t, uintptr_t>> spans;
+    PyObject *out = nullptr;
+    try {
+        spans.reserve(static_cast<size_t>(n));
+        for (Py_ssize_t i = 0; i < n; i++) {
+            fetch_ahead(owners, i, n, true);
+            PyObject *o = PyList_GET_ITEM(owners, i), *q = PyList_GET_ITEM(pieces, i);
+            if (!THPVariable_CheckExact(o) || !THPVariable_Check(q)) Py_RETURN_NONE;
+            const at::Tensor &t = THPVariable_Unpack(o), &piece = THPVariable_Unpack(q);
+            if (!t.defined() || t.key_set().has_any(WRAPPERS) || !t.has_storage() || t.layout() != at::kStrided ||
+                t.scalar_type() != piece.scalar_type() || t.device() != piece.device() ||
+                t.sizes() != piece.sizes() || !t.is_contiguous() || t.requires_grad() || t.is_neg() || t.is_inference())
+                Py_RETURN_NONE;
+            const uintptr_t at = reinterpret_cast<uintptr_t>(t.data_ptr());
+            if (at == 0 && t.numel() != 0) Py_RETURN_NONE;
+            spans.emplace_back(at, at + t.nbytes());
+            same = same && PyLong_AsUnsignedLongLong(PyList_GET_ITEM(known, i)) == at;
+        }
+        if (same) {  // looked at when they were written down
+            Py_INCREF(known);
+            return known;
+        }
+        out = PyList_New(n);
+        if (!out) return nullptr;
+        for (Py_ssize_t i = 0; i < n; i++) {
+            PyObject *a = PyLong_FromUnsignedLongLong(spans[static_cast<size_t>(i)].first);
+            if (!a) {
+                Py_DECREF(out);
+                return nullptr;
+            }
+            PyList_SET_ITEM(out, i, a);
+        }
+        std::sort(spans.begin(), spans.end());
+        uintptr_t end = 0;
+        for (const auto &span : spans) {
+            if (span.first == span.second) continue;
+            if (span.first < end) {
+                Py_DECREF(out);
+                Py_RETURN_NONE;
+            }
+            end = span.second;
+        }
+        return out;
+    } catch (...) {  // a tensor that answers none of this
+        Py_XDECREF(out);
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+}
+
 PyMethodDef methods[] = {
+    {"in_place", in_place, METH_VARARGS,
+     "in_place(owners, pieces, known): the owners' addresses if kernels may work on them in place of the pieces, or None"},
     {"describe", describe, METH_VARARGS,
      "describe(tensors, most): (bytes that tell lists apart, device, addresses) of a short list of 2-D tensors, or None"},
     {"scan", scan, METH_VARARGS,
