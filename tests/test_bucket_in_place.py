@@ -90,22 +90,26 @@ def test_host_time_per_tensor():
     assert min(times) < 2000 * 0.15e-6
 
 
-def step(peers, ws, dtype, capacity, op, way, monkeypatch):
-    """Two steps on copies of the peers' tensors; what every rank holds after each"""
+def step(peers, ws, dtype, capacity, op, way, monkeypatch, aliased=False):
+    """Two steps on copies of the peers' tensors; what every rank holds after each, and the buckets.
+    `aliased`: in the first step two tensors of one storage"""
     group, seen = SimGroup(ws), [[] for _ in range(ws)]
     mine = [[t.cuda() for t in tensors] for tensors in peers]
     if way == "copies":
         monkeypatch.setattr(ar.BucketizedAllreduce, "_in_place", lambda self, bucket, whole: None)
-    if way == "aliased":  # two tensors of one storage, on both ways the same
+    if aliased:
         for tensors in mine:
             tensors[2] = tensors[3][:tensors[2].numel()].view_as(tensors[2])
     averaging = [ar.BucketizedAllreduce(tensors, capacity * tensors[0].element_size()) for tensors in mine]
+    for a in averaging:
+        a.made = []  # after each step: the buckets in place that exist
 
     def rank_fn(r):
         for _ in range(2):
             works = averaging[r].allreduce(group.rank(r), ws, reduce_op=op)
             assert all(w.wait() and w.get_future().value() == [] for w in works)
             seen[r].append([t.clone() for t in mine[r]])
+            averaging[r].made.append([len(b["piecewise"]) for b in averaging[r].buckets])
             for t in mine[r]:
                 t.data = t * 0.5  # storage of its own for the second step
 
@@ -142,9 +146,11 @@ def test_in_place_step_has_the_bytes_of_the_copies(monkeypatch, dtype, ws, sizes
 def test_shared_memory_and_storage_that_moves_in_flight(monkeypatch):
     g = torch.Generator().manual_seed(3)
     peers = [[torch.randn(s, generator=g) for s in [(16,), (9, 9), (5, 4), (300,)]] for _ in range(2)]
-    _, averaging = step(peers, 2, torch.float32, 1 << 20, ReduceOp.AVG, "aliased", monkeypatch)
+    got, averaging = step(peers, 2, torch.float32, 1 << 20, ReduceOp.AVG, "in place", monkeypatch, aliased=True)
     # the first step has shared memory and copies; afterwards every tensor has storage of its own
-    assert all(len(a.buckets[0]["piecewise"]) == 1 for a in averaging)
+    assert all(a.made == [[0], [1]] for a in averaging)
+    want, _ = step(peers, 2, torch.float32, 1 << 20, ReduceOp.AVG, "copies", monkeypatch, aliased=True)
+    assert all(torch.equal(a, b) for r in range(2) for k in range(2) for a, b in zip(got[r][k], want[r][k]))
 
     want, _ = step(peers, 2, torch.float32, 1 << 20, ReduceOp.AVG, "copies", monkeypatch)
     group = SimGroup(2)
