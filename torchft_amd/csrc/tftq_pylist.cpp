@@ -28,9 +28,10 @@ namespace {
 
 // A tensor is three objects one behind the other (the Python object, the tensor, its storage), and a
 // walk that asks for each when it needs it waits for memory three times per tensor.  The objects of
-// the tensors ahead are asked for before their turn.
+// the tensors ahead are asked for before their turn.  (Inlined by force: with two callers the compiler
+// makes it a call per tensor, and a pass of three walks over 10 000 tensors took 250 us instead of 230.)
 constexpr Py_ssize_t AHEAD = 8;
-inline void fetch_ahead(PyObject *list, Py_ssize_t i, Py_ssize_t n, bool storages)
+__attribute__((always_inline)) inline void fetch_ahead(PyObject *list, Py_ssize_t i, Py_ssize_t n, bool storages)
 {
     if (i + 3 * AHEAD < n) __builtin_prefetch(PyList_GET_ITEM(list, i + 3 * AHEAD));
     if (i + 2 * AHEAD < n) {
