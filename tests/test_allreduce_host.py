@@ -144,7 +144,7 @@ def test_capture_is_asked_of_the_tensors_device(monkeypatch):
         def __exit__(self, *exc):
             current[0] = self.before
 
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    monkeypatch.setattr(q, "_current_device", lambda: current[0])
     monkeypatch.setattr(torch.cuda, "device", Guard)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: current[0] == 0)
     assert q._capturing(torch.device("cuda", 0)) and not q._capturing(torch.device("cuda", 1))

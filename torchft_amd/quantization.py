@@ -68,9 +68,12 @@ _PLAN_CACHE_SIZE = 4096
 _PLAN_CACHE_TENSORS = 1 << 18
 
 
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)  # 0.1 us instead of 0.4
+
+
 def _capturing(device: torch.device) -> bool:
     """Whether the current stream of `device`, which need not be the current device, is being captured."""
-    if torch.cuda.current_device() == device.index:
+    if _current_device() == device.index:
         return torch.cuda.is_current_stream_capturing()
     with torch.cuda.device(device):
         return torch.cuda.is_current_stream_capturing()
@@ -257,7 +260,7 @@ def _match_short_list(inputs, ws: int):
     """(plan, device, addresses) of a list of up to 16 plain 2-D tensors on a GPU.  None for any
     other list: the caller takes prepare(), which says what is wrong with it, if anything is, and
     turns 1-D tensors into ``[k, 1]`` in the caller's list."""
-    if _pylist is None or len(inputs) > _N_INLINE or type(ws) is not int:
+    if _pylist is None or type(ws) is not int:
         return None
     said = _pylist.describe(inputs, _N_INLINE)
     if said is None or said[1] < 0:
@@ -634,7 +637,7 @@ def fused_quantize_into_fp8(
     Returns:
         the packed uint8 tensor (``numel() % all_reduce_group_size == 0``)
     """
-    hit = _match_short_list(inputs, all_reduce_group_size)
+    hit = _match_short_list(inputs, all_reduce_group_size) if len(inputs) <= _N_INLINE else None
     if hit is not None:
         plan, device, ptrs = hit
         out = torch.empty(plan.output_size, dtype=torch.uint8, device=device)
@@ -672,7 +675,7 @@ def fused_dequantize_from_fp8(
     Python number on the GPU gives.
     """
     table = pointers = lock = None
-    hit = _match_short_list(inputs, all_reduce_group_size)
+    hit = _match_short_list(inputs, all_reduce_group_size) if len(inputs) <= _N_INLINE else None
     if hit is None:
         hit = _match_long_list(inputs, all_reduce_group_size, True)
         if hit is None:
@@ -711,7 +714,7 @@ def fused_reduce_fp8(
     ``inputs`` only supplies the shapes.
     """
     table = None
-    hit = _match_short_list(inputs, all_reduce_group_size)
+    hit = _match_short_list(inputs, all_reduce_group_size) if len(inputs) <= _N_INLINE else None
     if hit is None:
         hit = _match_long_list(inputs, all_reduce_group_size, False)
         if hit is None:
