@@ -2,10 +2,11 @@
 // (tftq_quantize.hip, tftq_reduce.hip, tftq_dequantize.hip): HIP kernels for
 // gfx950 (MI355X) and the compute entry points of the C ABI.
 //
-// Three kernels, one launch per stage:
-//   k_quantize<T>    fused_quantize_into_fp8   (torchft/quantization.py:53-162)
-//   k_reduce         fused_reduce_fp8          (:261-428)
-//   k_dequantize<T>  fused_dequantize_from_fp8 (:165-258)
+// Three stages, one launch each, and a second one in quantize for a list's matrices that are stored
+// column by column and large enough:
+//   k_quantize<T>, k_quantize_cols<T>  fused_quantize_into_fp8   (torchft/quantization.py:53-162)
+//   k_reduce                           fused_reduce_fp8          (:261-428)
+//   k_dequantize<T>                    fused_dequantize_from_fp8 (:165-258)
 //
 // Design (none of it follows the reference's launch shape):
 //   * a row is owned by a "team" of 1 to 256 lanes chosen from the row length
@@ -14,8 +15,8 @@
 //     registers, reduces |x| with DPP inside the wavefront (LDS across the four
 //     wavefronts of a 256-lane team) and converts from registers with the
 //     packed fp8 converts of gfx950.  Every stage reads HBM once.
-//   * all tensors of a call are covered by one launch: a workgroup finds its
-//     tensor in a table of 64-byte descriptors (in the kernel arguments for
+//   * a launch covers all the tensors of a call (k_quantize and k_quantize_cols
+//     share them between them): a workgroup finds its tensor in a table of 64-byte descriptors (in the kernel arguments for
 //     short lists) and branches on the team size stored there.
 //   * workgroup ids are remapped so that each of the 8 XCDs works on
 //     contiguous pieces of every tensor (neighbouring packed rows share cache

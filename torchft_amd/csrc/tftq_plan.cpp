@@ -130,8 +130,12 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
     // and the next 8).  218 M bf16 elements, 8 peers, a lane per row against the team: 24 columns
     // 81.1 -> 66.7 us, 28: 89.2 -> 64.4, 32: 65.0 -> 64.4, 44: 92.1 -> 68.7, 60: 95.6 -> 64.7, 64:
     // 70.6 -> 65.0.  45 to 48 columns are three whole vectors, of which a lane alone wastes none:
-    // [2097152, 48], 2, 4, 8 and 16 peers: 41.1 -> 38.6 us, 33.1 -> 31.2, 29.6 -> 28.2, 27.7 -> 30; in a
-    // tensor of a few rows the lane alone waits 33 us for its 16 peers, the team 7 us.
+    // [2097152, 48] on rotating buffers, 4, 8, 15, 16 and 24 peers: 36.5 -> 35.2 us, 32.8 -> 31.2, 38.3 ->
+    // 33.6, 31.7 -> 32.7 and 39.1 -> 33.1; in a tensor of a few rows the lane alone waits 33 us for its
+    // 16 peers, the team 7 us.  (In groups of 17 to 24 peers the lane alone is up to 12 % faster on
+    // millions of full rows, [4194304, 32] 17 peers 40.5 against 45.1 us, [2097152, 64] 37.0 against 42.0, and
+    // up to 3 times slower on all others: [2097152, 32] 24 peers 29.2 against 24.5, 3 MB of 60 columns 17
+    // peers 21.8 against 7.0.)
     if (ndw > 8 && ndw <= 16) return K_GEN4;
     if (ndw > 4 && ndw <= 8) return K_GEN2;
     if (ndw <= 16) return K_GEN1;
@@ -165,8 +169,8 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
 // What either costs, in us: a kernel takes the longest of its workgroups' latencies, or BASE and the
 // work of all its tensors, whichever is more.  Fitted to kernels back to back in a graph, 2248 lists in
 // quantize and 562 in dequantize: one tensor and lists of up to 10000, 16 to 65536 rows, 17 to 16384
-// columns, 1 to 64 slots, both sizes of element.  On all but a few percent of them the choice takes
-// the faster kernel or one within 5 % or 0.3 us of it.  Teams against blocks in quantize, bf16:
+// columns, 1 to 64 slots, both sizes of element.  On all but 33 of them the choice takes the faster
+// kernel or one within 5 % or 0.3 us of it.  Teams against blocks in quantize, bf16:
 // [4096, 14336] 267 against 41 us, [256, 8192] 41 against 12.3, [1024, 128] 7.0 against 4.4,
 // [100000, 32] 9.7 against 35, 10000 [32, 32] in 16 slots 26 against 644; teams against tiles in
 // dequantize: [4096, 14336] 290 against 28, [256, 256] 4.0 against 5.8, 10000 [32, 32] 18 against 22.

@@ -618,12 +618,13 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize(const KParam
 // neighbouring bytes of a packed row with one store, with no exchange between lanes.  Only the row
 // maxima go through LDS.  A block of 16 (fp32: 8) rows stays in the registers of a workgroup of 512
 // lanes, up to NS steps of 1024 columns, so that the tensor is read once; what a row has beyond
-// that is read twice.  Bound by the L1's requests in flight, which are 32 bytes each here (HBM
-// traffic is the algorithmic 1.0 times): transposed [4096, 14336] and [4096, 4096] bf16, 227 MB,
-// one element per lane and access and two passes 486 us, this kernel 79 us.  Alone, [4096, 14336]
-// 65.7 us: with blocks of 32 rows 101 (half the compute units idle), workgroups of 256 lanes 89
+// that is read twice.  Bound by the L1's requests in flight, of which a block uses 29 bytes each
+// (5.2 million for 151 MB; HBM traffic is the algorithmic 1.08 times): transposed [4096, 14336] and
+// [4096, 4096] bf16, 227 MB, one element per lane and access and two passes 486 us, this kernel 79 us.
+// Alone, [4096, 14336] 66 to 69 us: with blocks of 32 rows 101 (half the compute units idle), workgroups of 256 lanes 89
 // (half of the row read twice), of 1024 lanes 72, streaming loads 77 (neighbouring blocks share
-// lines); a launch for the maxima and one for tiles of 64 rows 82 us.
+// lines); a launch for the maxima and one for tiles of 64 rows 82 us.  Where the blocks lose against
+// teams of lanes (few columns, few rows per slot) the planner leaves them out: pick_column_kinds.
 template <typename T, int NS>
 DEV void quantize_cols(const Seg &s, const KParams &p, int blk, int tid, float *part, float *scale)
 {
