@@ -12,7 +12,8 @@ from concurrent.futures import ThreadPoolExecutor
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(_HERE, "libtftq.so")
-SOURCES = ["tftq_quantize.hip", "tftq_reduce.hip", "tftq_dequantize.hip", "tftq_runtime.hip", "tftq_plan.cpp"]
+SOURCES = ["tftq_quantize.hip", "tftq_dequantize.hip", "tftq_reduce.hip", "tftq_reduce_all.hip", "tftq_reduce_wide.hip",
+           "tftq_reduce_long.hip", "tftq_reduce_one.hip", "tftq_runtime.hip", "tftq_plan.cpp"]
 # Streaming kernels without arithmetic that bench.py times beside the product kernels
 # (benchmark infrastructure; torchft_amd never loads this library).
 CEILING_LIB_PATH = os.path.join(_HERE, "libtftq_ceiling.so")
@@ -24,10 +25,13 @@ PYLIST_SOURCE = "tftq_pylist.cpp"
 # -ffp-contract=off: the arithmetic contract is separate IEEE multiply, divide
 # and add; fused multiply-adds are written out where they are wanted.
 # packed-fp32-ops off: no v_pk_*_f32 instructions are generated.
+# amdgpu-kernarg-preload-count: the first single values among a kernel's arguments are in scalar
+# registers when a wavefront starts (the kernels for one tensor, KOne in tftq_internal.h).
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-ffp-contract=off", "-fno-fast-math",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wall", "-Wno-unused-command-line-argument",
 ]
 

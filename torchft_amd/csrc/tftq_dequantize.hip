@@ -35,7 +35,7 @@ DEV void stage_elem(LDS_AS uint8_t *srow, int col, float v)
 // caller's `tensor /= num_participants` (manager.py:450-452) without a second
 // pass over the tensor.
 template <typename T, bool POST>
-DEV float fin(float v, const KParams &p)
+DEV float fin(float v, const KCall &p)
 {
 
     return POST ? Elem<T>::rounded(v) * p.post_scale : v;
@@ -44,7 +44,7 @@ DEV float fin(float v, const KParams &p)
 // Any strides; also the path of rows whose scale is outside the range of the
 // fast exact division (plain IEEE divide, one element per lane and step).
 template <typename T, int TEAM, bool POST>
-DEV void dequantize_gen(const Seg &s, const KParams &p, int row, int lane)
+DEV void dequantize_gen(const Seg &s, const KCall &p, int row, int lane)
 {
     if (row >= s.m) return;
     GLOBAL const uint8_t *in = as_global<const uint8_t>(p.packed + row_addr(s, p.slot_size, row));
@@ -73,7 +73,7 @@ DEV void dequantize_gen(const Seg &s, const KParams &p, int row, int lane)
 // v0, v1: the row's vectors v0 ... v1 - 1 only (a row dealt to several workgroups,
 // tftq_d_row_parts); `last`: with the columns behind the last whole vector.
 template <typename T, int TEAM, bool STAGED, int DV, bool POST>
-DEV void dequantize_vec_k(const Seg &s, const KParams &p, int row, int lane, LDS_AS uint8_t *srow, int v0 = 0,
+DEV void dequantize_vec_k(const Seg &s, const KCall &p, int row, int lane, LDS_AS uint8_t *srow, int v0 = 0,
                           int v1 = -1, bool last = true)
 {
     if (row >= s.m) return;
@@ -152,7 +152,7 @@ DEV void dequantize_vec_k(const Seg &s, const KParams &p, int row, int lane, LDS
 // through the LDS stage in pieces of 1024 vectors (16 KB), each written as whole lines; the
 // columns behind the last whole vector travel with the last piece.
 template <typename T, bool POST>
-DEV void dequantize_vec_pieces(const Seg &s, const KParams &p, int row, int tid, uint8_t *stage, int v0, int v1, bool last)
+DEV void dequantize_vec_pieces(const Seg &s, const KCall &p, int row, int tid, uint8_t *stage, int v0, int v1, bool last)
 {
     constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, DV = 4, STEP = DV * TFTQ_WG;
     if (row >= s.m) return;  // the whole workgroup
@@ -222,7 +222,7 @@ DEV void dequantize_vec_pieces(const Seg &s, const KParams &p, int row, int tid,
 // Longer rows go through the stage a piece at a time (dequantize_vec_pieces).  What is left
 // (strided rows of up to 16 KB) is written from the registers, partial blocks included.
 template <typename T, int TEAM, bool POST>
-DEV void dequantize_vec_rows(const Seg &s, const KParams &p, int blk, int tid, uint8_t *stage)
+DEV void dequantize_vec_rows(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage)
 {
     constexpr int R = TFTQ_WG / TEAM;
     const int r0 = blk * R;
@@ -273,7 +273,7 @@ DEV void dequantize_vec_rows(const Seg &s, const KParams &p, int blk, int tid, u
 // Rows of one column: one plain divide per row.  Any element stride: four rows
 // per lane, interleaved.
 template <typename T, bool POST>
-DEV void dequantize_col1_strided(const Seg &s, const KParams &p, int row0, int tid)
+DEV void dequantize_col1_strided(const Seg &s, const KCall &p, int row0, int tid)
 {
     const float inv = 1.0f / (float)s.slice_rows;
     u32x2 w[4];
@@ -294,7 +294,7 @@ DEV void dequantize_col1_strided(const Seg &s, const KParams &p, int row0, int t
 // two packed rows of a pair with one 16-byte load and writes the two elements
 // with one store (the mapping of quantize_col1).
 template <typename T, bool POST>
-DEV void dequantize_col1(const Seg &s, const KParams &p, int row0, int tid)
+DEV void dequantize_col1(const Seg &s, const KCall &p, int row0, int tid)
 {
     if (s.row_stride != 1) {  // same for the whole workgroup
 #pragma nounroll
@@ -367,7 +367,7 @@ DEV u32x2 load_small_codes(GLOBAL const u32 *in, int col)
 // Rows RBEG * teams .. REND * teams - 1 of the workgroup's rows.  STAGED: they are
 // neighbours in memory (row stride = row length) and go through the LDS stage as one span.
 template <typename T, int C, bool STAGED, bool POST, int RBEG, int REND>
-DEV void dequantize_small_rows(const Seg &s, const KParams &p, const SmallShape &h, const u32x2 (&w)[8 / C][C],
+DEV void dequantize_small_rows(const Seg &s, const KCall &p, const SmallShape &h, const u32x2 (&w)[8 / C][C],
                                const float (&sc)[8 / C], bool fast, int row0, uint8_t *stage, int tid)
 {
     constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ;
@@ -423,7 +423,7 @@ DEV void dequantize_small_rows(const Seg &s, const KParams &p, const SmallShape 
 }
 
 template <typename T, int C, bool STAGED, bool TAIL, bool POST>
-DEV void dequantize_small_c(const Seg &s, const KParams &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
+DEV void dequantize_small_c(const Seg &s, const KCall &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
 {
     constexpr int ROWS = 8 / C;  // 8 or 4
     const int nvec = tftq_small_nvec(s.n, Elem<T>::ESZ);
@@ -452,7 +452,7 @@ DEV void dequantize_small_c(const Seg &s, const KParams &p, int blk, int tid, co
 }
 
 template <typename T, bool STAGED, bool TAIL, bool POST>
-DEV void dequantize_small_s(const Seg &s, const KParams &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
+DEV void dequantize_small_s(const Seg &s, const KCall &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
 {
     // one or two vectors per lane (tftq_small_shape)
     if (h.c == 1) dequantize_small_c<T, 1, STAGED, TAIL, POST>(s, p, blk, tid, h, stage);
@@ -460,7 +460,7 @@ DEV void dequantize_small_s(const Seg &s, const KParams &p, int blk, int tid, co
 }
 
 template <typename T, bool POST>
-DEV void dequantize_small(const Seg &s, const KParams &p, int blk, int tid, uint8_t *stage)
+DEV void dequantize_small(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage)
 {
     const SmallShape h = small_shape(tftq_small_nvec(s.n, Elem<T>::ESZ), tid, ST_D);
     const int rowb = s.n * Elem<T>::ESZ;
@@ -483,7 +483,7 @@ DEV void dequantize_small(const Seg &s, const KParams &p, int blk, int tid, uint
 // Bound by memory: transposed [4096, 14336] and [4096, 4096] bf16, 227 MB, one element per lane and
 // access 443 us, this kernel 43.9 us (5.2 TB/s).  Where it is taken: pick_column_kinds.
 template <typename T, bool POST>
-DEV void dequantize_tile(const Seg &s, const KParams &p, int blk, int tid, uint8_t *stage, float (*coef)[3])
+DEV void dequantize_tile(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage, float (*coef)[3])
 {
     constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, RS = TFTQ_TILE_COLS / 4 + 1, G = TFTQ_TILE_ROWS / EPV;
     static_assert(TFTQ_TILE_ROWS * RS * 4 <= TFTQ_D_STAGE, "a tile fits the stage");
@@ -563,15 +563,15 @@ DEV void dequantize_tile(const Seg &s, const KParams &p, int blk, int tid, uint8
     }
 }
 
-template <typename T, bool INLINE, bool POST>
-__global__ __launch_bounds__(TFTQ_WG) void k_dequantize(const KParams p, const InlineTable inl)
+template <typename T, bool POST, typename A>
+DEV void dequantize_workgroup(const A &args)
 {
     __shared__ __align__(16) uint8_t stage[TFTQ_D_STAGE];  // see copy_out_span
     __shared__ float coef[TFTQ_TILE_ROWS][3];
     Seg s;
-    int vb;
-    if (!locate<INLINE, ST_D>(p, inl, s, vb)) return;
-    const int blk = vb - s.wg_begin[ST_D];
+    KCall p;
+    int blk;
+    if (!locate<ST_D>(args, p, s, blk)) return;
     const int tid = threadIdx.x;
     switch (s.kind[ST_D]) {
     case K_VEC256: dequantize_vec_rows<T, 256, POST>(s, p, blk, tid, stage); break;
@@ -594,32 +594,46 @@ __global__ __launch_bounds__(TFTQ_WG) void k_dequantize(const KParams p, const I
     }
 }
 
-template <typename T, bool POST>
-static int launch_d(const KParams &kp, const InlineTable &inl, bool use_inline, hipStream_t st)
+template <typename T, typename A, bool POST>
+__global__ __launch_bounds__(TFTQ_WG) void k_dequantize(const A args)
 {
-    if (use_inline) return launch_kernel(k_dequantize<T, true, POST>, grid_of(kp), 0, st, kp, inl);
-    return launch_kernel(k_dequantize<T, false, POST>, grid_of(kp), 0, st, kp, inl);
+    dequantize_workgroup<T, POST>(args);
+}
+template <typename T, bool POST>
+__global__ __launch_bounds__(TFTQ_WG) void k_dequantize_one(TFTQ_ONE_PARAMS)
+{
+    dequantize_workgroup<T, POST>(one_of(TFTQ_ONE));
+}
+
+template <typename T, bool POST>
+static int launch_d(const KArgs &ka, hipStream_t st)
+{
+    return with_args(ka, [&](const auto &args) {
+        typedef typename std::decay<decltype(args)>::type A;
+        if constexpr (std::is_same<A, KOne>::value) return launch_kernel(k_dequantize_one<T, POST>, ka, args, 0, st);
+        else return launch_kernel(k_dequantize<T, A, POST>, ka, args, 0, st);
+    });
 }
 
 template <bool POST>
 static int dequantize(const tftq_plan *plan, void *const *tensors, const void *table, void *pointers,
                       const void *packed, int64_t packed_bytes, float post_scale, int device, void *stream)
 {
-    KParams kp;
-    InlineTable inl = {};
-    bool use_inline;
     hipStream_t st = (hipStream_t)stream;
     DeviceScope scope(device);
     if (scope.err != hipSuccess) return (int)scope.err;
-    int rc = fill_params(plan, ST_D, (const void *const *)tensors, table, pointers, (void *)packed, packed_bytes, st,
-                         &kp, &inl, &use_inline);
+    int rc = check_call(plan, ST_D, (const void *const *)tensors, table, pointers, packed, packed_bytes);
+    if (rc || plan->nwg[ST_D] == 0) return rc;
+    rc = put_addresses(plan, (const void *const *)tensors, pointers, st);
     if (rc) return rc;
-    kp.post_scale = post_scale;
-    if (kp.nwg == 0) return 0;
+    KCall what = PLAIN_CALL;
+    what.post_scale = post_scale;
+    KArgs ka;
+    fill_args(plan, ST_D, (const void *const *)tensors, table, pointers, (void *)packed, what, &ka);
     switch (plan->dtype) {
-    case TFTQ_F32: return launch_d<float, POST>(kp, inl, use_inline, st);
-    case TFTQ_F16: return launch_d<f16_tag, POST>(kp, inl, use_inline, st);
-    case TFTQ_BF16: return launch_d<bf16_tag, POST>(kp, inl, use_inline, st);
+    case TFTQ_F32: return launch_d<float, POST>(ka, st);
+    case TFTQ_F16: return launch_d<f16_tag, POST>(ka, st);
+    case TFTQ_BF16: return launch_d<bf16_tag, POST>(ka, st);
     default: return TFTQ_E_DTYPE;
     }
 }

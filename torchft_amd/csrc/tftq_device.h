@@ -1,5 +1,5 @@
 // Device helpers and launch plumbing shared by the three kernel files
-// (tftq_quantize.hip, tftq_reduce.hip, tftq_dequantize.hip): HIP kernels for
+// (tftq_quantize.hip, tftq_reduce_kernels.h, tftq_dequantize.hip): HIP kernels for
 // gfx950 (MI355X) and the compute entry points of the C ABI.
 //
 // Three stages, one launch each, and a second one in quantize for a list's matrices that are stored
@@ -355,84 +355,131 @@ DEV void unpack_dword(u32 w, float (&f)[4 / Elem<T>::ESZ])
 // a bucket map plus a short binary search lead from the number to the segment.
 // Ids past the end of their XCD's work return false.
 //
-// The kernel arguments are (KParams, InlineTable).  Indexing those by-value
-// structs with a run-time index would make the compiler copy them to private
-// memory; reading the kernel-argument segment through a constant-address-space
-// pointer keeps the accesses scalar loads.
+// A list of one tensor needs no round of scalar loads (KOne: its arguments are in registers when the
+// wavefront starts), a longer one two or three.  A kernel that is one round of workgroups is that much
+// shorter: with the tables of a longer list, with KOne loaded as a structure and with KOne in registers,
+// quantize, reduce and dequantize of a bf16 [4096, 4096] for 8 peers 11.5, 6.4, 12.6 / 10.8, 6.0, 11.7 /
+// 10.8, 5.9, 11.4 us, of 315 fp32 elements 2.1, 3.2, 2.1 / 1.7, 2.9, 1.6 / 1.4, 2.5, 1.4 us.  (The
+// descriptors of up to four tensors loaded in one round and selected in registers gain nothing: 64
+// scalar registers and their selection cost what the second round does.)
+//
+// Indexing by-value kernel arguments with a run-time index would make the compiler copy them to
+// private memory; reading the kernel-argument segment through a constant-address-space pointer keeps
+// the accesses scalar loads.
 #define CONSTANT __attribute__((address_space(4)))
-constexpr size_t KARG_TABLE_OFF = (sizeof(KParams) + alignof(InlineTable) - 1) / alignof(InlineTable) * alignof(InlineTable);
 
-DEV const CONSTANT Seg *karg_table()
+// locate<STAGE>(kernel arguments, call, segment, workgroup of the segment); false: nothing to do.
+// KOne as kernel parameters, of which -amdgpu-kernarg-preload-count puts the first 56 bytes into
+// scalar registers, and back.
+#define TFTQ_ONE_PARAMS                                                                                            \
+    const uint64_t w0, const uint64_t w1, const uint64_t w2, const uint64_t w3, const uint64_t w4, const uint64_t w5, \
+        const uint64_t w6, const uint64_t w7
+#define TFTQ_ONE w0, w1, w2, w3, w4, w5, w6, w7
+DEV KOne one_of(TFTQ_ONE_PARAMS)
 {
-    return (const CONSTANT Seg *)((const CONSTANT char *)__builtin_amdgcn_kernarg_segment_ptr() + KARG_TABLE_OFF);
+    const uint64_t w[8] = {TFTQ_ONE};
+    return __builtin_bit_cast(KOne, w);
 }
 
-template <bool INLINE, int STAGE>
-DEV bool locate(const KParams &p, const InlineTable &inl, Seg &s, int &vb)
+template <int STAGE>
+DEV bool locate(const KOne &a, KCall &p, Seg &s, int &blk)
+{
+    constexpr bool R = STAGE == ST_R;
+    blk = tftq_one_piece(a.nwg, a.natural, blockIdx.x);
+    s.ptr = R ? 0 : a.ptr;
+    s.slot_off = 0;
+    s.row_stride = R ? 0 : a.row_stride;
+    s.col_stride = R ? 0 : a.col_stride;
+    s.m = a.m;
+    s.n = a.n;
+    s.slice_rows = a.slice_rows;
+    s.row_bytes = ((a.n + 3) & ~3) + 4;
+    s.kind[STAGE] = a.kind;
+    s.side = a.side;
+    p.packed = a.packed;
+    p.slot_size = (int64_t)a.slice_rows * s.row_bytes;
+    p.ws = a.ws;
+    p.rank = R ? a.rank : 0;
+    p.div_mode = a.div_mode;
+    p.div = R ? a.div : 1.0f;
+    p.inv_div = R ? a.inv_div : 1.0f;
+    p.post_scale = a.post_scale;
+    return blk >= 0;
+}
+
+template <int STAGE>
+DEV bool locate(const KInline &a, KCall &p, Seg &s, int &blk)
 {
     const int x = (int)(blockIdx.x & 7);
     int i = (int)(blockIdx.x >> 3);
-    if (INLINE) {
-        // One round of scalar loads fetches this XCD's three table rows; the position
-        // is then found in registers, and only the segment descriptor needs a second round.
-        const CONSTANT char *karg = (const CONSTANT char *)__builtin_amdgcn_kernarg_segment_ptr();
-        const CONSTANT int32_t *d = (const CONSTANT int32_t *)(karg + offsetof(KParams, dealt)) + x * TFTQ_N_INLINE;
-        typedef int32_t Row __attribute__((ext_vector_type(TFTQ_N_INLINE)));  // one 64-byte scalar load
-        const Row cum_end = *(const CONSTANT Row *)(d + offsetof(Dealt, cum_end) / 4);
-        const Row base = *(const CONSTANT Row *)(d + offsetof(Dealt, base) / 4);
-        const Row seg = *(const CONSTANT Row *)(d + offsetof(Dealt, seg) / 4);
-        Row cum_end_ = cum_end, base_ = base, seg_ = seg;
-        // all scalar loads of this round, and the common parameters, are issued before the first wait
-        int natural = p.natural;
-        asm volatile("" : "+s"(cum_end_), "+s"(base_), "+s"(seg_), "+s"(natural) : "s"(p.packed), "s"(p.slot_size), "s"(p.ws), "s"(p.rank));
-        if (natural) i = (int)blockIdx.x;  // all eight rows of the table describe the whole work
-        int b = base_[0], sg = seg_[0];
+    // One round of scalar loads fetches this XCD's three table rows; the position
+    // is then found in registers, and only the segment descriptor needs a second round.
+    const CONSTANT char *karg = (const CONSTANT char *)__builtin_amdgcn_kernarg_segment_ptr();
+    const CONSTANT int32_t *d = (const CONSTANT int32_t *)(karg + offsetof(KInline, dealt)) + x * TFTQ_N_INLINE;
+    typedef int32_t Row __attribute__((ext_vector_type(TFTQ_N_INLINE)));  // one 64-byte scalar load
+    const Row cum_end = *(const CONSTANT Row *)(d + offsetof(Dealt, cum_end) / 4);
+    const Row base = *(const CONSTANT Row *)(d + offsetof(Dealt, base) / 4);
+    const Row seg = *(const CONSTANT Row *)(d + offsetof(Dealt, seg) / 4);
+    Row cum_end_ = cum_end, base_ = base, seg_ = seg;
+    // all scalar loads of this round, and the common parameters, are issued before the first wait
+    int natural = a.natural;
+    asm volatile("" : "+s"(cum_end_), "+s"(base_), "+s"(seg_), "+s"(natural)
+                 : "s"(a.call.packed), "s"(a.call.slot_size), "s"(a.call.ws), "s"(a.call.rank));
+    p = a.call;
+    if (natural) i = (int)blockIdx.x;  // all eight rows of the table describe the whole work
+    int b = base_[0], sg = seg_[0];
 #pragma unroll
-        for (int j = 1; j < TFTQ_N_INLINE; j++) {
-            const bool past = i >= cum_end_[j - 1];  // cum_end is non-decreasing: the last hit wins
-            b = past ? base_[j] : b;
-            sg = past ? seg_[j] : sg;
-        }
-        if (sg < 0 || i >= cum_end_[TFTQ_N_INLINE - 1]) return false;
-        vb = b + i;
-        const CONSTANT u32x4 *src = (const CONSTANT u32x4 *)(karg_table() + sg);
-        const u32x4 v[4] = {src[0], src[1], src[2], src[3]};
-        __builtin_memcpy(&s, v, sizeof(Seg));
-        return true;
-    } else {
-        // everything the first steps need from the kernel arguments in one round of scalar loads
-        asm volatile("" ::"s"(p.table), "s"(p.ptrs), "s"(p.map_off), "s"(p.sorted_off), "s"(p.map_shift), "s"(p.chunk_shift),
-                     "s"(p.nwg), "s"(p.pieces), "s"(p.packed), "s"(p.slot_size), "s"(p.ws), "s"(p.rank));
-        // chunks of 2^chunk_shift consecutive workgroups go to the XCDs in turn
-        const int cs = p.chunk_shift;
-        vb = ((((i >> cs) << 3) + x) << cs) + (i & ((1 << cs) - 1));
-        if (vb >= p.nwg) return false;
-        if (STAGE == ST_R && p.pieces) {  // this wavefront's quarter of the workgroup (tftq_reduce_pieces)
-            vb = 4 * vb + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-            if (vb >= p.pieces) return false;
-        }
-        const uint64_t tab = (uint64_t)p.table;
-        typedef int32_t MapPair __attribute__((ext_vector_type(4), aligned(8)));
-        const MapPair m = *(const CONSTANT MapPair *)(tab + (uint64_t)p.map_off +
-                                                      (uint64_t)(vb >> p.map_shift) * sizeof(MapEnt));
-        int lo = m.x, sg = m.y, hi = m.z;
-        if (lo != hi) {  // last position whose first workgroup is <= vb
-            const CONSTANT SortEnt *sorted = (const CONSTANT SortEnt *)(tab + (uint64_t)p.sorted_off);
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (sorted[mid].begin <= vb) lo = mid; else hi = mid - 1;
-            }
-            sg = sorted[lo].seg;
-        }
-        const CONSTANT u32x4 *src = (const CONSTANT u32x4 *)(tab + (uint64_t)sg * sizeof(Seg));
-        const u32x4 v[4] = {src[0], src[1], src[2], src[3]};
-        // the table holds no addresses: the tensor's comes from the call's pointer array
-        uint64_t tptr = 0;
-        if (STAGE != ST_R) tptr = *(const CONSTANT uint64_t *)((uint64_t)p.ptrs + (uint64_t)sg * 8u);
-        __builtin_memcpy(&s, v, sizeof(Seg));
-        s.ptr = tptr;
-        return true;
+    for (int j = 1; j < TFTQ_N_INLINE; j++) {
+        const bool past = i >= cum_end_[j - 1];  // cum_end is non-decreasing: the last hit wins
+        b = past ? base_[j] : b;
+        sg = past ? seg_[j] : sg;
     }
+    if (sg < 0 || i >= cum_end_[TFTQ_N_INLINE - 1]) return false;
+    const CONSTANT u32x4 *src = (const CONSTANT u32x4 *)(karg + offsetof(KInline, s) + (uint64_t)(u32)sg * sizeof(Seg));
+    const u32x4 v[4] = {src[0], src[1], src[2], src[3]};
+    __builtin_memcpy(&s, v, sizeof(Seg));
+    blk = b + i - s.wg_begin[STAGE];
+    return true;
+}
+
+template <int STAGE>
+DEV bool locate(const KTable &a, KCall &p, Seg &s, int &blk)
+{
+    const int x = (int)(blockIdx.x & 7), i = (int)(blockIdx.x >> 3);
+    // everything the first steps need from the kernel arguments in one round of scalar loads
+    asm volatile("" ::"s"(a.table), "s"(a.ptrs), "s"(a.map_off), "s"(a.sorted_off), "s"(a.map_shift), "s"(a.chunk_shift),
+                 "s"(a.nwg), "s"(a.pieces), "s"(a.call.packed), "s"(a.call.slot_size), "s"(a.call.ws), "s"(a.call.rank));
+    p = a.call;
+    // chunks of 2^chunk_shift consecutive workgroups go to the XCDs in turn
+    const int cs = a.chunk_shift;
+    int vb = ((((i >> cs) << 3) + x) << cs) + (i & ((1 << cs) - 1));
+    if (vb >= a.nwg) return false;
+    if (STAGE == ST_R && a.pieces) {  // this wavefront's quarter of the workgroup (tftq_reduce_pieces)
+        vb = 4 * vb + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        if (vb >= a.pieces) return false;
+    }
+    const uint64_t tab = (uint64_t)a.table;
+    typedef int32_t MapPair __attribute__((ext_vector_type(4), aligned(8)));
+    const MapPair m = *(const CONSTANT MapPair *)(tab + (uint64_t)a.map_off +
+                                                  (uint64_t)(vb >> a.map_shift) * sizeof(MapEnt));
+    int lo = m.x, sg = m.y, hi = m.z;
+    if (lo != hi) {  // last position whose first workgroup is <= vb
+        const CONSTANT SortEnt *sorted = (const CONSTANT SortEnt *)(tab + (uint64_t)a.sorted_off);
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (sorted[mid].begin <= vb) lo = mid; else hi = mid - 1;
+        }
+        sg = sorted[lo].seg;
+    }
+    const CONSTANT u32x4 *src = (const CONSTANT u32x4 *)(tab + (uint64_t)sg * sizeof(Seg));
+    const u32x4 v[4] = {src[0], src[1], src[2], src[3]};
+    // the table holds no addresses: the tensor's comes from the call's pointer array
+    uint64_t tptr = 0;
+    if (STAGE != ST_R) tptr = *(const CONSTANT uint64_t *)((uint64_t)a.ptrs + (uint64_t)sg * 8u);
+    __builtin_memcpy(&s, v, sizeof(Seg));
+    s.ptr = tptr;
+    blk = vb - s.wg_begin[STAGE];
+    return true;
 }
 
 DEV int64_t row_addr(const Seg &s, int64_t slot_size, int row)
@@ -507,27 +554,18 @@ DEV void copy_out_span(const uint8_t *stage, uint8_t *g0, int len, int tid)
 }
 
 // ---------------------------------------------------------------------------
-// host side: kernel parameters of a launch
+// host side: kernel arguments of a launch
 // ---------------------------------------------------------------------------
-static inline void work_mapping(const tftq_plan *plan, int stage, KParams *kp)
-{
-    if (plan->nseg <= TFTQ_N_INLINE) {
-        kp->dealt = plan->dealt[stage];
-        kp->per_xcd = plan->dealt_per_xcd[stage];
-        kp->natural = plan->natural[stage] ? 1 : 0;
-        kp->pieces = 0;
-        kp->map_shift = kp->chunk_shift = 0;
-        kp->sorted_off = kp->map_off = 0;
-    } else {
-        kp->per_xcd = plan->index[stage].per_xcd;
-        kp->natural = 0;
-        kp->pieces = plan->index[stage].pieces;
-        kp->map_shift = plan->index[stage].shift;
-        kp->chunk_shift = plan->index[stage].chunk_shift;
-        kp->sorted_off = plan->index[stage].sorted_off;
-        kp->map_off = plan->index[stage].map_off;
-    }
-}
+struct KArgs {
+    enum { ONE, INLINE, TABLE } where;
+    unsigned grid;
+    union {
+        KOne one;
+        KInline inl;
+        KTable table;
+    };
+    KArgs() {}
+};
 
 // Makes `device` current for the lifetime of the object and restores the caller's device
 // afterwards; device < 0 leaves the current device alone.
@@ -564,66 +602,121 @@ __attribute__((visibility("hidden"))) int tftq_put_bytes(void *dst_device, const
 __attribute__((visibility("hidden"))) int tftq_static_table_setup(void);
 
 // One kernel launch with the launch's own error (not whatever an earlier call left behind).
-template <typename K>
-static inline int launch_kernel(K kernel, unsigned grid, unsigned lds_bytes, hipStream_t st, const KParams &kp,
-                                const InlineTable &inl, int threads = TFTQ_WG)
+template <typename K, typename A>
+static inline int launch_kernel(K kernel, const KArgs &ka, const A &arg, unsigned lds_bytes, hipStream_t st, int threads = TFTQ_WG)
 {
-    void *args[2] = {(void *)&kp, (void *)&inl};
-    return (int)hipLaunchKernel((const void *)kernel, dim3(grid), dim3(threads), args, lds_bytes, st);
+    void *args[8];
+    const bool one = std::is_same<A, KOne>::value;  // eight words
+    for (int i = 0; i < (one ? 8 : 1); i++) args[i] = (char *)&arg + 8 * i;
+    return (int)hipLaunchKernel((const void *)kernel, dim3(ka.grid), dim3(threads), args, lds_bytes, st);
 }
 
-// Kernel parameters of one call.  tensors: host array of the tensors' device addresses (null
-// in reduce); table / pointers: the caller's device buffers of a long list.  For a long list
-// with `tensors` the addresses are written to `pointers` on `st` first.
-static inline int fill_params(const tftq_plan *plan, int stage, const void *const *tensors, const void *table,
-                              void *pointers, void *packed, int64_t packed_bytes, hipStream_t st, KParams *kp,
-                              InlineTable *inl, bool *use_inline)
+// f(the arguments) with the type of the list's length.
+template <typename F>
+static inline int with_args(const KArgs &ka, F f)
+{
+    switch (ka.where) {
+    case KArgs::ONE: return f(ka.one);
+    case KArgs::INLINE: return f(ka.inl);
+    default: return f(ka.table);
+    }
+}
+
+// What a call of a stage must bring along: tensors, a host array of the tensors' device addresses
+// (null in reduce); table and pointers, the caller's device buffers of a long list.
+static inline int check_call(const tftq_plan *plan, int stage, const void *const *tensors, const void *table,
+                             const void *pointers, const void *packed, int64_t packed_bytes)
 {
     if (!plan) return TFTQ_E_ARG;
     if (packed_bytes != plan->output_size) return TFTQ_E_SIZE;
     // a list of empty tensors has an empty packed buffer, whose address may be null
     if (!packed && plan->output_size != 0) return TFTQ_E_ARG;
     if (((uintptr_t)packed & 3) != 0) return TFTQ_E_ARG;
-    *use_inline = plan->nseg <= TFTQ_N_INLINE;
     const bool needs_tensors = stage != ST_R && plan->nwg[stage] > 0;
-    if (*use_inline) {
+    auto missing = [&](int i) { return !tensors[i] && plan->segs[(size_t)i].m > 0 && plan->segs[(size_t)i].n > 0; };
+    if (plan->nseg <= TFTQ_N_INLINE) {
         if (needs_tensors && !tensors) return TFTQ_E_ARG;
-        for (int i = 0; i < plan->nseg; i++) {
-            inl->s[i] = plan->segs[(size_t)i];
-            if (stage != ST_R) {
-                inl->s[i].ptr = (uint64_t)(uintptr_t)(tensors ? tensors[i] : nullptr);
-                if (inl->s[i].ptr == 0 && inl->s[i].m > 0 && inl->s[i].n > 0) return TFTQ_E_ARG;
-            }
-        }
-    } else if (plan->nwg[stage] > 0) {
+        if (stage == ST_R) return 0;
+    } else {
+        if (plan->nwg[stage] == 0) return 0;
         if (!table || ((uintptr_t)table & 255) != 0) return TFTQ_E_NOTABLE;
-        if (needs_tensors) {
-            if (!pointers || ((uintptr_t)pointers & 7) != 0) return TFTQ_E_NOTABLE;
-            if (tensors) {
-                for (int i = 0; i < plan->nseg; i++)
-                    if (!tensors[i] && plan->segs[(size_t)i].m > 0 && plan->segs[(size_t)i].n > 0) return TFTQ_E_ARG;
-                const int rc = tftq_put_bytes(pointers, tensors, (size_t)plan->nseg * 8, st);
-                if (rc) return rc;
-            }
-        }
+        if (!needs_tensors) return 0;
+        if (!pointers || ((uintptr_t)pointers & 7) != 0) return TFTQ_E_NOTABLE;
+        if (!tensors) return 0;
     }
-    kp->table = *use_inline ? nullptr : (const Seg *)table;
-    kp->ptrs = (*use_inline || stage == ST_R) ? nullptr : (const uint64_t *)pointers;
-    kp->packed = (uint8_t *)packed;
-    kp->slot_size = plan->slot_size;
-    kp->nseg = plan->nseg;
-    kp->nwg = plan->nwg[stage];
-    kp->ws = plan->ws;
-    work_mapping(plan, stage, kp);
-    kp->rank = 0;
-    kp->div_mode = 0;
-    kp->div = 1.0f;
-    kp->inv_div = 1.0f;
-    kp->post_scale = 1.0f;
+    for (int i = 0; i < plan->nseg; i++)
+        if (tensors ? missing(i) : plan->segs[(size_t)i].m > 0 && plan->segs[(size_t)i].n > 0) return TFTQ_E_ARG;
     return 0;
 }
 
-static inline unsigned grid_of(const KParams &kp)
+// Writes the addresses of a long list's tensors, where the call has them, to `pointers` on `st`.
+static inline int put_addresses(const tftq_plan *plan, const void *const *tensors, void *pointers, hipStream_t st)
 {
-    return (unsigned)(8 * kp.per_xcd);
+    return tensors && plan->nseg > TFTQ_N_INLINE ? tftq_put_bytes(pointers, tensors, (size_t)plan->nseg * 8, st) : 0;
+}
+
+constexpr KCall PLAIN_CALL = {nullptr, 0, 0, 0, 0, 1.0f, 1.0f, 1.0f};
+
+// The kernel arguments of a launch.  what: all but packed, slot_size and ws, which the plan knows.
+static inline void fill_args(const tftq_plan *plan, int stage, const void *const *tensors, const void *table,
+                             const void *pointers, void *packed, const KCall &what, KArgs *ka)
+{
+    const int field = stage == ST_QC ? (int)ST_Q : stage;
+    const bool natural = plan->nseg <= TFTQ_N_INLINE && plan->natural[stage];
+    auto address = [&](int i) { return stage == ST_R || !tensors ? (uint64_t)0 : (uint64_t)(uintptr_t)tensors[i]; };
+    ka->grid = 8u * (unsigned)(plan->nseg <= TFTQ_N_INLINE ? plan->dealt_per_xcd[stage] : plan->index[stage].per_xcd);
+    if (plan->nseg == 1) {
+        const Seg &s = plan->segs[0];
+        KOne &a = ka->one;
+        ka->where = KArgs::ONE;
+        a.packed = (uint8_t *)packed;
+        if (stage == ST_R) {
+            a.rank = what.rank;
+            a.div = what.div;
+            a.inv_div = what.inv_div;
+        } else {
+            a.ptr = address(0);
+            a.row_stride = s.row_stride;
+            a.col_stride = s.col_stride;
+        }
+        a.m = s.m;
+        a.n = s.n;
+        a.slice_rows = s.slice_rows;
+        a.ws = plan->ws;
+        a.nwg = plan->nwg[stage];
+        a.kind = s.kind[field];
+        a.side = s.side;
+        a.natural = natural;
+        a.div_mode = (uint8_t)what.div_mode;
+        a.post_scale = what.post_scale;
+        return;
+    }
+    KCall call = what;
+    call.packed = (uint8_t *)packed;
+    call.slot_size = plan->slot_size;
+    call.ws = plan->ws;
+    if (plan->nseg <= TFTQ_N_INLINE) {
+        KInline &a = ka->inl;
+        ka->where = KArgs::INLINE;
+        a.call = call;
+        a.natural = natural;
+        a.dealt = plan->dealt[stage];
+        for (int i = 0; i < plan->nseg; i++) {
+            a.s[i] = plan->segs[(size_t)i];
+            a.s[i].ptr = address(i);
+        }
+    } else {
+        const TableIndex &index = plan->index[stage];
+        KTable &a = ka->table;
+        ka->where = KArgs::TABLE;
+        a.call = call;
+        a.table = (const Seg *)table;
+        a.ptrs = stage == ST_R ? nullptr : (const uint64_t *)pointers;
+        a.nwg = plan->nwg[stage];
+        a.pieces = index.pieces;
+        a.map_shift = index.shift;
+        a.chunk_shift = index.chunk_shift;
+        a.sorted_off = index.sorted_off;
+        a.map_off = index.map_off;
+    }
 }

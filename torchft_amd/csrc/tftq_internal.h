@@ -259,10 +259,6 @@ static inline int64_t tftq_reduce_pieces(const Seg &s, int esz, int ws, int64_t 
 }
 
 
-struct InlineTable {
-    Seg s[TFTQ_N_INLINE];
-};
-
 // Inline tables (at most TFTQ_N_INLINE segments): XCD x works through the
 // segments in the stage's work order (reduce: heaviest workgroups first;
 // quantize and dequantize: list order) and takes a contiguous eighth of each.
@@ -320,26 +316,77 @@ struct tftq_plan {
     size_t static_bytes;        // what tftq_reduce_static writes of it: all but the index of quantize's second launch
 };
 
-// Kernel parameters common to the three stages.
-struct KParams {
-    const Seg *table;   // device table, or nullptr when the inline table is used
-    const uint64_t *ptrs;  // device table only: the tensors' addresses, in list order (null in reduce)
+// ---------------------------------------------------------------------------
+// kernel arguments
+// ---------------------------------------------------------------------------
+// What a call is about, whatever its list looks like.
+struct KCall {
     uint8_t *packed;
     int64_t slot_size;
-    int32_t nseg;
-    int32_t nwg;
     int32_t ws;
     int32_t rank;
-    int32_t per_xcd;    // workgroup ids per XCD in the grid
-    int32_t natural;    // inline table only: workgroup id b is piece b of the work, not piece b / 8 of XCD b % 8
-    int32_t pieces;     // device table, reduce: number of quarter-workgroup pieces (0: whole workgroups)
-    int32_t map_shift;  // device table only, as are the next three
-    int32_t chunk_shift;
-    int64_t sorted_off;
-    int64_t map_off;
-    Dealt dealt;        // inline table only
     int32_t div_mode;   // reduce: 0 = SUM, 1 = AVG with power-of-two ws, 2 = AVG, other ws < 1024, 3 = AVG, larger ws
     float div;          // reduce: 1.0 or float(ws)
     float inv_div;      // reduce: RN(1 / div); exact when div_mode == 1
     float post_scale;   // dequantize: factor applied to the rounded result (scaled variant only)
 };
+
+// A list of one tensor: 64 bytes.  The first 56 travel as single values, which the hardware puts into
+// registers before a wavefront starts; what a kernel needs beside them it computes.
+struct KOne {
+    union {
+        uint64_t ptr;        // device address of element (0,0)
+        int32_t rank;        // reduce: as in KCall, as are div and inv_div
+    };
+    uint8_t *packed;
+    union {
+        int64_t row_stride;  // elements, as is col_stride
+        float div;
+    };
+    union {
+        int64_t col_stride;
+        float inv_div;
+    };
+    int32_t m, n, slice_rows, ws;
+    int32_t nwg;         // workgroups
+    uint8_t kind, side;  // of the stage
+    uint8_t natural;     // see natural_order
+    uint8_t div_mode;    // as in KCall
+    float post_scale;    // dequantize: as in KCall
+    int32_t pad_;
+};
+static_assert(sizeof(KOne) == 64, "KOne must be 64 bytes");
+
+// Lists of up to TFTQ_N_INLINE tensors.
+struct KInline {
+    KCall call;
+    int32_t natural;    // workgroup id b is piece b of the work, not piece b / 8 of XCD b % 8
+    int32_t pad_[5];
+    Dealt dealt;        // 64-byte rows, each fetched with one load
+    Seg s[TFTQ_N_INLINE];
+};
+static_assert(sizeof(KInline) <= 4096, "kernel arguments");
+
+// Longer lists.
+struct KTable {
+    KCall call;
+    const Seg *table;
+    const uint64_t *ptrs;  // the tensors' addresses, in list order (null in reduce)
+    int32_t nwg;
+    int32_t pieces;     // reduce: number of quarter-workgroup pieces (0: whole workgroups)
+    int32_t map_shift;
+    int32_t chunk_shift;
+    int64_t sorted_off;
+    int64_t map_off;
+};
+
+// The workgroup of a list's only tensor that workgroup id b of the launch is, or -1: the mapping of
+// deal_to_xcds.
+TFTQ_HD static inline int32_t tftq_one_piece(int32_t nwg, bool natural, uint32_t b)
+{
+    if (natural) return b < (uint32_t)nwg ? (int32_t)b : -1;
+    const int32_t x = (int32_t)(b & 7), i = (int32_t)(b >> 3);
+    const int32_t whole = nwg >> 3, rest = nwg & 7;
+    const int32_t lo = whole * x + ((rest * x) >> 3), hi = whole * (x + 1) + ((rest * (x + 1)) >> 3);
+    return i < hi - lo ? lo + i : -1;
+}

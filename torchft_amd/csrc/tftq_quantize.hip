@@ -67,7 +67,7 @@ constexpr int Q_STAGE_BYTES_WIDE = 32912;
 // the maximum) and simply do not store.
 // STAGED: the row is a real one and its packed image goes to LDS at srow (see copy_out_span).
 template <typename T, int TEAM, int KMAX, bool STAGED = false>
-DEV void quantize_vec_k(const Seg &s, const KParams &p, int row, int lane, float *lds, LDS_AS u32 *srow = nullptr)
+DEV void quantize_vec_k(const Seg &s, const KCall &p, int row, int lane, float *lds, LDS_AS u32 *srow = nullptr)
 {
     GLOBAL u32 *out = nullptr;
     if (!STAGED) {
@@ -141,7 +141,7 @@ DEV void quantize_vec_k(const Seg &s, const KParams &p, int row, int lane, float
 // current one is parked.  What a longer row has beyond 7936 vectors is read
 // twice, once for the maximum and once to be quantized.
 template <typename T>
-DEV void quantize_vec_lds(const Seg &s, const KParams &p, int row, int tid, float *lds, u32x4 *park)
+DEV void quantize_vec_lds(const Seg &s, const KCall &p, int row, int tid, float *lds, u32x4 *park)
 {
     constexpr int KR = 2 * QV, G = TFTQ_Q_PARK_GROUP, NG = TFTQ_Q_PARKED / G;
     static_assert(NG * G == TFTQ_Q_PARKED, "groups of five");
@@ -227,7 +227,7 @@ DEV void quantize_vec_lds(const Seg &s, const KParams &p, int row, int tid, floa
 }
 
 template <typename T, int TEAM, bool WIDE>
-DEV void quantize_vec(const Seg &s, const KParams &p, int row, int lane, float *lds, u32x4 *park)
+DEV void quantize_vec(const Seg &s, const KCall &p, int row, int lane, float *lds, u32x4 *park)
 {
     // same branch for the whole workgroup
     const int nvec = s.n / Elem<T>::EPV;
@@ -242,7 +242,7 @@ DEV void quantize_vec(const Seg &s, const KParams &p, int row, int lane, float *
 // but the workgroups at the end of a slot or of the tensor) and fit the staging buffer,
 // their packed rows are assembled in LDS and written as one span; otherwise row by row.
 template <typename T, int TEAM, bool WIDE>
-DEV void quantize_vec_rows(const Seg &s, const KParams &p, int blk, int tid, float *lds, u32x4 *park, uint8_t *stage)
+DEV void quantize_vec_rows(const Seg &s, const KCall &p, int blk, int tid, float *lds, u32x4 *park, uint8_t *stage)
 {
     constexpr int R = TFTQ_WG / TEAM;
     const int r0 = blk * R;
@@ -276,7 +276,7 @@ DEV void quantize_vec_rows(const Seg &s, const KParams &p, int blk, int tid, flo
 // Any strides, any alignment, any n: element loads, two passes over the row
 // (the second one is served by the caches).
 template <typename T, int TEAM>
-DEV void quantize_gen(const Seg &s, const KParams &p, int row, int lane)
+DEV void quantize_gen(const Seg &s, const KCall &p, int row, int lane)
 {
     const bool active = row < s.slice_rows * p.ws;
     if (!active) return;
@@ -325,7 +325,7 @@ DEV u32x2 quantize_one(float x)
 // Any element stride: four rows per lane, interleaved so that every 8-byte
 // [scale, code] store of a wavefront is contiguous.
 template <typename T>
-DEV void quantize_col1_strided(const Seg &s, const KParams &p, int row0, int tid)
+DEV void quantize_col1_strided(const Seg &s, const KCall &p, int row0, int tid)
 {
     const int m_pad = s.slice_rows * p.ws;
     const float inv = 1.0f / (float)s.slice_rows;
@@ -352,7 +352,7 @@ DEV void quantize_col1_strided(const Seg &s, const KParams &p, int row0, int tid
 // with one 16-byte streaming store (a wavefront writes 1 KB of whole lines).
 // A pair that straddles the end of a slot or of the tensor is stored row by row.
 template <typename T>
-DEV void quantize_col1(const Seg &s, const KParams &p, int row0, int tid)
+DEV void quantize_col1(const Seg &s, const KCall &p, int row0, int tid)
 {
     if (s.row_stride != 1) {  // same for the whole workgroup
 #pragma nounroll
@@ -494,7 +494,7 @@ DEV void quantize_small_span(const Seg &s, const SmallShape &h, const u32x4 (&v)
 // one span of bytes, which goes through LDS (copy_out_span) in two halves (rows of 8 to 64
 // 16-bit columns make up to 24 KB per workgroup, more than the stage holds).
 template <typename T, int C, bool TAIL>
-DEV void quantize_small_c(const Seg &s, const KParams &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
+DEV void quantize_small_c(const Seg &s, const KCall &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
 {
     constexpr int ROWS = 8 / C;  // C vectors per lane and row, ROWS rows per lane: 8 or 4
     const int nvec = tftq_small_nvec(s.n, Elem<T>::ESZ);
@@ -563,7 +563,7 @@ DEV void quantize_small_c(const Seg &s, const KParams &p, int blk, int tid, cons
 }
 
 template <typename T>
-DEV void quantize_small(const Seg &s, const KParams &p, int blk, int tid, uint8_t *stage)
+DEV void quantize_small(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage)
 {
     const SmallShape h = small_shape(tftq_small_nvec(s.n, Elem<T>::ESZ), tid, ST_Q);
     // one or two vectors per lane (tftq_small_shape); same branch for the whole workgroup
@@ -574,11 +574,8 @@ DEV void quantize_small(const Seg &s, const KParams &p, int blk, int tid, uint8_
     else quantize_small_c<T, 2, false>(s, p, blk, tid, h, stage);
 }
 
-template <typename T, bool INLINE, bool WIDE>
-// The wide variant is held to 128 registers (four waves per SIMD instead of three at the 153 to
-// 166 it would take): lists that mix rows of more than 32 KB with shorter ones run whole in
-// it, and the shorter rows gain 10 % (a Llama-3-70B layer bucket: 464 -> 420 us).
-__global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize(const KParams p, const InlineTable inl)
+template <typename T, bool WIDE, typename A>
+DEV void quantize_workgroup(const A &args)
 {
     __shared__ float lds[4];
     __shared__ __align__(16) uint8_t stage_regular[WIDE ? 16 : Q_STAGE_BYTES];  // see copy_out_span
@@ -588,9 +585,9 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize(const KParam
     extern __shared__ u32x4 park[];
     uint8_t *stage = WIDE ? (uint8_t *)park : stage_regular;
     Seg s;
-    int vb;
-    if (!locate<INLINE, ST_Q>(p, inl, s, vb)) return;
-    const int blk = vb - s.wg_begin[ST_Q];
+    KCall p;
+    int blk;
+    if (!locate<ST_Q>(args, p, s, blk)) return;
     const int tid = threadIdx.x;
     switch (s.kind[ST_Q]) {
     case K_VEC256: quantize_vec_rows<T, 256, WIDE>(s, p, blk, tid, lds, park, stage); break;
@@ -607,6 +604,20 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize(const KParam
     case K_VECS: quantize_small<T>(s, p, blk, tid, stage); break;
     default: break;
     }
+}
+
+// The wide variant is held to 128 registers (four waves per SIMD instead of three at the 153 to
+// 166 it would take): lists that mix rows of more than 32 KB with shorter ones run whole in
+// it, and the shorter rows gain 10 % (a Llama-3-70B layer bucket: 464 -> 420 us).
+template <typename T, typename A, bool WIDE>
+__global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize(const A args)
+{
+    quantize_workgroup<T, WIDE>(args);
+}
+template <typename T, bool WIDE>
+__global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize_one(TFTQ_ONE_PARAMS)
+{
+    quantize_workgroup<T, WIDE>(one_of(TFTQ_ONE));
 }
 
 // ---------------------------------------------------------------------------
@@ -626,7 +637,7 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize(const KParam
 // lines); a launch for the maxima and one for tiles of 64 rows 82 us.  Where the blocks lose against
 // teams of lanes (few columns, few rows per slot) the planner leaves them out: pick_column_kinds.
 template <typename T, int NS>
-DEV void quantize_cols(const Seg &s, const KParams &p, int blk, int tid, float *part, float *scale)
+DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, float *part, float *scale)
 {
     constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, G = TFTQ_QC_GROUPS, K = 64 / G, RB = G * EPV;
     constexpr int WAVES = TFTQ_QC_WG / 64, STEP = 4 * K * WAVES;  // columns per step
@@ -742,15 +753,15 @@ DEV void quantize_cols(const Seg &s, const KParams &p, int blk, int tid, float *
 // wavefronts per SIMD; 14 spill), else 4 (114 registers, four).
 constexpr int QC_MOST = 12;
 constexpr int QC_STEP = 4 * (64 / TFTQ_QC_GROUPS) * (TFTQ_QC_WG / 64);
-template <typename T, bool INLINE, int NSMAX>
-__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols(const KParams p, const InlineTable inl)
+template <typename T, int NSMAX, typename A>
+DEV void quantize_cols_workgroup(const A &args)
 {
     __shared__ float part[4 * TFTQ_QC_WG / 64 * TFTQ_QC_GROUPS * Elem<T>::EPV];
     __shared__ float scale[TFTQ_QC_GROUPS * Elem<T>::EPV];
     Seg s;
-    int vb;
-    if (!locate<INLINE, ST_Q>(p, inl, s, vb)) return;
-    const int blk = vb - s.wg_begin[ST_Q];
+    KCall p;
+    int blk;
+    if (!locate<ST_Q>(args, p, s, blk)) return;
     const int tid = threadIdx.x;
     const int steps = (s.n + QC_STEP - 1) / QC_STEP;  // same for the whole workgroup
     if (steps <= 1) quantize_cols<T, 1>(s, p, blk, tid, part, scale);
@@ -759,64 +770,74 @@ __global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols
     else if (steps <= 8) quantize_cols<T, NSMAX == 4 ? 4 : 8>(s, p, blk, tid, part, scale);
     else quantize_cols<T, NSMAX>(s, p, blk, tid, part, scale);
 }
-
-template <typename T>
-static int launch_qc(const KParams &kp, const InlineTable &inl, bool use_inline, int most, hipStream_t st)
+template <typename T, typename A, int NSMAX>
+__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols(const A args)
 {
-    const unsigned grid = grid_of(kp);
-    if (most > 4 * QC_STEP) {
-        if (use_inline) return launch_kernel(k_quantize_cols<T, true, QC_MOST>, grid, 0, st, kp, inl, TFTQ_QC_WG);
-        return launch_kernel(k_quantize_cols<T, false, QC_MOST>, grid, 0, st, kp, inl, TFTQ_QC_WG);
-    }
-    if (use_inline) return launch_kernel(k_quantize_cols<T, true, 4>, grid, 0, st, kp, inl, TFTQ_QC_WG);
-    return launch_kernel(k_quantize_cols<T, false, 4>, grid, 0, st, kp, inl, TFTQ_QC_WG);
+    quantize_cols_workgroup<T, NSMAX>(args);
+}
+template <typename T, int NSMAX>
+__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols_one(TFTQ_ONE_PARAMS)
+{
+    quantize_cols_workgroup<T, NSMAX>(one_of(TFTQ_ONE));
 }
 
 template <typename T>
-static int launch_q(const KParams &kp, const InlineTable &inl, bool use_inline, bool wide, int parked,
-                    hipStream_t st)
+static int launch_qc(const tftq_plan *plan, const KArgs &ka, hipStream_t st)
 {
-    const unsigned grid = grid_of(kp);
-    if (wide) {
-        // the parking area also serves as the stage
-        const unsigned lds = std::max((unsigned)parked * TFTQ_Q_PARK_GROUP * TFTQ_WG * 16u, (unsigned)Q_STAGE_BYTES_WIDE);
-        if (use_inline) return launch_kernel(k_quantize<T, true, true>, grid, lds, st, kp, inl);
-        return launch_kernel(k_quantize<T, false, true>, grid, lds, st, kp, inl);
-    }
-    if (use_inline) return launch_kernel(k_quantize<T, true, false>, grid, 0, st, kp, inl);
-    return launch_kernel(k_quantize<T, false, false>, grid, 0, st, kp, inl);
+    return with_args(ka, [&](const auto &args) {
+        typedef typename std::decay<decltype(args)>::type A;
+        const bool most = plan->cols_most > 4 * QC_STEP;
+        if constexpr (std::is_same<A, KOne>::value)
+            return launch_kernel(most ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
+        else
+            return launch_kernel(most ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
+    });
+}
+
+template <typename T>
+static int launch_q(const tftq_plan *plan, const KArgs &ka, hipStream_t st)
+{
+    // the parking area also serves as the stage
+    const bool wide = plan->wide[ST_Q];
+    const unsigned lds = !wide ? 0 : std::max((unsigned)plan->parked * TFTQ_Q_PARK_GROUP * TFTQ_WG * 16u, (unsigned)Q_STAGE_BYTES_WIDE);
+    return with_args(ka, [&](const auto &args) {
+        typedef typename std::decay<decltype(args)>::type A;
+        if constexpr (std::is_same<A, KOne>::value)
+            return launch_kernel(wide ? k_quantize_one<T, true> : k_quantize_one<T, false>, ka, args, lds, st);
+        else
+            return launch_kernel(wide ? k_quantize<T, A, true> : k_quantize<T, A, false>, ka, args, lds, st);
+    });
 }
 
 extern "C" int tftq_quantize(const tftq_plan *plan, const void *const *tensors, const void *table,
                              void *pointers, void *packed, int64_t packed_bytes, int device, void *stream)
 {
-    KParams kp;
-    InlineTable inl = {};
-    bool use_inline;
     hipStream_t st = (hipStream_t)stream;
     DeviceScope scope(device);
     if (scope.err != hipSuccess) return (int)scope.err;
     if (!plan) return TFTQ_E_ARG;
-    const bool only_cols = plan->nwg[ST_Q] == 0 && plan->nwg[ST_QC] != 0;
-    int rc = fill_params(plan, only_cols ? ST_QC : ST_Q, tensors, table, pointers, packed, packed_bytes, st, &kp, &inl,
-                         &use_inline);
+    const bool rows = plan->nwg[ST_Q] != 0, cols = plan->nwg[ST_QC] != 0;
+    int rc = check_call(plan, cols && !rows ? ST_QC : ST_Q, tensors, table, pointers, packed, packed_bytes);
+    if (rc || (!rows && !cols)) return rc;
+    rc = put_addresses(plan, tensors, pointers, st);
     if (rc) return rc;
-    if (kp.nwg != 0 && !only_cols) {
+    KArgs ka;
+    if (rows) {
+        fill_args(plan, ST_Q, tensors, table, pointers, packed, PLAIN_CALL, &ka);
         switch (plan->dtype) {
-        case TFTQ_F32: rc = launch_q<float>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st); break;
-        case TFTQ_F16: rc = launch_q<f16_tag>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st); break;
-        case TFTQ_BF16: rc = launch_q<bf16_tag>(kp, inl, use_inline, plan->wide[ST_Q], plan->parked, st); break;
+        case TFTQ_F32: rc = launch_q<float>(plan, ka, st); break;
+        case TFTQ_F16: rc = launch_q<f16_tag>(plan, ka, st); break;
+        case TFTQ_BF16: rc = launch_q<bf16_tag>(plan, ka, st); break;
         default: return TFTQ_E_DTYPE;
         }
         if (rc) return rc;
     }
-    if (plan->nwg[ST_QC] == 0) return 0;
-    kp.nwg = plan->nwg[ST_QC];
-    work_mapping(plan, ST_QC, &kp);
+    if (!cols) return 0;
+    fill_args(plan, ST_QC, tensors, table, pointers, packed, PLAIN_CALL, &ka);
     switch (plan->dtype) {
-    case TFTQ_F32: return launch_qc<float>(kp, inl, use_inline, plan->cols_most, st);
-    case TFTQ_F16: return launch_qc<f16_tag>(kp, inl, use_inline, plan->cols_most, st);
-    case TFTQ_BF16: return launch_qc<bf16_tag>(kp, inl, use_inline, plan->cols_most, st);
+    case TFTQ_F32: return launch_qc<float>(plan, ka, st);
+    case TFTQ_F16: return launch_qc<f16_tag>(plan, ka, st);
+    case TFTQ_BF16: return launch_qc<bf16_tag>(plan, ka, st);
     default: return TFTQ_E_DTYPE;
     }
 }
