@@ -366,14 +366,14 @@ DEV u32x2 load_small_codes(GLOBAL const u32 *in, int col)
 
 // Rows RBEG * teams .. REND * teams - 1 of the workgroup's rows.  STAGED: they are
 // neighbours in memory (row stride = row length) and go through the LDS stage as one span.
-template <typename T, int C, bool STAGED, bool POST, int RBEG, int REND>
-DEV void dequantize_small_rows(const Seg &s, const KCall &p, const SmallShape &h, const u32x2 (&w)[8 / C][C],
-                               const float (&sc)[8 / C], bool fast, int row0, uint8_t *stage, int tid)
+template <typename T, int C, bool STAGED, bool POST, int ROWS, int RBEG, int REND>
+DEV void dequantize_small_rows(const Seg &s, const KCall &p, const SmallShape &h, const u32x2 (&w)[ROWS][C],
+                               const float (&sc)[ROWS], bool fast, int row0, uint8_t *stage, int tid)
 {
     constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ;
     const int nvec = tftq_small_nvec(s.n, ESZ);
     const int rowb = s.n * ESZ;
-    const int last = min(row0 + h.teams * (8 / C), s.m) - 1;
+    const int last = min(row0 + h.teams * ROWS, s.m) - 1;
     const int first = row0 + RBEG * h.teams;
     if (first > last) return;  // same for the whole workgroup
     uint8_t *gp = (uint8_t *)s.ptr + (int64_t)first * rowb;  // used when STAGED
@@ -422,10 +422,11 @@ DEV void dequantize_small_rows(const Seg &s, const KCall &p, const SmallShape &h
     }
 }
 
-template <typename T, int C, bool STAGED, bool TAIL, bool POST>
+// VECS: vectors per lane, 8 (K_VECS) or 2 (K_VECS_FEW).
+template <typename T, int C, bool STAGED, bool TAIL, bool POST, int VECS>
 DEV void dequantize_small_c(const Seg &s, const KCall &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
 {
-    constexpr int ROWS = 8 / C;  // 8 or 4
+    constexpr int ROWS = VECS / C;
     const int nvec = tftq_small_nvec(s.n, Elem<T>::ESZ);
     const int row0 = blk * (h.teams * ROWS);
     const float inv = 1.0f / (float)s.slice_rows;
@@ -445,21 +446,25 @@ DEV void dequantize_small_c(const Seg &s, const KCall &p, int blk, int tid, cons
 #pragma unroll
     for (int r = 0; r < ROWS; r++) all_fast = all_fast && scale_is_fast(sc[r]);
     const bool fast = __builtin_amdgcn_ballot_w64(!all_fast) == 0;  // one code path per wavefront
-    // a workgroup writes up to 32 KB: two halves through the stage
-    dequantize_small_rows<T, C, STAGED, POST, 0, ROWS / 2>(s, p, h, w, sc, fast, row0, stage, tid);
-    if constexpr (STAGED) __syncthreads();  // the first half has been copied out of the stage
-    dequantize_small_rows<T, C, STAGED, POST, ROWS / 2, ROWS>(s, p, h, w, sc, fast, row0, stage, tid);
+    if constexpr (VECS == TFTQ_SMALL_VECS) {
+        // a workgroup writes up to 32 KB: two halves through the stage
+        dequantize_small_rows<T, C, STAGED, POST, ROWS, 0, ROWS / 2>(s, p, h, w, sc, fast, row0, stage, tid);
+        if constexpr (STAGED) __syncthreads();  // the first half has been copied out of the stage
+        dequantize_small_rows<T, C, STAGED, POST, ROWS, ROWS / 2, ROWS>(s, p, h, w, sc, fast, row0, stage, tid);
+    } else {
+        dequantize_small_rows<T, C, STAGED, POST, ROWS, 0, ROWS>(s, p, h, w, sc, fast, row0, stage, tid);
+    }
 }
 
-template <typename T, bool STAGED, bool TAIL, bool POST>
+template <typename T, bool STAGED, bool TAIL, bool POST, int VECS>
 DEV void dequantize_small_s(const Seg &s, const KCall &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
 {
     // one or two vectors per lane (tftq_small_shape)
-    if (h.c == 1) dequantize_small_c<T, 1, STAGED, TAIL, POST>(s, p, blk, tid, h, stage);
-    else dequantize_small_c<T, 2, STAGED, TAIL, POST>(s, p, blk, tid, h, stage);
+    if (h.c == 1) dequantize_small_c<T, 1, STAGED, TAIL, POST, VECS>(s, p, blk, tid, h, stage);
+    else dequantize_small_c<T, 2, STAGED, TAIL, POST, VECS>(s, p, blk, tid, h, stage);
 }
 
-template <typename T, bool POST>
+template <typename T, bool POST, int VECS>
 DEV void dequantize_small(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage)
 {
     const SmallShape h = small_shape(tftq_small_nvec(s.n, Elem<T>::ESZ), tid, ST_D);
@@ -467,11 +472,11 @@ DEV void dequantize_small(const Seg &s, const KCall &p, int blk, int tid, uint8_
     // same branches for the whole workgroup
     const bool staged = !rows_fill_lines<T>(s) && s.row_stride == s.n && ((s.ptr | (uint64_t)rowb) & 1u) == 0;
     if (s.n % Elem<T>::EPV) {
-        if (staged) dequantize_small_s<T, true, true, POST>(s, p, blk, tid, h, stage);
-        else dequantize_small_s<T, false, true, POST>(s, p, blk, tid, h, stage);
+        if (staged) dequantize_small_s<T, true, true, POST, VECS>(s, p, blk, tid, h, stage);
+        else dequantize_small_s<T, false, true, POST, VECS>(s, p, blk, tid, h, stage);
     } else {
-        if (staged) dequantize_small_s<T, true, false, POST>(s, p, blk, tid, h, stage);
-        else dequantize_small_s<T, false, false, POST>(s, p, blk, tid, h, stage);
+        if (staged) dequantize_small_s<T, true, false, POST, VECS>(s, p, blk, tid, h, stage);
+        else dequantize_small_s<T, false, false, POST, VECS>(s, p, blk, tid, h, stage);
     }
 }
 
@@ -588,7 +593,8 @@ DEV void dequantize_workgroup(const A &args)
     case K_COL1:
         if (s.m > 0) dequantize_col1<T, POST>(s, p, blk * tftq_col1_rows_per_wg(ST_D), tid);
         break;
-    case K_VECS: dequantize_small<T, POST>(s, p, blk, tid, stage); break;
+    case K_VECS: dequantize_small<T, POST, TFTQ_SMALL_VECS>(s, p, blk, tid, stage); break;
+    case K_VECS_FEW: dequantize_small<T, POST, TFTQ_SMALL_VECS_FEW>(s, p, blk, tid, stage); break;
     case K_TILE: dequantize_tile<T, POST>(s, p, blk, tid, stage, coef); break;
     default: break;
     }

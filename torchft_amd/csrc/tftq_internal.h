@@ -38,6 +38,9 @@ enum : uint8_t {
     K_COL1 = 8,    // rows of a single column (1-D tensors); reduce: 4 rows per lane, 1024 per workgroup
     K_COLS = 17,   // columns contiguous in memory (row stride 1: a transposed matrix), quantize: a workgroup of 512 lanes per 16 (fp32: 8) rows
     K_TILE = 18,   // the same in dequantize: a workgroup per tile of 64 rows and 256 columns
+    // for work too little to keep the machine busy (pick_few_kinds):
+    K_COL1_FEW = 19,  // K_COL1, quantize: a pair of rows per lane; reduce: one row, up to 16 peers in flight
+    K_VECS_FEW = 20,  // K_VECS with two vectors per lane
 };
 
 // Helpers shared by the planner (host compiler) and the kernels (hipcc).
@@ -139,11 +142,12 @@ TFTQ_HD static inline int tftq_small_nvec(int n, int esz)
     const int epv = 16 / esz;
     return (n + epv - 1) / epv;
 }
-static inline int tftq_small_rows_per_wg(int nvec, int stage)
+constexpr int TFTQ_SMALL_VECS = 8, TFTQ_SMALL_VECS_FEW = 2;  // per lane: K_VECS, K_VECS_FEW
+static inline int tftq_small_rows_per_wg(int nvec, int stage, int vecs)
 {
     int lt, c;
     tftq_small_shape(nvec, &lt, &c, stage);
-    return (TFTQ_WG >> lt) * (8 / c);
+    return (TFTQ_WG >> lt) * (vecs / c);
 }
 
 // K_COL1, rows of one column.  Quantize and dequantize: a lane takes a few pairs of
@@ -153,8 +157,9 @@ static inline int tftq_small_rows_per_wg(int nvec, int stage)
 // dequantize bf16 118 / 117 / 122 us, fp32 131 / 140 / 147 us.
 // Reduce: four rows per lane and peer.
 constexpr int TFTQ_COL1_PAIRS_Q = 4, TFTQ_COL1_PAIRS_D = 2;
-TFTQ_HD static inline int tftq_col1_rows_per_wg(int stage)
+TFTQ_HD static inline int tftq_col1_rows_per_wg(int stage, bool few = false)
 {
+    if (few) return stage == ST_R ? TFTQ_WG : 2 * TFTQ_WG;  // K_COL1_FEW
     return stage == ST_Q ? 2 * TFTQ_COL1_PAIRS_Q * TFTQ_WG
          : stage == ST_D ? 2 * TFTQ_COL1_PAIRS_D * TFTQ_WG
                          : 4 * TFTQ_WG;
@@ -204,10 +209,11 @@ static_assert(sizeof(Seg) == 64, "Seg must be 64 bytes");
 // Rows of segment s that one workgroup takes in a stage.
 static inline int tftq_rows_per_wg(const Seg &s, int st, int esz, int ws)
 {
-    if (s.kind[st] == K_COL1) return tftq_col1_rows_per_wg(st);
+    if (s.kind[st] == K_COL1 || s.kind[st] == K_COL1_FEW) return tftq_col1_rows_per_wg(st, s.kind[st] == K_COL1_FEW);
     if (s.kind[st] == K_COLS) return tftq_qc_rows(esz);
     if (s.kind[st] == K_TILE) return TFTQ_TILE_ROWS;
-    if (s.kind[st] == K_VECS) return tftq_small_rows_per_wg(tftq_small_nvec(s.n, esz), st);
+    if (s.kind[st] == K_VECS || s.kind[st] == K_VECS_FEW)
+        return tftq_small_rows_per_wg(tftq_small_nvec(s.n, esz), st, s.kind[st] == K_VECS ? TFTQ_SMALL_VECS : TFTQ_SMALL_VECS_FEW);
     const int teams = TFTQ_WG / tftq_team_of(s.kind[st]);
     if (st == ST_R)
         return teams * tftq_reduce_rows_at_once(s.kind[st], s.row_bytes / 4 - 1, ws) * s.side;

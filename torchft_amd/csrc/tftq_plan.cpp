@@ -61,6 +61,13 @@ extern "C" int tftq_layout(int n_tensors, const int64_t *shapes, int ws, int64_t
     return 0;
 }
 
+// Rows that need the kernel variants with more registers (tftq_internal.h).
+static bool wide_quantize(const Seg &s, int esz) { return s.kind[ST_Q] == K_VEC256 && s.n / (16 / esz) > TFTQ_Q_VECS && s.m > 0; }
+static bool wide_reduce(const Seg &s, int ws)
+{
+    return s.kind[ST_R] == K_GEN256 && s.row_bytes / 4 - 1 > TFTQ_R_DWORDS && s.m > 0 && ws <= 64;
+}
+
 static uint8_t pick_io_kind(const Seg &s, int esz)
 {
     // Vector kinds: contiguous rows of at least 64 bytes.  Neither the row start nor the
@@ -253,6 +260,56 @@ static void pick_column_kinds(tftq_plan *p, int st, uint8_t blocks)
         if (stored_by_columns(s) &&
             (best == ALL || cost_of(s, blocks, st, p->esz, p->ws).work < cost_of(s, s.kind[st], st, p->esz, p->ws).work))
             s.kind[st] = blocks;
+}
+
+// Kinds for little work.  K_VECS gives a lane 8 vectors, in 2 to 8 rows one after the other, and K_COL1
+// up to 8 rows (reduce: 4 rows and a peer at a time), which is what a machine full of workgroups wants;
+// where there are too few to fill it, a stage takes as long as one workgroup lives, and a quarter of the
+// work per lane takes half as long.  Measured with the kernels back to back, 8 peers unless said:
+//   quantize, K_VECS: [630, 13] bf16 5.3 -> 3.3 us, [3449, 38] 6.8 -> 3.5, [256, 256] 5.7 -> 3.7; 8 MB of
+//     [20971, 200] 7.1 -> 5.9, of fp32 [55188, 38] 7.3 -> 6.3; 16 MB of 38 to 256 columns 10.3 -> 9.8 to 8.5 ->
+//     8.4, of fp32 [110376, 38] 9.4 -> 9.6; 32 MB mostly slower ([441505, 38] 14.5 -> 16.0);
+//   dequantize, K_VECS: [630, 13] 5.2 -> 3.3, [3449, 38] 5.3 -> 3.6, [256, 256] 4.6 -> 3.2; 8 MB of [20971, 200]
+//     7.5 -> 6.5, of fp32 [55188, 38] 6.2 -> 5.5; rows that fill their 64-byte blocks: 4 MB of [8192, 256] 5.5 ->
+//     4.6, 8 MB of [16384, 256] 5.8 -> 6.0;
+//   either, in long lists: a tensor whose rows are those of one workgroup of K_VECS leaves most of its lanes'
+//     rows empty: 10000 tensors of up to 4096 elements, 16 peers, 48.6 -> 44.3 and 30.2 -> 27.8;
+//   quantize, K_COL1: vectors of up to 4 MB, bf16 2^12 elements 3.6 -> 2.8 us, 2^21 6.9 -> 5.8, 2^22 11.4 -> 12.2
+//     (not in long lists: 48.6 -> 51.0);
+//   reduce, K_COL1, up to 262144 rows per slot, 2 / 4 / 8 / 16 / 64 peers: 2^17 elements 3.2 -> 2.9, 4.3 -> 3.0,
+//     4.9 -> 3.2, 7.1 -> 3.4, 39.5 -> 7.0; 2 to 8 peers at 262144 rows 3.5 -> 3.4, 5.3 -> 3.8, 8.0 -> 5.9, at
+//     524288 6.2 -> 7.2, 6.5 -> 6.7, 10.1 -> 10.6; more peers at 524288 rows 17.9 -> 13.8 (16), 59 -> 47 (64), at
+//     1048576 24.0 -> 24.2 (16), 44.3 -> 45.7 (32); in long lists where a tensor has no more rows than a workgroup of
+//     K_COL1: 20000 tensors, 8 peers, 48.9 -> 43.0 (2 peers: 28.7 -> 34.8).  Not in lists that the kernel for long
+//     rows (R_LONG) takes, which holds no such code, unless they are small as a whole.
+static void pick_few_kinds(tftq_plan *p)
+{
+    constexpr double MB = 1 << 20;
+    constexpr double Q_VECS = 12 * MB, D_VECS = 8 * MB, D_VECS_FILLED = 4 * MB, Q_COL1 = 4 * MB, R_LONG_LIST = 4 * MB;
+    double bytes = 0.0, vector_rows = 0.0;
+    bool wide_q = false, wide_r = false, long_rows = true, vectors_only = true;
+    for (const Seg &s : p->segs) {
+        bytes += (double)s.m * s.n * p->esz;
+        if (s.kind[ST_R] == K_COL1) vector_rows += s.slice_rows;
+        else if (s.m > 0) vectors_only = false;
+        if (s.m > 0 && s.kind[ST_R] != K_COL1 && s.kind[ST_R] != K_GEN64 && s.kind[ST_R] != K_GEN256) long_rows = false;
+        wide_q = wide_q || wide_quantize(s, p->esz);
+        wide_r = wide_r || wide_reduce(s, p->ws);
+    }
+    const bool few_vectors = vector_rows <= (p->ws > 8 ? 524288 : 262144);
+    for (Seg &s : p->segs) {
+        if (s.kind[ST_Q] == K_VECS || s.kind[ST_D] == K_VECS) {
+            const int64_t per_wg = tftq_small_rows_per_wg(tftq_small_nvec(s.n, p->esz), ST_Q, TFTQ_SMALL_VECS);
+            const bool filled = ((int64_t)s.n * p->esz) % 64 == 0;
+            if (s.kind[ST_Q] == K_VECS && !wide_q && (bytes <= Q_VECS || (int64_t)s.slice_rows * p->ws <= per_wg))
+                s.kind[ST_Q] = K_VECS_FEW;
+            if (s.kind[ST_D] == K_VECS && (bytes <= (filled ? D_VECS_FILLED : D_VECS) || s.m <= per_wg)) s.kind[ST_D] = K_VECS_FEW;
+        }
+        if (s.kind[ST_Q] == K_COL1 && !wide_q && p->nseg <= TFTQ_N_INLINE && bytes <= Q_COL1) s.kind[ST_Q] = K_COL1_FEW;
+        if (s.kind[ST_R] == K_COL1 && !wide_r && (vectors_only || !long_rows || bytes <= R_LONG_LIST) &&
+            (few_vectors || (s.slice_rows <= tftq_col1_rows_per_wg(ST_R) && p->ws >= 4)))
+            s.kind[ST_R] = K_COL1_FEW;
+    }
 }
 
 // Bytes one workgroup of segment s moves in reduce.
@@ -476,6 +533,7 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         s.kind[ST_R] = pick_reduce_kind(s, p->ws);
         s.side = (uint8_t)tftq_reduce_rows_side(s.kind[ST_R], s.row_bytes / 4 - 1, s.slice_rows, p->ws);
     }
+    pick_few_kinds(p);
     pick_column_kinds(p, ST_Q, K_COLS);
     pick_column_kinds(p, ST_D, K_TILE);
     for (int i = 0; i < n_tensors; i++) {
@@ -500,15 +558,13 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
     p->reduce_long_rows = p->reduce_one_column = true;
     for (int i = 0; i < n_tensors; i++) {
         const Seg &s = p->segs[(size_t)i];
-        const int nvec = s.n / (16 / p->esz), ndw = s.row_bytes / 4 - 1;
+        const int nvec = s.n / (16 / p->esz);
         if (s.m > 0 && s.kind[ST_R] != K_GEN256 && s.kind[ST_R] != K_GEN64 && s.kind[ST_R] != K_COL1)
             p->reduce_long_rows = false;
-        if (s.m > 0 && s.kind[ST_R] != K_COL1) p->reduce_one_column = false;
-        if (s.kind[ST_Q] == K_VEC256 && nvec > TFTQ_Q_VECS && s.m > 0) p->wide[ST_Q] = true;
+        if (s.m > 0 && s.kind[ST_R] != K_COL1 && s.kind[ST_R] != K_COL1_FEW) p->reduce_one_column = false;
+        if (wide_quantize(s, p->esz)) p->wide[ST_Q] = true;
         if (s.kind[ST_Q] == K_VEC256 && nvec > TFTQ_Q_VECS_WIDE && s.m > 0) p->parked = std::max(p->parked, tftq_q_park_groups(nvec));
-        if (s.kind[ST_R] == K_GEN256 && ndw > TFTQ_R_DWORDS && s.m > 0 && ws <= 64)
-            p->wide[ST_R] = true;
-
+        if (wide_reduce(s, ws)) p->wide[ST_R] = true;
     }
     try {
         if (p->nseg <= TFTQ_N_INLINE) {

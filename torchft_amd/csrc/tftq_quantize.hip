@@ -324,19 +324,19 @@ DEV u32x2 quantize_one(float x)
 
 // Any element stride: four rows per lane, interleaved so that every 8-byte
 // [scale, code] store of a wavefront is contiguous.
-template <typename T>
+template <typename T, int ROWS>
 DEV void quantize_col1_strided(const Seg &s, const KCall &p, int row0, int tid)
 {
     const int m_pad = s.slice_rows * p.ws;
     const float inv = 1.0f / (float)s.slice_rows;
-    float x[4];
+    float x[ROWS];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < ROWS; k++) {
         const int row = min(row0 + k * TFTQ_WG + tid, s.m - 1);
         x[k] = s.m > 0 ? Elem<T>::load(s.ptr, (int64_t)row * s.row_stride) : 0.0f;
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < ROWS; k++) {
         const int row = row0 + k * TFTQ_WG + tid;
         if (row < m_pad) {
             u32x2 o = {0u, 0u};  // padding rows stay zero
@@ -346,32 +346,33 @@ DEV void quantize_col1_strided(const Seg &s, const KCall &p, int row0, int tid)
     }
 }
 
-// Contiguous elements: a lane takes TFTQ_COL1_PAIRS_Q pairs of neighbouring rows, so that it
+// Contiguous elements: a lane takes PAIRS pairs of neighbouring rows, so that it
 // reads two elements with one load (a wavefront reads 256 or 512 contiguous
 // bytes per load even for 2-byte elements) and writes their two packed rows
 // with one 16-byte streaming store (a wavefront writes 1 KB of whole lines).
 // A pair that straddles the end of a slot or of the tensor is stored row by row.
-template <typename T>
+template <typename T, int PAIRS>
 DEV void quantize_col1(const Seg &s, const KCall &p, int row0, int tid)
 {
+    constexpr int ROWS = PAIRS > 1 ? 4 : 2;  // of a step of the strided path
     if (s.row_stride != 1) {  // same for the whole workgroup
 #pragma nounroll
-        for (int r = 0; r < 2 * TFTQ_COL1_PAIRS_Q * TFTQ_WG && row0 + r < s.slice_rows * p.ws; r += 4 * TFTQ_WG)
-            quantize_col1_strided<T>(s, p, row0 + r, tid);
+        for (int r = 0; r < 2 * PAIRS * TFTQ_WG && row0 + r < s.slice_rows * p.ws; r += ROWS * TFTQ_WG)
+            quantize_col1_strided<T, ROWS>(s, p, row0 + r, tid);
         return;
     }
     const int m_pad = s.slice_rows * p.ws;
     const float inv = 1.0f / (float)s.slice_rows;
-    float x[TFTQ_COL1_PAIRS_Q][2];
+    float x[PAIRS][2];
 #pragma unroll
-    for (int k = 0; k < TFTQ_COL1_PAIRS_Q; k++) {
+    for (int k = 0; k < PAIRS; k++) {
         const int row = row0 + 2 * (k * TFTQ_WG + tid);
         x[k][0] = x[k][1] = 0.0f;
         if (row + 1 < s.m) Elem<T>::load2(s.ptr, row, x[k][0], x[k][1]);
         else if (row < s.m) x[k][0] = Elem<T>::load(s.ptr, row);
     }
 #pragma unroll
-    for (int k = 0; k < TFTQ_COL1_PAIRS_Q; k++) {
+    for (int k = 0; k < PAIRS; k++) {
         const int row = row0 + 2 * (k * TFTQ_WG + tid);
         if (row >= m_pad) continue;
         u32x2 a = {0u, 0u}, b = {0u, 0u};  // padding rows stay zero
@@ -457,8 +458,8 @@ DEV float small_row_scale(const u32x4 (&v)[C], const SmallShape &h)
 
 // Rows RBEG * teams .. REND * teams - 1 of the workgroup's rows (those up to `last`)
 // through the LDS stage: g0 is the address of the workgroup's first packed row.
-template <typename T, int C, bool TAIL, int RBEG, int REND>
-DEV void quantize_small_span(const Seg &s, const SmallShape &h, const u32x4 (&v)[8 / C][C], int row0, int last,
+template <typename T, int C, bool TAIL, int ROWS, int RBEG, int REND>
+DEV void quantize_small_span(const Seg &s, const SmallShape &h, const u32x4 (&v)[ROWS][C], int row0, int last,
                              uint8_t *g0, uint8_t *stage, int tid)
 {
     const int nvec = tftq_small_nvec(s.n, Elem<T>::ESZ);
@@ -493,10 +494,11 @@ DEV void quantize_small_span(const Seg &s, const SmallShape &h, const u32x4 (&v)
 // The rows of a workgroup are neighbours; when they lie in one slot their packed rows are
 // one span of bytes, which goes through LDS (copy_out_span) in two halves (rows of 8 to 64
 // 16-bit columns make up to 24 KB per workgroup, more than the stage holds).
-template <typename T, int C, bool TAIL>
+// VECS: vectors per lane, 8 (K_VECS) or 2 (K_VECS_FEW).
+template <typename T, int C, bool TAIL, int VECS>
 DEV void quantize_small_c(const Seg &s, const KCall &p, int blk, int tid, const SmallShape &h, uint8_t *stage)
 {
-    constexpr int ROWS = 8 / C;  // C vectors per lane and row, ROWS rows per lane: 8 or 4
+    constexpr int ROWS = VECS / C;  // C vectors per lane and row, ROWS rows per lane
     const int nvec = tftq_small_nvec(s.n, Elem<T>::ESZ);
     const int nrows = h.teams * ROWS;
     const int row0 = blk * nrows;
@@ -533,9 +535,13 @@ DEV void quantize_small_c(const Seg &s, const KCall &p, int blk, int tid, const 
             // common, the scales of all rows, in front of the branch (20 more registers)
             asm volatile("; rows through the stage");
             uint8_t *g0 = p.packed + (int64_t)slot0 * p.slot_size + s.slot_off + (int64_t)j0 * s.row_bytes;
-            quantize_small_span<T, C, TAIL, 0, ROWS / 2>(s, h, v, row0, last, g0, stage, tid);
-            __syncthreads();  // the first half has been copied out of the stage
-            quantize_small_span<T, C, TAIL, ROWS / 2, ROWS>(s, h, v, row0, last, g0, stage, tid);
+            if constexpr (VECS == TFTQ_SMALL_VECS) {
+                quantize_small_span<T, C, TAIL, ROWS, 0, ROWS / 2>(s, h, v, row0, last, g0, stage, tid);
+                __syncthreads();  // the first half has been copied out of the stage
+                quantize_small_span<T, C, TAIL, ROWS, ROWS / 2, ROWS>(s, h, v, row0, last, g0, stage, tid);
+            } else {
+                quantize_small_span<T, C, TAIL, ROWS, 0, ROWS>(s, h, v, row0, last, g0, stage, tid);
+            }
             return;
         }
     }
@@ -562,21 +568,22 @@ DEV void quantize_small_c(const Seg &s, const KCall &p, int blk, int tid, const 
     }
 }
 
-template <typename T>
+template <typename T, int VECS>
 DEV void quantize_small(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage)
 {
     const SmallShape h = small_shape(tftq_small_nvec(s.n, Elem<T>::ESZ), tid, ST_Q);
     // one or two vectors per lane (tftq_small_shape); same branch for the whole workgroup
     if (s.n % Elem<T>::EPV) {
-        if (h.c == 1) quantize_small_c<T, 1, true>(s, p, blk, tid, h, stage);
-        else quantize_small_c<T, 2, true>(s, p, blk, tid, h, stage);
-    } else if (h.c == 1) quantize_small_c<T, 1, false>(s, p, blk, tid, h, stage);
-    else quantize_small_c<T, 2, false>(s, p, blk, tid, h, stage);
+        if (h.c == 1) quantize_small_c<T, 1, true, VECS>(s, p, blk, tid, h, stage);
+        else quantize_small_c<T, 2, true, VECS>(s, p, blk, tid, h, stage);
+    } else if (h.c == 1) quantize_small_c<T, 1, false, VECS>(s, p, blk, tid, h, stage);
+    else quantize_small_c<T, 2, false, VECS>(s, p, blk, tid, h, stage);
 }
 
 template <typename T, bool WIDE, typename A>
 DEV void quantize_workgroup(const A &args)
 {
+    constexpr bool FEW = !WIDE;  // the kinds for little work (pick_few_kinds)
     __shared__ float lds[4];
     __shared__ __align__(16) uint8_t stage_regular[WIDE ? 16 : Q_STAGE_BYTES];  // see copy_out_span
     // Dynamic LDS of the wide kernel: Q_STAGE_BYTES_WIDE as its stage, or the 40 or 60 KB that the
@@ -600,8 +607,14 @@ DEV void quantize_workgroup(const A &args)
         break;
     case K_GEN8: quantize_gen<T, 8>(s, p, blk * 32 + (tid >> 3), tid & 7); break;
     case K_GEN1: quantize_gen<T, 1>(s, p, blk * 256 + tid, 0); break;
-    case K_COL1: quantize_col1<T>(s, p, blk * tftq_col1_rows_per_wg(ST_Q), tid); break;
-    case K_VECS: quantize_small<T>(s, p, blk, tid, stage); break;
+    case K_COL1: quantize_col1<T, TFTQ_COL1_PAIRS_Q>(s, p, blk * tftq_col1_rows_per_wg(ST_Q), tid); break;
+    case K_VECS: quantize_small<T, TFTQ_SMALL_VECS>(s, p, blk, tid, stage); break;
+    case K_COL1_FEW:
+        if constexpr (FEW) quantize_col1<T, 1>(s, p, blk * tftq_col1_rows_per_wg(ST_Q, true), tid);
+        break;
+    case K_VECS_FEW:
+        if constexpr (FEW) quantize_small<T, TFTQ_SMALL_VECS_FEW>(s, p, blk, tid, stage);
+        break;
     default: break;
     }
 }

@@ -1210,6 +1210,16 @@ DEV void reduce_col1_pairs(const Seg &s, const KCall &p, int j0, int tid)
     }
 }
 
+template <bool GDIV, bool IEEE>
+DEV void reduce_col1_lane(const Seg &s, const KCall &p, int row)
+{
+    // a wavefront none of whose lanes has a row leaves at once
+    if (__builtin_amdgcn_ballot_w64(row < s.slice_rows) == 0) return;
+    const int j = min(row, s.slice_rows - 1);
+    if (p.ws <= 4) reduce_col1_few<4, GDIV, IEEE>(s, p, j, row < s.slice_rows);
+    else reduce_col1_few<16, GDIV, IEEE>(s, p, j, row < s.slice_rows);
+}
+
 // More peers: four rows per lane, a peer at a time (16-byte accesses and two or four peers at a
 // time are 2 to 8 % slower from 4 peers on: 33.5 M rows, 8 peers 51.9 us, 54 to 55 us).
 // PLAIN: always so (the vectors beside matrices in a layer bucket).
@@ -1223,9 +1233,7 @@ DEV void reduce_col1(const Seg &s, const KCall &p, int j0, int tid)
     // a wavefront none of whose lanes has a row (rows go up with k) leaves at once
     if (__builtin_amdgcn_ballot_w64(j0 + tid < s.slice_rows) == 0) return;
     if (!PLAIN && s.slice_rows - j0 <= TFTQ_WG) {
-        const int j = min(j0 + tid, s.slice_rows - 1);
-        if (p.ws <= 4) reduce_col1_few<4, GDIV, IEEE>(s, p, j, j0 + tid < s.slice_rows);
-        else reduce_col1_few<16, GDIV, IEEE>(s, p, j, j0 + tid < s.slice_rows);
+        reduce_col1_lane<GDIV, IEEE>(s, p, j0 + tid);
         return;
     }
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1291,11 +1299,12 @@ template <int FLAVOUR>
 DEV int kind_of(int kind)
 {
     if (FLAVOUR == R_LONG) return kind == K_GEN64 ? K_GEN64 : kind == K_COL1 ? K_COL1 : K_GEN256;
-    return FLAVOUR == R_ONE ? (int)K_COL1 : kind;
+    return FLAVOUR == R_ONE && kind != K_COL1_FEW ? (int)K_COL1 : kind;
 }
 template <bool GDIV, int FLAVOUR, typename A>
 DEV void reduce_workgroup(const A &args)
 {
+    constexpr bool FEW = FLAVOUR == R_ALL || FLAVOUR == R_ONE;  // the kind for little work (pick_few_kinds)
     constexpr bool WIDE = FLAVOUR == R_WIDE;
     __shared__ float lds[16];
     __shared__ float parked[WIDE ? R_PARKED_CHUNKS * 16 * TFTQ_WG : 1];  // wide kernel: 64 KB (two workgroups per CU fit)
@@ -1340,6 +1349,9 @@ DEV void reduce_workgroup(const A &args)
             if (blk * 256 + tid < s.slice_rows) reduce_row_slow<1, true, true>(s, p, blk * 256 + tid, 0, lds);
             break;
         case K_COL1: reduce_col1<true, true, FLAVOUR == R_LONG>(s, p, blk * tftq_col1_rows_per_wg(ST_R), tid); break;
+        case K_COL1_FEW:
+            if constexpr (FEW) reduce_col1_lane<true, true>(s, p, blk * TFTQ_WG + tid);
+            break;
         default: break;
         }
         return;
@@ -1459,6 +1471,9 @@ DEV void reduce_workgroup(const A &args)
         break;
     }
     case K_COL1: reduce_col1<GDIV, false, FLAVOUR == R_LONG>(s, p, blk * tftq_col1_rows_per_wg(ST_R), tid); break;
+    case K_COL1_FEW:
+        if constexpr (FEW) reduce_col1_lane<GDIV, false>(s, p, blk * TFTQ_WG + tid);
+        break;
     default: break;
     }
 }
