@@ -156,13 +156,23 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
     // (Only for tensors with rows enough to keep the machine busy: a tensor of a few rows is
     // done sooner with more lanes per row; 10 000 tensors of up to 4096 elements: 65.0 us
     // with the smaller teams, 62.8 us without.)
-    const bool many = s.slice_rows >= 512;
+    // In groups of more peers it takes more rows to keep the machine busy, as a row lives longer, the
+    // more so the fewer loads its lanes have in flight: packed rows of 700 columns, 3 peers, 1986 rows 4.7
+    // (16 lanes) against 5.5 us (64), 4 peers, 1490 rows 5.9 against 5.3, 8 peers, 2979 rows 8.7 against 6.4, 16
+    // peers 13.9 against 10.5, from 5 peers on even at 4800 to 6000 rows; of 2560 and 3000 columns, 8 peers, 698 rows
+    // 8.9 (64 lanes) against 6.9 us (256), 16 peers, 699 rows 13.8 against 10.6, 1818 rows 18.0 against 19.5.
+    // For the same reason rows of 257 to 512 dwords, two vectors per lane in a wavefront, go to a whole
+    // workgroup: 2048 columns, 8 peers, 256 rows 5.3 -> 4.4 us (1022 rows 6.3 -> 7.7), 16 peers, 511 rows 10.9
+    // -> 8.1, 32 peers, 256 rows 18.3 -> 8.5, 64 peers, 128 rows 33.6 -> 13.3; not in groups of up to 4.
+    const int rows = s.slice_rows;
+    const bool many = rows >= 512;
     if (ndw <= 128) return K_GEN32;
-    if (ndw <= 192 && ws <= 16 && many) return K_GEN16;
+    if (ndw <= 192 && ws <= 16 && rows >= (ws <= 3 ? 512 : ws == 4 ? 2048 : 4096)) return K_GEN16;
     if (ndw <= 256) return K_GEN64;
+    if (ndw <= 512 && ws >= 5 && rows < (ws > 12 ? 768 : 512)) return K_GEN256;
     if (ndw <= 384 && ws <= 32 && many) return K_GEN32;
     if (ndw <= 512) return K_GEN64;
-    if (ndw <= 768 && ws <= 64 && many) return K_GEN64;
+    if (ndw <= 768 && ws <= 64 && rows >= (ws <= 5 ? 512 : ws <= 8 ? 1024 : 1280)) return K_GEN64;
     return K_GEN256;
 }
 

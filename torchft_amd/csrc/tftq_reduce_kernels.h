@@ -626,6 +626,72 @@ DEV void reduce_rows(const Seg &s, const KCall &p, int j, int lane, float *lds, 
     if (valid && lane == 0) orow[0] = as_u(s2);  // :375; all lanes read the old scale before team_max
 }
 
+// Rows of one vector per lane and peer in groups of more than 8 peers: the vectors of WINDOW (12 or 16)
+// peers are in flight at any time; as soon as a peer's has been taken out of its registers, that of the
+// peer WINDOW further on is loaded into them (reduce_rows has 8 in flight and waits for 4 at a time).
+// 64 MB of packed bf16 rows, 16 peers: 4096 columns 19.1 -> 16.1 us (4.2 TB/s), 512 columns 18.8 -> 15.9,
+// 32 peers 4096 columns 17.2 -> 15.9; a few rows, where the loads' latency is all there is: 32 and 64 peers
+// 11.1 -> 7.9 and 19.5 -> 12.5.  A window longer than the group loads its last peer again for nothing:
+// with 16 in place of 12, 256 MB of 4096 columns, 9 and 24 peers 61.8 -> 64.8 and 53.8 -> 56.3.
+// Requirements as in reduce_rows.
+template <int TEAM, int WINDOW, bool GDIV>
+DEV void reduce_rows_window(const Seg &s, const KCall &p, int j, int lane, float *lds, bool valid = true)
+{
+    // the marker keeps the compiler from moving the loads that the two windows have in common in front
+    // of the branch between them (48 registers, which it then spills)
+    if constexpr (WINDOW == 12) asm volatile("; window of 12");
+    const int ndw = (s.row_bytes >> 2) - 1;  // >= 4 here
+    const int ws = p.ws;
+    const int wlane = TEAM >= 64 ? (int)(threadIdx.x & 63u) : lane;
+    const int64_t off = s.slot_off + (int64_t)j * s.row_bytes;
+    const int doff = min(4 * lane, ndw - 4);  // the last vector ends with the row (see reduce_rows)
+    const u32 padmask = (doff == ndw - 4 && (s.n & 3)) ? (1u << (8 * (s.n & 3))) - 1u : 0xFFFFFFFFu;
+
+    const float raw_scale = as_f(peer_row(p, min(wlane, ws - 1), off)[0]);
+    u32x4 w[WINDOW];
+    auto issue = [&](int i, int k) { w[i] = LOAD_STREAM((GLOBAL const u32x4_a4 *)(peer_row(p, min(k, ws - 1), off) + 1 + doff)); };
+#pragma unroll
+    for (int i = 0; i < WINDOW; i++) issue(i, i);
+    __builtin_amdgcn_sched_barrier(0);  // all loads are issued before anything below
+
+    const DivCoef c = make_div(raw_scale == 0.0f ? 1.0f : raw_scale);  // padding rows (:419)
+    if (__builtin_amdgcn_ballot_w64(!c.fast) != 0) {  // same in all wavefronts of the team
+        if (valid) reduce_row_slow<TEAM, GDIV>(s, p, j, lane, lds);  // some peer needs the plain divide
+        return;
+    }
+    float acc[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+    auto take = [&](int i, int k, auto more_c) {
+        const float pr = team_bcast<TEAM>(c.r, k), pl = team_bcast<TEAM>(c.r_lo, k);
+        w[i].w &= padmask;
+        accumulate16(acc, w[i], pr, pl);
+        __builtin_amdgcn_sched_barrier(0);  // peer after peer, and the registers are loaded again behind their last use
+        if constexpr (decltype(more_c)::value) issue(i, k + WINDOW);
+    };
+    int k0 = 0;
+    if constexpr (TEAM >= 64) {
+#pragma nounroll
+        for (; k0 + WINDOW < ws; k0 += WINDOW) {
+#pragma unroll
+            for (int i = 0; i < WINDOW; i++) take(i, k0 + i, std::true_type());
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < WINDOW; i++)
+        if (k0 + i < ws) take(i, k0 + i, std::false_type());
+
+    float amax = 0.0f;  // duplicates held by lanes past the row's end do not change it
+#pragma unroll
+    for (int e = 0; e < 16; e++) amax = fmaxf(amax, __builtin_fabsf(acc[e]));
+    amax = team_max<TEAM>(amax, lds);
+    const float s2 = calc_scale(amax_div<GDIV>(amax, p));  // :340
+    GLOBAL u32 *orow = as_global<u32>(p.packed + (int64_t)p.rank * p.slot_size + off);
+    const u32x4 o = requant16<GDIV>(acc, s2, p);
+    if (valid && 4 * lane < ndw) STORE_CODES(o, (GLOBAL u32x4_a4 *)(orow + 1 + doff));
+    if (valid && lane == 0) orow[0] = as_u(s2);  // :375; all lanes read the old scale before team_max
+}
+
 // Rows of up to 16 * TEAM bytes of codes in teams of 1, 2 or 4 lanes: one vector per lane and
 // peer, groups of up to MAXWS (2, 4, 8, 12 or 16) peers, every load of the row in flight at once.  (One
 // lane per row reads such a row with two or four loads that lie a row apart from its
@@ -1258,12 +1324,24 @@ DEV void reduce_col1(const Seg &s, const KCall &p, int j0, int tid)
     }
 }
 
+// The window of reduce_rows_window for rows of one vector per lane, the one of 12 and 16 that loads
+// fewer peers for nothing; 0: reduce_rows.  (A team of 32 lanes gains from 13 peers on, [3461, 400] 12 peers
+// 8.1 -> 8.7 us, 13 peers 9.2 -> 8.1; more than 16 peers in a team that is no whole wavefront are more than twice
+// slower than in reduce_rows, 19.6 against 40.7 us for 64 MB of 512 columns and 24 peers.)
+DEV int reduce_window(int team, int ws)
+{
+    if (ws <= 8 || (team == 32 && ws <= 12) || (team < 64 && ws > 16)) return 0;
+    return (ws + 11) / 12 * 12 < (ws + 15) / 16 * 16 ? 12 : 16;
+}
+
 // reduce_rows for a team of TEAM lanes with UNITS vectors per lane and peer: groups of 8 and
 // of 4 peers run straight-line code (averages over such groups never need GDIV)
 #define TFTQ_REDUCE_ROWS(TEAM, UNITS, ...)                                                        \
     do {                                                                                          \
         if (!GDIV && p.ws == 8) reduce_rows<TEAM, UNITS, true, GDIV, GDIV ? 0 : 8>(__VA_ARGS__);  \
         else if (!GDIV && p.ws == 4) reduce_rows<TEAM, UNITS, true, GDIV, GDIV ? 0 : 4>(__VA_ARGS__); \
+        else if (UNITS == 1 && TEAM > 8 && reduce_window(TEAM, p.ws) == 16) reduce_rows_window<TEAM, 16, GDIV>(__VA_ARGS__); \
+        else if (UNITS == 1 && TEAM > 8 && TEAM != 32 && reduce_window(TEAM, p.ws) == 12) reduce_rows_window<TEAM, 12, GDIV>(__VA_ARGS__); \
         else reduce_rows<TEAM, UNITS, true, GDIV>(__VA_ARGS__);                                   \
     } while (0)
 
