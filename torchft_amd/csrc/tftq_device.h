@@ -396,6 +396,7 @@ DEV bool locate(const KOne &a, KCall &p, Seg &s, int &blk)
     s.row_bytes = ((a.n + 3) & ~3) + 4;
     s.kind[STAGE] = a.kind;
     s.side = a.side;
+    s.lg_groups = a.lg_groups;
     p.packed = a.packed;
     p.slot_size = (int64_t)a.slice_rows * s.row_bytes;
     p.ws = a.ws;
@@ -531,6 +532,7 @@ DEV int64_t row_addr_fast(const Seg &s, int64_t slot_size, int row, float inv)
 // and the last 16 bytes of the span can be partial and go out as halfwords.
 #define LDS_AS __attribute__((address_space(3)))
 
+template <int LANES = TFTQ_WG>
 DEV void copy_out_span(const uint8_t *stage, uint8_t *g0, int len, int tid)
 {
     const int mis = (int)((uintptr_t)g0 & 127u);
@@ -538,7 +540,7 @@ DEV void copy_out_span(const uint8_t *stage, uint8_t *g0, int len, int tid)
     const int end = mis + len;
     const int nchunks = (end + 15) >> 4;
 #pragma nounroll
-    for (int c = tid; c < nchunks; c += TFTQ_WG) {
+    for (int c = tid; c < nchunks; c += LANES) {
         const int lo = 16 * c;
         const u32x4 v = *(const LDS_AS u32x4 *)(const LDS_AS uint8_t *)(stage + lo);
         if (lo >= mis && lo + 16 <= end) {
@@ -686,6 +688,7 @@ static inline void fill_args(const tftq_plan *plan, int stage, const void *const
         a.nwg = plan->nwg[stage];
         a.kind = s.kind[field];
         a.side = s.side;
+        a.lg_groups = s.lg_groups;
         a.natural = natural;
         a.div_mode = (uint8_t)what.div_mode;
         a.post_scale = what.post_scale;

@@ -36,7 +36,7 @@ enum : uint8_t {
     K_GEN64 = 6,   // one wavefront per row
     K_GEN256 = 7,  // one workgroup per row (reduce only)
     K_COL1 = 8,    // rows of a single column (1-D tensors); reduce: 4 rows per lane, 1024 per workgroup
-    K_COLS = 17,   // columns contiguous in memory (row stride 1: a transposed matrix), quantize: a workgroup of 512 lanes per 16 (fp32: 8) rows
+    K_COLS = 17,   // columns contiguous in memory (row stride 1: a transposed matrix), quantize: a workgroup of 512 lanes per 16 to 256 (fp32: 8 to 128) rows
     K_TILE = 18,   // the same in dequantize: a workgroup per tile of 64 rows and 256 columns
     // for work too little to keep the machine busy (pick_few_kinds):
     K_COL1_FEW = 19,  // K_COL1, quantize: a pair of rows per lane; reduce: one row, up to 16 peers in flight
@@ -68,11 +68,17 @@ TFTQ_HD static inline int tftq_team_of(uint8_t kind)
 
 constexpr int TFTQ_WG = 256;       // threads per workgroup, all kernels but k_quantize_cols
 
-// K_COLS (k_quantize_cols): TFTQ_QC_WG lanes hold TFTQ_QC_GROUPS groups of rows, 16 bytes of a
-// column each.  The blocks of a tensor start at the slots' first rows, so a block's packed rows
-// are neighbours.
-constexpr int TFTQ_QC_WG = 512, TFTQ_QC_GROUPS = 2;
-TFTQ_HD static inline int tftq_qc_rows(int esz) { return TFTQ_QC_GROUPS * (16 / esz); }
+// K_COLS (k_quantize_cols): TFTQ_QC_WG lanes hold 2, 4, 8, 16 or 32 groups of rows (Seg::lg_groups),
+// 16 bytes of a column each.  The blocks of a tensor start at the slots' first rows, so a block's
+// packed rows are neighbours.
+constexpr int TFTQ_QC_WG = 512;
+TFTQ_HD static inline int tftq_qc_rows(int lg_groups, int esz) { return (16 / esz) << lg_groups; }
+// steps, one vector of four columns for every lane each, that a row of n columns takes
+TFTQ_HD static inline int tftq_qc_steps(int n, int lg_groups)
+{
+    const int step = 4 * TFTQ_QC_WG >> lg_groups;
+    return (n + step - 1) / step;
+}
 // K_TILE
 constexpr int TFTQ_TILE_ROWS = 64, TFTQ_TILE_COLS = 256;
 
@@ -202,7 +208,8 @@ struct Seg {
     int32_t row_bytes;   // 4 + round_up(n, 4)
     int32_t wg_begin[3]; // first workgroup of this segment, per stage
     uint8_t kind[3];     // lane mapping, per stage
-    uint8_t side;        // reduce: rows that a team of 2 to 32 lanes takes at once (tftq_reduce_rows_side)
+    uint8_t side : 4;    // reduce: rows that a team of 2 to 32 lanes takes at once (tftq_reduce_rows_side)
+    uint8_t lg_groups : 4;  // quantize, K_COLS: 1 to 5 (pick_groups)
 };
 static_assert(sizeof(Seg) == 64, "Seg must be 64 bytes");
 
@@ -210,7 +217,7 @@ static_assert(sizeof(Seg) == 64, "Seg must be 64 bytes");
 static inline int tftq_rows_per_wg(const Seg &s, int st, int esz, int ws)
 {
     if (s.kind[st] == K_COL1 || s.kind[st] == K_COL1_FEW) return tftq_col1_rows_per_wg(st, s.kind[st] == K_COL1_FEW);
-    if (s.kind[st] == K_COLS) return tftq_qc_rows(esz);
+    if (s.kind[st] == K_COLS) return tftq_qc_rows(s.lg_groups, esz);
     if (s.kind[st] == K_TILE) return TFTQ_TILE_ROWS;
     if (s.kind[st] == K_VECS || s.kind[st] == K_VECS_FEW)
         return tftq_small_rows_per_wg(tftq_small_nvec(s.n, esz), st, s.kind[st] == K_VECS ? TFTQ_SMALL_VECS : TFTQ_SMALL_VECS_FEW);
@@ -312,7 +319,8 @@ struct tftq_plan {
     bool reduce_long_rows;     // every row of the list runs in a team of 64 or 256 lanes in reduce or has one column (k_reduce's R_LONG)
     bool reduce_one_column;    // every row of the list has one column (R_ONE)
     int parked;                // quantize: groups of 5 vectors per lane (20 KB of LDS each, up to 3) that the longest row parks in LDS (rows above TFTQ_Q_VECS_WIDE)
-    int cols_most;             // quantize: columns of the widest K_COLS tensor
+    int cols_most;             // quantize: most steps of a K_COLS tensor
+    bool cols_two;             // quantize: every K_COLS tensor has 2 groups of rows
     Dealt dealt[N_LAUNCHES];   // inline table only
     int32_t dealt_per_xcd[N_LAUNCHES];  // inline table only: workgroups of the busiest XCD
     bool natural[N_LAUNCHES];  // inline table only: workgroup ids keep their order (see deal_to_xcds)
@@ -355,7 +363,8 @@ struct KOne {
     };
     int32_t m, n, slice_rows, ws;
     int32_t nwg;         // workgroups
-    uint8_t kind, side;  // of the stage
+    uint8_t kind;        // of the stage
+    uint8_t side : 4, lg_groups : 4;  // as in Seg
     uint8_t natural;     // see natural_order
     uint8_t div_mode;    // as in KCall
     float post_scale;    // dequantize: as in KCall

@@ -178,7 +178,7 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
 
 // Tensors whose columns are contiguous in memory (transposed matrices).  Their rows have two kernels
 // each way: teams of 8 or 64 lanes with an element per lane and access (K_GEN8 up to 128 columns,
-// K_GEN64), or blocks of 16 (fp32: 8) rows in quantize (K_COLS, a launch of its own) and tiles of 64
+// K_GEN64), or blocks of 16 to 256 (fp32: half as many) rows in quantize (K_COLS, a launch of its own) and tiles of 64
 // rows and 256 columns in dequantize (K_TILE).  The blocks and tiles read and write whole pieces of
 // columns, but cost the same however many rows and columns of them the tensor has (a block never
 // crosses a slot), so they lose on narrow tensors and where a slot has few rows of one.
@@ -200,15 +200,26 @@ constexpr double COST_HIDDEN = 4.2;  // of a latency, beside other tensors in th
 // rows and one transposed [64, 64], 9.6 us in one launch and 12.6 in two; [1024, 1024], 15.8 and 13.4.
 constexpr double COST_OVERLAP = 0.8;
 
+// Quantize's blocks of 2^lg groups of rows.  A block's time is a fixed part per step and the bytes it
+// moves at 6.2 TB/s, slower by SLOW where it uses a part of a line only and by more where two workgroups no
+// longer fit a compute unit (more than 4 steps); it counts padding lanes and rows as if they were real.
+static Cost cost_of_blocks(const Seg &s, int lg, int esz, int ws)
+{
+    static const double SLOW[2][6] = {{0, 1.3, 1.15, 1.05, 1.05, 1.05}, {0, 2.1, 1.45, 1.2, 1.05, 1.05}};  // 16 bits, fp32
+    const bool half = esz == 2;
+    const int rows = tftq_qc_rows(lg, esz), steps = tftq_qc_steps(s.n, lg);
+    const int held = steps <= 2 ? steps : steps <= 4 ? 4 : steps <= 8 ? 8 : 12;
+    double bytes = (double)rows * s.n * (esz + 1) * SLOW[!half][lg] * (held > 4 ? half ? 1.4 : 1.1 : 1.0);
+    if (steps > 12) bytes *= 2.0 - 12.0 / steps;  // what is read twice
+    const double block = sqrt(4.5e-3 * held * 4.5e-3 * held + bytes / 6.2e6 * (bytes / 6.2e6));
+    return {half ? 2.9 + 1.1 * held + 0.0006 * s.n : 2.6 + 0.6 * held + 0.0011 * s.n, (double)ws * ((s.slice_rows + rows - 1) / rows) * block};
+}
+
 static Cost cost_of(const Seg &s, uint8_t kind, int st, int esz, int ws)
 {
     const double m = s.m, n = s.n, padded = (double)s.slice_rows * ws;
     const bool half = esz == 2;
-    if (kind == K_COLS) {
-        const int rows = tftq_qc_rows(esz);
-        const double block = half ? 4.3e-3 + 3.6e-6 * n : 3.6e-3 + 3.0e-6 * n;
-        return {(half ? 4.1 : 3.8) + 0.0009 * n, (double)ws * ((s.slice_rows + rows - 1) / rows) * (block + 5e-10 * n * n)};
-    }
+    if (kind == K_COLS) return cost_of_blocks(s, s.lg_groups, esz, ws);
     if (kind == K_TILE) {
         const double tiles = (double)((s.m + TFTQ_TILE_ROWS - 1) / TFTQ_TILE_ROWS) * ((s.n + TFTQ_TILE_COLS - 1) / TFTQ_TILE_COLS);
         return {4.3 + 0.006 * std::min(n, 256.0), tiles * 1.45e-3 + m * n * esz * 1.35e-7};
@@ -220,21 +231,62 @@ static Cost cost_of(const Seg &s, uint8_t kind, int st, int esz, int ws)
                            : Cost{3.0 + 0.021 * n, m * (n * 1.0e-6 + (half ? 1.4e-5 : 2.0e-5))};
 }
 
+static bool stored_by_columns(const Seg &s, int st, int esz)
+{
+    // (fp32 rows of up to 32 columns stay with their teams in quantize.)
+    return s.row_stride == 1 && s.m >= 16 / esz && s.m < INT32_MAX - 4096 &&  // the blocks round up
+           (s.kind[st] == K_GEN8 || s.kind[st] == K_GEN64) && (st != ST_Q || esz == 2 || s.n > 32);
+}
+
+// How many groups of rows a block of quantize holds (Seg::lg_groups).  More make whole lines of what it
+// reads and fewer blocks, and fewer columns per step: rows of more than 12 steps keep 2 groups, more than 4
+// groups are for rows of up to 4 steps, and more than 4 steps (a workgroup per compute unit) for tensors
+// of 192 blocks: fp32 [1797, 3500] 10.4 us in 2 groups, 14.1 in 120 blocks of 4.  A tensor takes the groups that are the least work, or, if the launch
+// has little else to do, those that are done soonest.  us in 2 / 4 / 8 / 16 / 32 groups, bf16, 8 slots:
+// [2330168, 18] 920 / 458 / 232 / 126 / 65, [42799, 147] 18.5 / 11.0 / 8.0 / 7.0 / 8.1, [3495, 300] 4.7 / 4.6 / 5.8 /
+// 8.3 / -, [41943, 1000] 30.4 / 25.1 / 21.9 / - / -, [1048, 1000] 5.1 / 6.3 / 9.0 / - / -, [11983, 3500] 28.9 / 34.0 / - / -
+// / -, fp32 63.6 / 51.6.
+static void pick_groups(tftq_plan *p)
+{
+    double least[2] = {0.0, 0.0};  // all tensors' work with the groups that are the least of it; one tensor's
+    for (int pass = 0; pass < 2; pass++)
+        for (Seg &s : p->segs) {
+            if (!stored_by_columns(s, ST_Q, p->esz)) continue;
+            Cost cost[6];
+            int most = 1;
+            for (int lg = 1; lg <= 5 && (lg == 1 || tftq_qc_steps(s.n, lg) <= (lg == 2 ? 12 : 4)); lg++) {
+                const int rows = tftq_qc_rows(lg, p->esz);
+                if (lg > 1 && tftq_qc_steps(s.n, lg) > 4 && (int64_t)p->ws * ((s.slice_rows + rows - 1) / rows) < 192) break;
+                cost[lg] = cost_of_blocks(s, lg, p->esz, p->ws);
+                most = lg;
+            }
+            least[1] = HUGE_VAL;
+            for (int lg = 1; lg <= most; lg++) least[1] = std::min(least[1], cost[lg].work);
+            if (pass == 0) {
+                least[0] += least[1];
+                continue;
+            }
+            double best = HUGE_VAL;
+            for (int lg = 1; lg <= most; lg++) {
+                const double t = std::max(cost[lg].latency, COST_BASE + least[0] - least[1] + cost[lg].work);
+                if (t >= best) continue;
+                best = t;
+                s.lg_groups = (uint8_t)lg;
+            }
+        }
+}
+
 // Chooses for a stage between the teams that the tensors have been given and `blocks` (K_COLS or
 // K_TILE): for none of them, for those that it makes less work, or for all (a few tensors that the
 // machine takes at once, where only the latency counts).
 static void pick_column_kinds(tftq_plan *p, int st, uint8_t blocks)
 {
-    auto stored_by_columns = [&](const Seg &s) {
-        return s.row_stride == 1 && s.m >= 16 / p->esz && s.m < INT32_MAX - 4096 &&  // the blocks round up
-               (s.kind[st] == K_GEN8 || s.kind[st] == K_GEN64);
-    };
     enum { NONE, LESS_WORK, ALL, N_WAYS };
     // per way: what is left to the teams, what goes to the blocks
     Cost teams[N_WAYS] = {}, taken[N_WAYS] = {};
     bool any[N_WAYS] = {}, others = false;
     for (const Seg &s : p->segs) {
-        if (!stored_by_columns(s)) {
+        if (!stored_by_columns(s, st, p->esz)) {
             others = others || s.m > 0;
             continue;
         }
@@ -267,7 +319,7 @@ static void pick_column_kinds(tftq_plan *p, int st, uint8_t blocks)
     }
     if (!any[best]) return;
     for (Seg &s : p->segs)
-        if (stored_by_columns(s) &&
+        if (stored_by_columns(s, st, p->esz) &&
             (best == ALL || cost_of(s, blocks, st, p->esz, p->ws).work < cost_of(s, s.kind[st], st, p->esz, p->ws).work))
             s.kind[st] = blocks;
 }
@@ -522,6 +574,7 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         delete p;
         return rc;
     }
+    p->cols_two = true;
     int64_t wg[N_LAUNCHES] = {0, 0, 0, 0};
     int32_t (*wgs)[N_LAUNCHES] = (int32_t (*)[N_LAUNCHES])wgs_flat.data();  // workgroups per segment and launch
     for (int i = 0; i < n_tensors; i++) {
@@ -544,6 +597,7 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         s.side = (uint8_t)tftq_reduce_rows_side(s.kind[ST_R], s.row_bytes / 4 - 1, s.slice_rows, p->ws);
     }
     pick_few_kinds(p);
+        pick_groups(p);
     pick_column_kinds(p, ST_Q, K_COLS);
     pick_column_kinds(p, ST_D, K_TILE);
     for (int i = 0; i < n_tensors; i++) {
@@ -560,7 +614,10 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
                 return TFTQ_E_SHAPE;
             }
         }
-        if (s.kind[ST_Q] == K_COLS) p->cols_most = std::max(p->cols_most, s.n);
+        if (s.kind[ST_Q] == K_COLS) {
+            p->cols_most = std::max(p->cols_most, tftq_qc_steps(s.n, s.lg_groups));
+            p->cols_two = p->cols_two && s.lg_groups == 1;
+        }
     }
     for (int st = 0; st < N_LAUNCHES; st++) p->nwg[st] = (int32_t)wg[st];
     p->wide[ST_Q] = p->wide[ST_R] = p->wide[ST_D] = false;

@@ -638,21 +638,216 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize_one(TFTQ_ONE
 // ---------------------------------------------------------------------------
 // A transposed matrix: a row's elements are a whole column length apart, a column's lie side by
 // side.  A lane takes 16 bytes of a column, 8 (fp32: 4) rows, of four neighbouring columns: it then
-// holds one dword of codes of each of these rows, and the 32 lanes that share its rows write 128
-// neighbouring bytes of a packed row with one store, with no exchange between lanes.  Only the row
-// maxima go through LDS.  A block of 16 (fp32: 8) rows stays in the registers of a workgroup of 512
-// lanes, up to NS steps of 1024 columns, so that the tensor is read once; what a row has beyond
-// that is read twice.  Bound by the L1's requests in flight, of which a block uses 29 bytes each
-// (5.2 million for 151 MB; HBM traffic is the algorithmic 1.08 times): transposed [4096, 14336] and
-// [4096, 4096] bf16, 227 MB, one element per lane and access and two passes 486 us, this kernel 79 us.
-// Alone, [4096, 14336] 66 to 69 us: with blocks of 32 rows 101 (half the compute units idle), workgroups of 256 lanes 89
-// (half of the row read twice), of 1024 lanes 72, streaming loads 77 (neighbouring blocks share
-// lines); a launch for the maxima and one for tiles of 64 rows 82 us.  Where the blocks lose against
-// teams of lanes (few columns, few rows per slot) the planner leaves them out: pick_column_kinds.
-template <typename T, int NS>
-DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, float *part, float *scale)
+// holds one dword of codes of each of these rows, with no exchange between lanes.  Only the row
+// maxima go through LDS, and the packed rows where a block's fit (they are one span of bytes:
+// copy_out_span).  A block of G such groups of rows stays in the registers of a workgroup of 512
+// lanes, up to NS steps of 2048 / G columns, so that the tensor is read once; what a row has beyond
+// that, in 2 groups only, is read twice.  Bound by memory where 8 or more groups make whole lines of
+// what a block reads; with 2 groups it uses 32 bytes of a line and the L1's requests in flight are the
+// limit.  bf16, 8 slots, 2 groups and dwords stored from the registers -> with the groups that
+// pick_groups takes and the stage: [285326, 147] 101 -> 26 us (4.8 TB/s), [1310720, 32] 447 -> 29, [41943, 1000]
+// 50 -> 22, [20971, 2000] 46 -> 23, [6990, 6000] 48 -> 34; fp32 [285326, 147] 161 -> 42, [41943, 1000] 75 -> 46.
+// [4096, 14336] in 2 groups, 66 to 69 us: with blocks of 32 rows 101 (half the compute units idle), workgroups of
+// 256 lanes 89 (half of the row read twice), of 1024 lanes 72, streaming loads 77 (neighbouring blocks
+// share lines); a launch for the maxima and one for tiles of 64 rows 82 us.  Where the blocks lose against
+// teams of lanes (few rows per slot) the planner leaves them out: pick_column_kinds.
+template <typename T, int G, int NS, int STAGE>
+DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage, float *scale)
 {
-    constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, G = TFTQ_QC_GROUPS, K = 64 / G, RB = G * EPV;
+    constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, K = 64 / G, RB = G * EPV;
+    constexpr int WAVES = TFTQ_QC_WG / 64, STEP = 4 * K * WAVES;  // columns per step
+    constexpr int RPD = 4 / ESZ;                                  // rows per dword of a column
+    constexpr int SETS = G <= 16 ? 4 : 2;                         // of lanes that hold all groups, per wavefront
+    constexpr bool STAGED = RB * (4 + NS * STEP) + 127 <= STAGE;  // the block's packed rows fit the stage
+    static_assert(SETS * WAVES * RB * 4 <= STAGE, "the maxima fit the stage");
+    float *part = (float *)stage;
+    const int per_slot = (s.slice_rows + RB - 1) / RB;
+    const int slot = blk / per_slot;
+    const int j0 = (blk - slot * per_slot) * RB;
+    const int srow = slot * s.slice_rows;  // the slot's first row
+    const int real = min(max(s.m - srow, 0), s.slice_rows);
+    GLOBAL uint8_t *g0 = as_global<uint8_t>(p.packed + (int64_t)slot * p.slot_size + s.slot_off + (int64_t)j0 * s.row_bytes);
+    if (!STAGED || j0 >= real) {   // padding rows: zero (:93-95 on a zero-filled buffer)
+        const int z0 = max(real - j0, 0), z1 = min(RB, s.slice_rows - j0);
+        for (int z = z0; z < z1; z++)
+            for (int d = tid; d < (s.row_bytes >> 2); d += TFTQ_QC_WG) ((GLOBAL u32 *)(g0 + (int64_t)z * s.row_bytes))[d] = 0;
+    }
+    if (j0 >= real) return;  // the whole workgroup
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+    const int g = l & (G - 1), k = l / G;
+    const int ndw = (s.row_bytes >> 2) - 1;
+    // the lane's rows; the last group of the tensor is moved back to end with it (its rows are
+    // another lane's too: both write the same bytes)
+    const int first = min(srow + j0 + g * EPV, s.m - EPV);
+    const int jf = first - srow - j0, jstop = min(RB, real - j0);  // rows jf + i in [0, jstop) are written
+    const uint64_t col0 = s.ptr + (uint64_t)((int64_t)first * ESZ);
+    const int64_t cs = s.col_stride * ESZ;
+    const int c0 = 4 * (wave * K + k);
+    auto load = [&](u32x4 (&v)[4], int base) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)  // columns past the last one re-read it
+            v[e] = *as_global<const u32x4_a2>(col0 + (uint64_t)((int64_t)min(base + c0 + e, s.n - 1) * cs));
+    };
+    float amax[EPV];
+#pragma unroll
+    for (int i = 0; i < EPV; i++) amax[i] = 0.0f;
+    auto maxima = [&](const u32x4 (&v)[4]) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float f[EPV];
+            Elem<T>::unpack(v[e], f);
+#pragma unroll
+            for (int i = 0; i < EPV; i++) amax[i] = fmaxf(amax[i], __builtin_fabsf(f[i]));
+        }
+    };
+    u32x4 v[NS][4];
+#pragma unroll
+    for (int t = 0; t < NS; t++) load(v[t], t * STEP);
+#pragma unroll
+    for (int t = 0; t < NS; t++) maxima(v[t]);
+#pragma nounroll
+    for (int base = NS * STEP; base < s.n; base += STEP) {  // first pass over the rest
+        u32x4 x[4];
+        load(x, base);
+        maxima(x);
+    }
+#pragma unroll
+    for (int i = 0; i < EPV; i++) {  // over the lanes of the same group in a row of 16
+        if constexpr (G <= 8) amax[i] = fmaxf(amax[i], dpp_mov<0x128>(amax[i]));  // row_ror:8
+        if constexpr (G <= 4) amax[i] = fmaxf(amax[i], dpp_mov<0x124>(amax[i]));  // row_ror:4
+        if constexpr (G <= 2) amax[i] = fmaxf(amax[i], dpp_mov<0x122>(amax[i]));  // row_ror:2
+        if ((l & 15) < G) part[(wave * SETS + l / (64 / SETS)) * RB + g * EPV + i] = amax[i];
+    }
+    static_assert(G == 2 || G == 4 || G == 8 || G == 16 || G == 32, "the rotations above");
+    __syncthreads();
+    if (tid < RB) {
+        float a = 0.0f;
+#pragma unroll
+        for (int w = 0; w < SETS * WAVES; w++) a = fmaxf(a, part[w * RB + tid]);
+        const float sc = calc_scale(a);
+        scale[tid] = sc;
+        if constexpr (!STAGED) {
+            const int j = min(srow + j0 + tid / EPV * EPV, s.m - EPV) - srow - j0 + tid % EPV;
+            if (j >= 0 && j < jstop) *(GLOBAL u32 *)(g0 + (int64_t)j * s.row_bytes) = as_u(sc);
+        }
+    }
+    __syncthreads();  // the maxima have been read: the stage is free
+    LDS_AS uint8_t *span = (LDS_AS uint8_t *)(stage + (int)((uintptr_t)g0 & 127u));  // STAGED: where g0 is
+    if constexpr (STAGED) {
+        const int j = min(srow + j0 + tid / EPV * EPV, s.m - EPV) - srow - j0 + tid % EPV;
+        if (tid < RB && j >= 0 && j < jstop) *(LDS_AS u32 *)(span + j * s.row_bytes) = as_u(scale[tid]);
+        for (int z = real - j0; z < min(RB, s.slice_rows - j0); z++)  // padding rows
+            for (int d = tid; d < (s.row_bytes >> 2); d += TFTQ_QC_WG) ((LDS_AS u32 *)(span + z * s.row_bytes))[d] = 0;
+    }
+    float sc[EPV];
+#pragma unroll
+    for (int i = 0; i < EPV; i++) sc[i] = scale[g * EPV + i];
+    GLOBAL uint8_t *out = g0 + (int64_t)jf * s.row_bytes + 4;
+    auto store = [&](const u32x4 (&v)[4], int base) {
+        const int d = (base + c0) >> 2;  // the lane's dword of the payload
+        if (d >= ndw) return;
+        const int over = 4 * d + 4 - s.n;  // columns of the dword past the last one
+        const u32 mask = over > 0 ? 0xFFFFFFFFu >> (8 * over) : 0xFFFFFFFFu;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {  // dword w of the four vectors: rows RPD * w ...
+            float f[4][RPD];
+#pragma unroll
+            for (int e = 0; e < 4; e++) unpack_dword<T>(v[e][w], f[e]);
+#pragma unroll
+            for (int h = 0; h < RPD; h++) {
+                const int i = RPD * w + h;
+                const u32 o = pack_fp8x4(f[0][h] * sc[i], f[1][h] * sc[i], f[2][h] * sc[i], f[3][h] * sc[i]) & mask;
+                if (jf + i >= 0 && jf + i < jstop) {
+                    if constexpr (STAGED) ((LDS_AS u32 *)(span + (jf + i) * s.row_bytes + 4))[d] = o;
+                    // plain stores: a packed row starts anywhere in its line, the L2 puts the runs together
+                    else ((GLOBAL u32 *)(out + (int64_t)i * s.row_bytes))[d] = o;
+                }
+            }
+        }
+    };
+#pragma unroll
+    for (int t = 0; t < NS; t++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) asm volatile("" : "+v"(v[t][e].x), "+v"(v[t][e].y), "+v"(v[t][e].z), "+v"(v[t][e].w));
+    }
+#pragma unroll
+    for (int t = 0; t < NS; t++) store(v[t], t * STEP);
+#pragma nounroll
+    for (int base = NS * STEP; base < s.n; base += STEP) {  // second pass over the rest
+        u32x4 x[4];
+        load(x, base);
+        store(x, base);
+    }
+    if constexpr (STAGED) {
+        __syncthreads();
+        copy_out_span<TFTQ_QC_WG>(stage, (uint8_t *)g0, min(RB, s.slice_rows - j0) * s.row_bytes, tid);
+    }
+}
+
+// Steps that stay in registers: 12 for lists with rows of more than 4 steps (250 registers, two
+// wavefronts per SIMD; 14 spill), else 4 (115 registers, four).  More than 4 groups take no more than 4
+// steps (pick_groups).
+constexpr int QC_MOST = 12;
+// The stage: all packed rows of a block of up to 4 steps, or 8 (fp32, 4 groups: 12).  fp32 in 2 groups
+// does without: [41943, 1000] 75 us straight from the registers and 77 through the stage.
+template <typename T, int NSMAX>
+struct ColsStage {
+    static constexpr int VECTORS = NSMAX == 4 ? 4 : Elem<T>::ESZ == 4 ? NSMAX : 8;
+    static constexpr int BYTES = TFTQ_QC_WG * 4 * VECTORS * Elem<T>::EPV + 32 * Elem<T>::EPV * 4 + 128;
+};
+constexpr int QC_LEAST_STAGE = 4096;  // for the maxima of up to 4 groups alone
+template <typename T, int G, int NSMAX>
+DEV void quantize_cols_steps(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage, float *scale)
+{
+    constexpr int STAGE = ColsStage<T, NSMAX>::BYTES;
+    constexpr bool DIRECT = Elem<T>::ESZ == 4 && G == 2;
+    const int steps = tftq_qc_steps(s.n, __builtin_ctz(G));  // same for the whole workgroup
+    constexpr int SHORT = DIRECT ? QC_LEAST_STAGE : STAGE;
+    if (steps <= 1) quantize_cols<T, G, 1, SHORT>(s, p, blk, tid, stage, scale);
+    else if (steps <= 2) quantize_cols<T, G, 2, SHORT>(s, p, blk, tid, stage, scale);
+    else if (NSMAX == 4 || steps <= 4) quantize_cols<T, G, 4, SHORT>(s, p, blk, tid, stage, scale);
+    else if constexpr (NSMAX > 4) {
+        if (steps <= 8) quantize_cols<T, G, 8, SHORT>(s, p, blk, tid, stage, scale);
+        else if (Elem<T>::ESZ == 4 && G == 4) quantize_cols<T, G, NSMAX, STAGE>(s, p, blk, tid, stage, scale);
+        else quantize_cols<T, G, NSMAX, QC_LEAST_STAGE>(s, p, blk, tid, stage, scale);
+    }
+}
+template <typename T, int NSMAX, typename A>
+DEV void quantize_cols_workgroup(const A &args)
+{
+    __shared__ __align__(16) uint8_t stage[ColsStage<T, NSMAX>::BYTES];  // the rows' maxima, then see copy_out_span
+    __shared__ float scale[32 * Elem<T>::EPV];
+    Seg s;
+    KCall p;
+    int blk;
+    if (!locate<ST_Q>(args, p, s, blk)) return;
+    const int tid = threadIdx.x;
+    switch (s.lg_groups) {
+    case 5: quantize_cols_steps<T, 32, 4>(s, p, blk, tid, stage, scale); break;
+    case 4: quantize_cols_steps<T, 16, 4>(s, p, blk, tid, stage, scale); break;
+    case 3: quantize_cols_steps<T, 8, 4>(s, p, blk, tid, stage, scale); break;
+    case 2: quantize_cols_steps<T, 4, NSMAX>(s, p, blk, tid, stage, scale); break;
+    default: quantize_cols_steps<T, 2, NSMAX>(s, p, blk, tid, stage, scale); break;
+    }
+}
+template <typename T, typename A, int NSMAX>
+__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols(const A args)
+{
+    quantize_cols_workgroup<T, NSMAX>(args);
+}
+template <typename T, int NSMAX>
+__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols_one(TFTQ_ONE_PARAMS)
+{
+    quantize_cols_workgroup<T, NSMAX>(one_of(TFTQ_ONE));
+}
+
+// Lists whose tensors all have 2 groups and some of them more than 4 steps: the same straight from the
+// registers, in a kernel that holds nothing else and leaves a compute unit its LDS.  Between the two other
+// kernels of a pass: [4096, 14336] and [4096, 4096] bf16 80.6 us, in the general kernel 81.5.
+template <typename T, int NS>
+DEV void quantize_cols_two(const Seg &s, const KCall &p, int blk, int tid, float *part, float *scale)
+{
+    constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, G = 2, K = 64 / G, RB = G * EPV;
     constexpr int WAVES = TFTQ_QC_WG / 64, STEP = 4 * K * WAVES;  // columns per step
     constexpr int RPD = 4 / ESZ;                                  // rows per dword of a column
     const int per_slot = (s.slice_rows + RB - 1) / RB;
@@ -762,36 +957,32 @@ DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, float *pa
     }
 }
 
-// Steps that stay in registers: 12 for lists with rows of more than 4096 columns (250 registers, two
-// wavefronts per SIMD; 14 spill), else 4 (114 registers, four).
-constexpr int QC_MOST = 12;
-constexpr int QC_STEP = 4 * (64 / TFTQ_QC_GROUPS) * (TFTQ_QC_WG / 64);
-template <typename T, int NSMAX, typename A>
-DEV void quantize_cols_workgroup(const A &args)
+template <typename T, typename A>
+DEV void quantize_cols_two_workgroup(const A &args)
 {
-    __shared__ float part[4 * TFTQ_QC_WG / 64 * TFTQ_QC_GROUPS * Elem<T>::EPV];
-    __shared__ float scale[TFTQ_QC_GROUPS * Elem<T>::EPV];
+    __shared__ float part[4 * TFTQ_QC_WG / 64 * 2 * Elem<T>::EPV];
+    __shared__ float scale[2 * Elem<T>::EPV];
     Seg s;
     KCall p;
     int blk;
     if (!locate<ST_Q>(args, p, s, blk)) return;
     const int tid = threadIdx.x;
-    const int steps = (s.n + QC_STEP - 1) / QC_STEP;  // same for the whole workgroup
-    if (steps <= 1) quantize_cols<T, 1>(s, p, blk, tid, part, scale);
-    else if (steps <= 2) quantize_cols<T, 2>(s, p, blk, tid, part, scale);
-    else if (NSMAX == 4 || steps <= 4) quantize_cols<T, 4>(s, p, blk, tid, part, scale);
-    else if (steps <= 8) quantize_cols<T, NSMAX == 4 ? 4 : 8>(s, p, blk, tid, part, scale);
-    else quantize_cols<T, NSMAX>(s, p, blk, tid, part, scale);
+    const int steps = tftq_qc_steps(s.n, 1);  // same for the whole workgroup
+    if (steps <= 1) quantize_cols_two<T, 1>(s, p, blk, tid, part, scale);
+    else if (steps <= 2) quantize_cols_two<T, 2>(s, p, blk, tid, part, scale);
+    else if (steps <= 4) quantize_cols_two<T, 4>(s, p, blk, tid, part, scale);
+    else if (steps <= 8) quantize_cols_two<T, 8>(s, p, blk, tid, part, scale);
+    else quantize_cols_two<T, QC_MOST>(s, p, blk, tid, part, scale);
 }
-template <typename T, typename A, int NSMAX>
-__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols(const A args)
+template <typename T, typename A>
+__global__ __launch_bounds__(TFTQ_QC_WG, 2) void k_quantize_cols_two(const A args)
 {
-    quantize_cols_workgroup<T, NSMAX>(args);
+    quantize_cols_two_workgroup<T>(args);
 }
-template <typename T, int NSMAX>
-__global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols_one(TFTQ_ONE_PARAMS)
+template <typename T>
+__global__ __launch_bounds__(TFTQ_QC_WG, 2) void k_quantize_cols_two_one(TFTQ_ONE_PARAMS)
 {
-    quantize_cols_workgroup<T, NSMAX>(one_of(TFTQ_ONE));
+    quantize_cols_two_workgroup<T>(one_of(TFTQ_ONE));
 }
 
 template <typename T>
@@ -799,11 +990,11 @@ static int launch_qc(const tftq_plan *plan, const KArgs &ka, hipStream_t st)
 {
     return with_args(ka, [&](const auto &args) {
         typedef typename std::decay<decltype(args)>::type A;
-        const bool most = plan->cols_most > 4 * QC_STEP;
+        const bool most = plan->cols_most > 4, two = most && plan->cols_two;
         if constexpr (std::is_same<A, KOne>::value)
-            return launch_kernel(most ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
+            return launch_kernel(two ? k_quantize_cols_two_one<T> : most ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
         else
-            return launch_kernel(most ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
+            return launch_kernel(two ? k_quantize_cols_two<T, A> : most ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
     });
 }
 
