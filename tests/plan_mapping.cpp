@@ -273,6 +273,13 @@ int main()
         check_kinds(1000, 64, 256, TFTQ_BF16, 64, false, false, true) || check_kinds(1, 64, 64, TFTQ_BF16, 8, true, false, false) ||
         check_kinds(1, 256, 256, TFTQ_BF16, 8, false, false, false) || check_kinds(512, 16, 1024, TFTQ_F32, 64, true, false, true))
         return 1;
+    // widths up to the widest that a layout accepts: the blocks and tiles, whose last one is counted past
+    // the row's end, stay away from it
+    for (int dtype = 0; dtype < 3; dtype++)
+        for (const int64_t below : {8, 9, 63, 254, 255, 256, 511, 847, 1022, 1023, 1024, 2047, 4096})
+            if (check_kinds(1, 16 / (dtype == TFTQ_F32 ? 4 : 2), INT32_MAX - below, dtype, 1, false, false, false) ||
+                check_kinds(20, 64, INT32_MAX - below, dtype, 3, true, false, false))
+                return 1;
     // hand-picked lists: the Llama-3-8B layer bucket, empty tensors, one huge and many tiny
     const int64_t llama[] = {4096, 4096, 1024, 4096, 1024, 4096, 4096, 4096, 14336, 4096,
                              14336, 4096, 4096, 14336, 4096, 1, 4096, 1};

@@ -234,7 +234,8 @@ static Cost cost_of(const Seg &s, uint8_t kind, int st, int esz, int ws)
 static bool stored_by_columns(const Seg &s, int st, int esz)
 {
     // (fp32 rows of up to 32 columns stay with their teams in quantize.)
-    return s.row_stride == 1 && s.m >= 16 / esz && s.m < INT32_MAX - 4096 &&  // the blocks round up
+    constexpr int MOST = INT32_MAX - 4096;  // the blocks and tiles round rows and columns up
+    return s.row_stride == 1 && s.m >= 16 / esz && s.m < MOST && s.n < MOST &&
            (s.kind[st] == K_GEN8 || s.kind[st] == K_GEN64) && (st != ST_Q || esz == 2 || s.n > 32);
 }
 
