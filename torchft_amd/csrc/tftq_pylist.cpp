@@ -291,19 +291,29 @@ bool packed_buffer(PyObject *o, int64_t device, int64_t bytes, void **address)
     return true;
 }
 
+// Leaves the interpreter to other threads for the lifetime of the object, exceptions included.
+struct WithoutInterpreter {
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutInterpreter() { PyEval_RestoreThread(state); }
+};
+
 PyObject *launch_quantize(const Plan &plan, const void *const *tensors, int64_t device)
 {
     void *stream = nullptr;
     if (!current_stream(device, &stream)) Py_RETURN_NONE;
     try {
-        at::Tensor out = at::empty({plan.output_size}, at::TensorOptions(at::kByte).device(c10::Device(c10::kCUDA, static_cast<c10::DeviceIndex>(device))));
-        void *packed = out.data_ptr();
+        at::Tensor out;
         int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = library.quantize(plan.address, tensors, nullptr, nullptr, packed, plan.output_size, static_cast<int>(device), stream);
-        Py_END_ALLOW_THREADS
+        {
+            // The allocation too: it may have to wait for work on the GPU, and what ends that wait (the
+            // abort of a collective whose peer is gone, say) may be another thread's to do.
+            WithoutInterpreter others_run;
+            out = at::empty({plan.output_size}, at::TensorOptions(at::kByte).device(c10::Device(c10::kCUDA, static_cast<c10::DeviceIndex>(device))));
+            rc = library.quantize(plan.address, tensors, nullptr, nullptr, out.data_ptr(), plan.output_size, static_cast<int>(device), stream);
+        }
         return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
     } catch (...) {  // out of memory, say: Python says so
+        PyErr_Clear();
         Py_RETURN_NONE;
     }
 }
