@@ -264,6 +264,34 @@ int main()
             return 1;
         }
     }
+    // reduce's teams: what the whole list has to do decides, not the rows of one tensor.  Lists of `count`
+    // tensors of `rows` rows per slot behind `other` of 4096 columns
+    const struct { int count, rows, n, ws, other; uint8_t kind; } teams[] = {
+        {1, 256, 2048, 8, 0, K_GEN256}, {1, 512, 2048, 8, 0, K_GEN64}, {2, 256, 2048, 8, 0, K_GEN64}, {44, 256, 2048, 8, 0, K_GEN64},
+        {1, 256, 2048, 8, 128, K_GEN256}, {1, 256, 2048, 8, 129, K_GEN64}, {1, 511, 2048, 16, 0, K_GEN256}, {8, 511, 2048, 16, 0, K_GEN64},
+        {1, 256, 1536, 64, 0, K_GEN256}, {3, 256, 1536, 64, 0, K_GEN64}, {44, 256, 2048, 4, 0, K_GEN64},
+        {1, 8191, 640, 8, 0, K_GEN64}, {4, 1024, 640, 8, 0, K_GEN64}, {8, 1024, 640, 8, 0, K_GEN16}, {5, 1024, 640, 5, 0, K_GEN16}, {4, 1024, 640, 5, 0, K_GEN64}, {24, 512, 640, 4, 0, K_GEN16}, {24, 511, 640, 4, 0, K_GEN64},
+        {24, 1024, 704, 8, 0, K_GEN16}, {24, 1024, 705, 8, 0, K_GEN64}, {24, 1024, 768, 7, 0, K_GEN16},
+        {1, 698, 2560, 8, 0, K_GEN256}, {24, 698, 2560, 8, 0, K_GEN64}, {24, 511, 2560, 8, 0, K_GEN256}, {2, 640, 3000, 16, 0, K_GEN64}};
+    for (const auto &c : teams) {
+        std::vector<int64_t> shapes, strides;
+        if (c.other) {
+            shapes = {(int64_t)c.other * c.ws, 4096};
+            strides = {4096, 1};
+        }
+        for (int i = 0; i < c.count; i++) {
+            shapes.insert(shapes.end(), {(int64_t)c.rows * c.ws, c.n});
+            strides.insert(strides.end(), {c.n, 1});
+        }
+        tftq_plan *p = nullptr;
+        if (tftq_plan_create(TFTQ_BF16, (int)shapes.size() / 2, shapes.data(), strides.data(), c.ws, &p)) return 1;
+        const int got = p->segs.back().kind[ST_R];
+        tftq_plan_destroy(p);
+        if (got != c.kind) {
+            printf("%d x %d rows of %d columns in each of %d slots behind %d: kind %d, not %d\n", c.count, c.rows, c.n, c.ws, c.other, got, c.kind);
+            return 1;
+        }
+    }
     // which transposed tensors are worth blocks of columns: the faster side of measured pairs
     if (check_kinds(1, 4096, 14336, TFTQ_BF16, 8, false, true, true) || check_kinds(1, 1024, 4096, TFTQ_BF16, 8, false, true, true) ||
         check_kinds(1, 256, 8192, TFTQ_BF16, 16, true, true, true) || check_kinds(1, 4096, 4096, TFTQ_F32, 64, true, true, true) ||

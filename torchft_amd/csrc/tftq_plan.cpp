@@ -125,7 +125,8 @@ static uint8_t pick_d_kind(const Seg &s, int esz)
     return K_VEC256;
 }
 
-static uint8_t pick_reduce_kind(const Seg &s, int ws)
+// slot_size: bytes of the list's packed rows in a slot.
+static uint8_t pick_reduce_kind(const Seg &s, int ws, int64_t slot_size)
 {
     // one or two 16-byte vectors of codes per lane and peer, four for the longest rows
     const int ndw = s.row_bytes / 4 - 1;
@@ -157,22 +158,28 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws)
     // done sooner with more lanes per row; 10 000 tensors of up to 4096 elements: 65.0 us
     // with the smaller teams, 62.8 us without.)
     // In groups of more peers it takes more rows to keep the machine busy, as a row lives longer, the
-    // more so the fewer loads its lanes have in flight: packed rows of 700 columns, 3 peers, 1986 rows 4.7
-    // (16 lanes) against 5.5 us (64), 4 peers, 1490 rows 5.9 against 5.3, 8 peers, 2979 rows 8.7 against 6.4, 16
-    // peers 13.9 against 10.5, from 5 peers on even at 4800 to 6000 rows; of 2560 and 3000 columns, 8 peers, 698 rows
-    // 8.9 (64 lanes) against 6.9 us (256), 16 peers, 699 rows 13.8 against 10.6, 1818 rows 18.0 against 19.5.
+    // more so the fewer loads its lanes have in flight.  What counts is the whole list: its tensors run
+    // side by side, and it makes no difference whether it has 2048 rows in one tensor or in 32 (us, one
+    // tensor / 2 to 8 of 1024 or 512 rows).  128 to 192 dwords, 16 lanes against 64: packed rows of 640 columns, 4
+    // peers, 2048 rows 5.5, 5.0 / 6.0, 5.6, 4096 rows 5.7, 6.1 / 6.0, 6.4; 8 peers, 4096 rows 8.6, 6.9 / 8.9, 7.4, 8192 rows
+    // in 8 tensors 11.4, 11.5; 16 peers 13.5, 11.5 / 14.1, 12.0 and 19.3, 20.1.  From 8 peers on rows of more than 176
+    // dwords never win with 16: 768 columns, 60000 rows in 100 tensors 71.9, 67.4, one tensor of 40000 51.8, 46.9; with 5
+    // peers 640 columns at 4096 and 8192 rows 6.4, 6.6 and 8.4, 11.1.  513
+    // to 768 dwords, 64 lanes against 256: 2560 columns, 8 peers, 1024 rows 8.5, 6.9 / 9.0, 7.5, 2048 rows 10.4, 11.0 /
+    // 11.1, 11.5, 16752 rows in 24 tensors 62.1, 69.9; 16 peers, 1024 rows 13.5, 11.6, 2048 rows 16.8, 19.4.
     // For the same reason rows of 257 to 512 dwords, two vectors per lane in a wavefront, go to a whole
-    // workgroup: 2048 columns, 8 peers, 256 rows 5.3 -> 4.4 us (1022 rows 6.3 -> 7.7), 16 peers, 511 rows 10.9
-    // -> 8.1, 32 peers, 256 rows 18.3 -> 8.5, 64 peers, 128 rows 33.6 -> 13.3; not in groups of up to 4.
-    const int rows = s.slice_rows;
-    const bool many = rows >= 512;
+    // workgroup: 2048 columns, 8 peers, 256 rows 5.0 -> 4.0 us, 512 in 8 tensors 5.7 -> 5.6, 1024 5.9 -> 7.4, 11264
+    // in 44 35.3 -> 48.5; 16 peers, 256 rows 10.4 -> 5.4, 512 in 4 tensors 11.0 -> 7.8, 1024 11.2 -> 11.2, 4096 in 16 26.4 ->
+    // 33.7; 64 peers, 256 rows 32.4 -> 12.2, 1024 36.1 -> 35.7, 2048 49.0 -> 66.0; not in groups of up to 4.
+    const int64_t list_rows = slot_size / s.row_bytes;  // rows of this length that the whole list is worth
+    const bool many = s.slice_rows >= 512;
     if (ndw <= 128) return K_GEN32;
-    if (ndw <= 192 && ws <= 16 && rows >= (ws <= 3 ? 512 : ws == 4 ? 2048 : 4096)) return K_GEN16;
+    if (ndw <= (ws < 8 ? 192 : 176) && ws <= 16 && many && list_rows >= (ws <= 3 ? 512 : ws == 4 ? 2048 : ws < 8 ? 5120 : 8192)) return K_GEN16;
     if (ndw <= 256) return K_GEN64;
-    if (ndw <= 512 && ws >= 5 && rows < (ws > 12 ? 768 : 512)) return K_GEN256;
+    if (ndw <= 512 && ws >= 5 && list_rows < (ws > 12 ? 768 : 512)) return K_GEN256;
     if (ndw <= 384 && ws <= 32 && many) return K_GEN32;
     if (ndw <= 512) return K_GEN64;
-    if (ndw <= 768 && ws <= 64 && rows >= (ws <= 5 ? 512 : ws <= 8 ? 1024 : 1280)) return K_GEN64;
+    if (ndw <= 768 && ws <= 64 && many && list_rows >= (ws <= 5 ? 512 : ws <= 8 ? 1024 : 1280)) return K_GEN64;
     return K_GEN256;
 }
 
@@ -594,7 +601,7 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
 
         s.kind[ST_Q] = pick_io_kind(s, p->esz);
         s.kind[ST_D] = pick_d_kind(s, p->esz);
-        s.kind[ST_R] = pick_reduce_kind(s, p->ws);
+        s.kind[ST_R] = pick_reduce_kind(s, p->ws, p->slot_size);
         s.side = (uint8_t)tftq_reduce_rows_side(s.kind[ST_R], s.row_bytes / 4 - 1, s.slice_rows, p->ws);
     }
     pick_few_kinds(p);
