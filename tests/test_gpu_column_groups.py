@@ -29,3 +29,27 @@ def test_groups_of_rows(q, oracle, dtype, ws, together):  # noqa: F811
         for a, b in zip(gpu, part):
             a.copy_(b)
         same_bytes(q.fused_quantize_into_fp8(gpu, ws), packed, f"{[tuple(v.shape) for v in part]}")
+
+
+# slots and lists of 2 groups: launches of at most and of more than 48 blocks of rows of 5 to 8 steps and 192 of
+# rows of 1 to 4, alone and in lists, each number of steps at both ends and rows of more than 12
+FEW = [(1, [(768, 7001)]), (1, [(784, 7001)]), (1, [(3072, 2049)]), (1, [(3088, 2049)]), (3, [(130, 1024)]),
+       (3, [(133, 1025), (65, 2049), (40, 2048)]), (2, [(100, 4096), (31, 17), (64, 5000)]), (8, [(384, 8192)]),
+       (8, [(383, 8192), (70, 4097)]), (1, [(784, 8192), (16, 14000)]), (2, [(700, 8193), (33, 900)])]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ws, shapes", FEW)
+def test_few_blocks(q, oracle, dtype, ws, shapes):  # noqa: F811
+    """Rows straight from the registers: every element is in the maximum whatever the number of steps (each
+    row's largest is in its last column)."""
+    g = torch.Generator().manual_seed(len(shapes))
+    views = [transposed(m, n, i % 3, i % 5, dtype, g)[0] for i, (m, n) in enumerate(shapes)]
+    for v in views:
+        v[:, -1] = 3.0 + torch.arange(v.shape[0]).to(dtype) / 1024
+    packed = oracle.fused_quantize_into_fp8([v.clone() for v in views], ws, nthreads=NT)
+    gpu = [torch.empty(v.stride(1) * v.shape[1] + 8, dtype=dtype, device="cuda")[v.storage_offset():]
+           .as_strided(v.shape, v.stride(), v.storage_offset()) for v in views]
+    for a, b in zip(gpu, views):
+        a.copy_(b)
+    same_bytes(q.fused_quantize_into_fp8(gpu, ws), packed, f"{shapes}")

@@ -642,7 +642,7 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize_one(TFTQ_ONE
 // maxima go through LDS, and the packed rows where a block's fit (they are one span of bytes:
 // copy_out_span).  A block of G such groups of rows stays in the registers of a workgroup of 512
 // lanes, up to NS steps of 2048 / G columns, so that the tensor is read once; what a row has beyond
-// that, in 2 groups only, is read twice.  Bound by memory where 8 or more groups make whole lines of
+// that is read twice (in 2 groups; more groups hold their rows whole).  Bound by memory where 8 or more groups make whole lines of
 // what a block reads; with 2 groups it uses 32 bytes of a line and the L1's requests in flight are the
 // limit.  bf16, 8 slots, 2 groups and dwords stored from the registers -> with the groups that
 // pick_groups takes and the stage: [285326, 147] 101 -> 26 us (4.8 TB/s), [1310720, 32] 447 -> 29, [41943, 1000]
@@ -651,7 +651,11 @@ __global__ __launch_bounds__(TFTQ_WG, WIDE ? 4 : 1) void k_quantize_one(TFTQ_ONE
 // 256 lanes 89 (half of the row read twice), of 1024 lanes 72, streaming loads 77 (neighbouring blocks
 // share lines); a launch for the maxima and one for tiles of 64 rows 82 us.  Where the blocks lose against
 // teams of lanes (few rows per slot) the planner leaves them out: pick_column_kinds.
-template <typename T, int G, int NS, int STAGE>
+// REST: with the first pass over what a row has beyond NS steps, whether a row has that or not.  It changes the
+// order of the other loads: with it the compiler computes maxima between them, with some 8 in flight, without
+// it all loads of up to 8 steps come first.  The former suits blocks that have a compute unit's L1 to
+// themselves for long enough, the latter a machine full of them (see k_quantize_cols_two).
+template <typename T, int G, int NS, int STAGE, bool REST = true>
 DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage, float *scale)
 {
     constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, K = 64 / G, RB = G * EPV;
@@ -705,11 +709,13 @@ DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, uint8_t *
     for (int t = 0; t < NS; t++) load(v[t], t * STEP);
 #pragma unroll
     for (int t = 0; t < NS; t++) maxima(v[t]);
+    if constexpr (REST) {
 #pragma nounroll
-    for (int base = NS * STEP; base < s.n; base += STEP) {  // first pass over the rest
-        u32x4 x[4];
-        load(x, base);
-        maxima(x);
+        for (int base = NS * STEP; base < s.n; base += STEP) {  // first pass over the rest
+            u32x4 x[4];
+            load(x, base);
+            maxima(x);
+        }
     }
 #pragma unroll
     for (int i = 0; i < EPV; i++) {  // over the lanes of the same group in a row of 16
@@ -788,8 +794,9 @@ DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, uint8_t *
 // wavefronts per SIMD; 14 spill), else 4 (115 registers, four).  More than 4 groups take no more than 4
 // steps (pick_groups).
 constexpr int QC_MOST = 12;
-// The stage: all packed rows of a block of up to 4 steps, or 8 (fp32, 4 groups: 12).  fp32 in 2 groups
-// does without: [41943, 1000] 75 us straight from the registers and 77 through the stage.
+// The stage: all packed rows of a block of up to 4 steps, or 8 (fp32, 4 groups: 12).  2 groups do without in
+// fp32 ([41943, 1000] 75 us straight from the registers and 77 through the stage) and beside rows of more than 4
+// steps (bf16 [4096, 8192], [8192, 4096] and [4096, 1024] in one list, 4 slots, 73.6 us through the stage and 70.3).
 template <typename T, int NSMAX>
 struct ColsStage {
     static constexpr int VECTORS = NSMAX == 4 ? 4 : Elem<T>::ESZ == 4 ? NSMAX : 8;
@@ -800,7 +807,7 @@ template <typename T, int G, int NSMAX>
 DEV void quantize_cols_steps(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage, float *scale)
 {
     constexpr int STAGE = ColsStage<T, NSMAX>::BYTES;
-    constexpr bool DIRECT = Elem<T>::ESZ == 4 && G == 2;
+    constexpr bool DIRECT = G == 2 && (Elem<T>::ESZ == 4 || NSMAX > 4);
     const int steps = tftq_qc_steps(s.n, __builtin_ctz(G));  // same for the whole workgroup
     constexpr int SHORT = DIRECT ? QC_LEAST_STAGE : STAGE;
     if (steps <= 1) quantize_cols<T, G, 1, SHORT>(s, p, blk, tid, stage, scale);
@@ -808,8 +815,7 @@ DEV void quantize_cols_steps(const Seg &s, const KCall &p, int blk, int tid, uin
     else if (NSMAX == 4 || steps <= 4) quantize_cols<T, G, 4, SHORT>(s, p, blk, tid, stage, scale);
     else if constexpr (NSMAX > 4) {
         if (steps <= 8) quantize_cols<T, G, 8, SHORT>(s, p, blk, tid, stage, scale);
-        else if (Elem<T>::ESZ == 4 && G == 4) quantize_cols<T, G, NSMAX, STAGE>(s, p, blk, tid, stage, scale);
-        else quantize_cols<T, G, NSMAX, QC_LEAST_STAGE>(s, p, blk, tid, stage, scale);
+        else quantize_cols<T, G, NSMAX, Elem<T>::ESZ == 4 && G == 4 ? STAGE : QC_LEAST_STAGE>(s, p, blk, tid, stage, scale);
     }
 }
 template <typename T, int NSMAX, typename A>
@@ -841,126 +847,21 @@ __global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols
     quantize_cols_workgroup<T, NSMAX>(one_of(TFTQ_ONE));
 }
 
-// Lists whose tensors all have 2 groups and some of them more than 4 steps: the same straight from the
-// registers, in a kernel that holds nothing else and leaves a compute unit its LDS.  Between the two other
-// kernels of a pass: [4096, 14336] and [4096, 4096] bf16 80.6 us, in the general kernel 81.5.
-template <typename T, int NS>
-DEV void quantize_cols_two(const Seg &s, const KCall &p, int blk, int tid, float *part, float *scale)
+// Lists whose tensors all have 2 groups: the same straight from the registers, in kernels that hold
+// nothing else and leave a compute unit its LDS.  us with the rest's first pass in rows of up to 8 steps / without
+// it (kernels of up to 12 steps, 8 slots):
+//   bf16 16 blocks of 4500 / 7001 columns 8.1, 9.8 / 9.1, 10.9; 24 of 7500 16.5 / 17.1; 48 18.1 / 18.3; 64 20.0 / 19.7;
+//     512 of 8192 76.6 / 70.7; and in the same kernel rows of 9 to 14 steps, [8192, 9000] 88.5 / 77.1, [4096, 14336]
+//     67.0 / 62.6, alone, and 70.5 / 68.2 beside [4096, 4096], whose loads the compiler orders differently too;
+//   fp32 [1024, 4500] 12.4 / 10.8, [3200, 8000] 47.8 / 40.5, [4999, 8191] 76.9 / 62.6.
+// FEW, 16 bits, up to 8 steps: with it, also for rows of up to 4 steps, which a launch of few blocks does sooner
+// straight from the registers than through the stage: [128, 700] 4.0 -> 3.7, [384, 2000] 5.5 -> 4.8, [2048, 4096] (128
+// blocks) 12.5 -> 11.3, 192 blocks 15.1 -> 14.1, 256 13.4 -> 13.7.
+template <typename T, bool FEW, typename A>
+DEV void quantize_cols_two(const A &args)
 {
-    constexpr int EPV = Elem<T>::EPV, ESZ = Elem<T>::ESZ, G = 2, K = 64 / G, RB = G * EPV;
-    constexpr int WAVES = TFTQ_QC_WG / 64, STEP = 4 * K * WAVES;  // columns per step
-    constexpr int RPD = 4 / ESZ;                                  // rows per dword of a column
-    const int per_slot = (s.slice_rows + RB - 1) / RB;
-    const int slot = blk / per_slot;
-    const int j0 = (blk - slot * per_slot) * RB;
-    const int srow = slot * s.slice_rows;  // the slot's first row
-    const int real = min(max(s.m - srow, 0), s.slice_rows);
-    GLOBAL uint8_t *g0 = as_global<uint8_t>(p.packed + (int64_t)slot * p.slot_size + s.slot_off + (int64_t)j0 * s.row_bytes);
-    {   // padding rows: zero (:93-95 on a zero-filled buffer)
-        const int z0 = max(real - j0, 0), z1 = min(RB, s.slice_rows - j0);
-        for (int z = z0; z < z1; z++)
-            for (int d = tid; d < (s.row_bytes >> 2); d += TFTQ_QC_WG) ((GLOBAL u32 *)(g0 + (int64_t)z * s.row_bytes))[d] = 0;
-    }
-    if (j0 >= real) return;  // the whole workgroup
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
-    const int g = l & (G - 1), k = l / G;
-    const int ndw = (s.row_bytes >> 2) - 1;
-    // the lane's rows; the last group of the tensor is moved back to end with it (its rows are
-    // another lane's too: both write the same bytes)
-    const int first = min(srow + j0 + g * EPV, s.m - EPV);
-    const int jf = first - srow - j0, jstop = min(RB, real - j0);  // rows jf + i in [0, jstop) are written
-    const uint64_t col0 = s.ptr + (uint64_t)((int64_t)first * ESZ);
-    const int64_t cs = s.col_stride * ESZ;
-    const int c0 = 4 * (wave * K + k);
-    auto load = [&](u32x4 (&v)[4], int base) {
-#pragma unroll
-        for (int e = 0; e < 4; e++)  // columns past the last one re-read it
-            v[e] = *as_global<const u32x4_a2>(col0 + (uint64_t)((int64_t)min(base + c0 + e, s.n - 1) * cs));
-    };
-    float amax[EPV];
-#pragma unroll
-    for (int i = 0; i < EPV; i++) amax[i] = 0.0f;
-    auto maxima = [&](const u32x4 (&v)[4]) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            float f[EPV];
-            Elem<T>::unpack(v[e], f);
-#pragma unroll
-            for (int i = 0; i < EPV; i++) amax[i] = fmaxf(amax[i], __builtin_fabsf(f[i]));
-        }
-    };
-    u32x4 v[NS][4];
-#pragma unroll
-    for (int t = 0; t < NS; t++) load(v[t], t * STEP);
-#pragma unroll
-    for (int t = 0; t < NS; t++) maxima(v[t]);
-#pragma nounroll
-    for (int base = NS * STEP; base < s.n; base += STEP) {  // first pass over the rest
-        u32x4 x[4];
-        load(x, base);
-        maxima(x);
-    }
-#pragma unroll
-    for (int i = 0; i < EPV; i++) {  // over the lanes of the same parity in a row of 16
-        amax[i] = fmaxf(amax[i], dpp_mov<0x128>(amax[i]));  // row_ror:8
-        amax[i] = fmaxf(amax[i], dpp_mov<0x124>(amax[i]));  // row_ror:4
-        amax[i] = fmaxf(amax[i], dpp_mov<0x122>(amax[i]));  // row_ror:2
-        if ((l & 15) < G) part[(wave * 4 + (l >> 4)) * RB + g * EPV + i] = amax[i];
-    }
-    static_assert(G == 2, "the rotations above");
-    __syncthreads();
-    if (tid < RB) {
-        float a = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4 * WAVES; w++) a = fmaxf(a, part[w * RB + tid]);
-        const float sc = calc_scale(a);
-        scale[tid] = sc;
-        const int j = min(srow + j0 + tid / EPV * EPV, s.m - EPV) - srow - j0 + tid % EPV;
-        if (j >= 0 && j < jstop) *(GLOBAL u32 *)(g0 + (int64_t)j * s.row_bytes) = as_u(sc);
-    }
-    __syncthreads();
-    float sc[EPV];
-#pragma unroll
-    for (int i = 0; i < EPV; i++) sc[i] = scale[g * EPV + i];
-    GLOBAL uint8_t *out = g0 + (int64_t)jf * s.row_bytes + 4;
-    auto store = [&](const u32x4 (&v)[4], int base) {
-        const int d = (base + c0) >> 2;  // the lane's dword of the payload
-        if (d >= ndw) return;
-        const int over = 4 * d + 4 - s.n;  // columns of the dword past the last one
-        const u32 mask = over > 0 ? 0xFFFFFFFFu >> (8 * over) : 0xFFFFFFFFu;
-#pragma unroll
-        for (int w = 0; w < 4; w++) {  // dword w of the four vectors: rows RPD * w ...
-            float f[4][RPD];
-#pragma unroll
-            for (int e = 0; e < 4; e++) unpack_dword<T>(v[e][w], f[e]);
-#pragma unroll
-            for (int h = 0; h < RPD; h++) {
-                const int i = RPD * w + h;
-                const u32 o = pack_fp8x4(f[0][h] * sc[i], f[1][h] * sc[i], f[2][h] * sc[i], f[3][h] * sc[i]) & mask;
-                // plain stores: a packed row starts anywhere in its line, the L2 puts the runs together
-                if (jf + i >= 0 && jf + i < jstop) ((GLOBAL u32 *)(out + (int64_t)i * s.row_bytes))[d] = o;
-            }
-        }
-    };
-#pragma unroll
-    for (int t = 0; t < NS; t++) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) asm volatile("" : "+v"(v[t][e].x), "+v"(v[t][e].y), "+v"(v[t][e].z), "+v"(v[t][e].w));
-    }
-#pragma unroll
-    for (int t = 0; t < NS; t++) store(v[t], t * STEP);
-#pragma nounroll
-    for (int base = NS * STEP; base < s.n; base += STEP) {  // second pass over the rest
-        u32x4 x[4];
-        load(x, base);
-        store(x, base);
-    }
-}
-
-template <typename T, typename A>
-DEV void quantize_cols_two_workgroup(const A &args)
-{
-    __shared__ float part[4 * TFTQ_QC_WG / 64 * 2 * Elem<T>::EPV];
+    constexpr int STAGE = 4 * TFTQ_QC_WG / 64 * 2 * Elem<T>::EPV * 4;  // for the maxima alone
+    __shared__ __align__(16) uint8_t stage[STAGE];
     __shared__ float scale[2 * Elem<T>::EPV];
     Seg s;
     KCall p;
@@ -968,21 +869,21 @@ DEV void quantize_cols_two_workgroup(const A &args)
     if (!locate<ST_Q>(args, p, s, blk)) return;
     const int tid = threadIdx.x;
     const int steps = tftq_qc_steps(s.n, 1);  // same for the whole workgroup
-    if (steps <= 1) quantize_cols_two<T, 1>(s, p, blk, tid, part, scale);
-    else if (steps <= 2) quantize_cols_two<T, 2>(s, p, blk, tid, part, scale);
-    else if (steps <= 4) quantize_cols_two<T, 4>(s, p, blk, tid, part, scale);
-    else if (steps <= 8) quantize_cols_two<T, 8>(s, p, blk, tid, part, scale);
-    else quantize_cols_two<T, QC_MOST>(s, p, blk, tid, part, scale);
+    if (steps <= 1) quantize_cols<T, 2, 1, STAGE, FEW>(s, p, blk, tid, stage, scale);
+    else if (steps <= 2) quantize_cols<T, 2, 2, STAGE, FEW>(s, p, blk, tid, stage, scale);
+    else if (steps <= 4) quantize_cols<T, 2, 4, STAGE, FEW>(s, p, blk, tid, stage, scale);
+    else if (FEW || steps <= 8) quantize_cols<T, 2, 8, STAGE, FEW>(s, p, blk, tid, stage, scale);
+    else if constexpr (!FEW) quantize_cols<T, 2, QC_MOST, STAGE>(s, p, blk, tid, stage, scale);
 }
-template <typename T, typename A>
+template <typename T, typename A, bool FEW>
 __global__ __launch_bounds__(TFTQ_QC_WG, 2) void k_quantize_cols_two(const A args)
 {
-    quantize_cols_two_workgroup<T>(args);
+    quantize_cols_two<T, FEW>(args);
 }
-template <typename T>
+template <typename T, bool FEW>
 __global__ __launch_bounds__(TFTQ_QC_WG, 2) void k_quantize_cols_two_one(TFTQ_ONE_PARAMS)
 {
-    quantize_cols_two_workgroup<T>(one_of(TFTQ_ONE));
+    quantize_cols_two<T, FEW>(one_of(TFTQ_ONE));
 }
 
 template <typename T>
@@ -991,10 +892,15 @@ static int launch_qc(const tftq_plan *plan, const KArgs &ka, hipStream_t st)
     return with_args(ka, [&](const auto &args) {
         typedef typename std::decay<decltype(args)>::type A;
         const bool most = plan->cols_most > 4, two = most && plan->cols_two;
+        constexpr bool HALF = Elem<T>::ESZ == 2;
+        // few blocks: the figures at k_quantize_cols_two
+        const bool few = HALF && plan->cols_two && plan->cols_most <= 8 && plan->nwg[ST_QC] <= (most ? 48 : 192);
         if constexpr (std::is_same<A, KOne>::value)
-            return launch_kernel(two ? k_quantize_cols_two_one<T> : most ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
+            return launch_kernel(few ? k_quantize_cols_two_one<T, HALF> : two ? k_quantize_cols_two_one<T, false>
+                                 : most ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
         else
-            return launch_kernel(two ? k_quantize_cols_two<T, A> : most ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
+            return launch_kernel(few ? k_quantize_cols_two<T, A, HALF> : two ? k_quantize_cols_two<T, A, false>
+                                 : most ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
     });
 }
 
