@@ -1571,6 +1571,10 @@ __global__ __launch_bounds__(TFTQ_WG, reduce_waves(FLAVOUR)) void k_reduce_one(T
 // The launch of a flavour; defined in tftq_reduce_<flavour>.hip.
 template <int FLAVOUR>
 __attribute__((visibility("hidden"))) int reduce_flavour(const KArgs &ka, bool gdiv, unsigned lds_bytes, hipStream_t st);
+template <> int reduce_flavour<R_ALL>(const KArgs &ka, bool gdiv, unsigned lds_bytes, hipStream_t st);
+template <> int reduce_flavour<R_WIDE>(const KArgs &ka, bool gdiv, unsigned lds_bytes, hipStream_t st);
+template <> int reduce_flavour<R_LONG>(const KArgs &ka, bool gdiv, unsigned lds_bytes, hipStream_t st);
+template <> int reduce_flavour<R_ONE>(const KArgs &ka, bool gdiv, unsigned lds_bytes, hipStream_t st);
 
 #define TFTQ_REDUCE_FLAVOUR(FLAVOUR)                                                                                   \
     template <>                                                                                                        \
