@@ -847,19 +847,21 @@ __global__ __launch_bounds__(TFTQ_QC_WG, NSMAX > 4 ? 2 : 4) void k_quantize_cols
     quantize_cols_workgroup<T, NSMAX>(one_of(TFTQ_ONE));
 }
 
-// Lists whose tensors all have 2 groups: the same straight from the registers, in kernels that hold
-// nothing else and leave a compute unit its LDS.  us with the rest's first pass in rows of up to 8 steps / without
+// Lists whose tensors all have 2 groups, rows of up to MOST steps: the same straight from the registers, in
+// kernels that hold nothing else and leave a compute unit its LDS.  us with the rest's first pass in rows of up to 8 steps / without
 // it (kernels of up to 12 steps, 8 slots):
 //   bf16 16 blocks of 4500 / 7001 columns 8.1, 9.8 / 9.1, 10.9; 24 of 7500 16.5 / 17.1; 48 18.1 / 18.3; 64 20.0 / 19.7;
 //     512 of 8192 76.6 / 70.7; and in the same kernel rows of 9 to 14 steps, [8192, 9000] 88.5 / 77.1, [4096, 14336]
 //     67.0 / 62.6, alone, and 70.5 / 68.2 beside [4096, 4096], whose loads the compiler orders differently too;
 //   fp32 [1024, 4500] 12.4 / 10.8, [3200, 8000] 47.8 / 40.5, [4999, 8191] 76.9 / 62.6.
-// FEW, 16 bits, up to 8 steps: with it, also for rows of up to 4 steps, which a launch of few blocks does sooner
-// straight from the registers than through the stage: [128, 700] 4.0 -> 3.7, [384, 2000] 5.5 -> 4.8, [2048, 4096] (128
-// blocks) 12.5 -> 11.3, 192 blocks 15.1 -> 14.1, 256 13.4 -> 13.7.
-template <typename T, bool FEW, typename A>
+// Few blocks in 16 bits, rows of up to 8 steps: with it; and those of up to 4 steps, in a kernel of two workgroups
+// per compute unit, which is done sooner than the one with the stage: us with / without the stage [256, 1000] 4.3 /
+// 3.7, [2048, 4096] (128 blocks) 12.4 / 11.5, [3072, 3300] 12.5 / 11.9, 256 blocks of 1000, 2000 and 4096 columns
+// 5.2, 8.7, 13.3 / 4.8, 8.7, 13.8, 400 of 2000 11.4 / 12.2.
+template <typename T, int MOST, typename A>
 DEV void quantize_cols_two(const A &args)
 {
+    constexpr bool FEW = MOST < QC_MOST;
     constexpr int STAGE = 4 * TFTQ_QC_WG / 64 * 2 * Elem<T>::EPV * 4;  // for the maxima alone
     __shared__ __align__(16) uint8_t stage[STAGE];
     __shared__ float scale[2 * Elem<T>::EPV];
@@ -871,19 +873,21 @@ DEV void quantize_cols_two(const A &args)
     const int steps = tftq_qc_steps(s.n, 1);  // same for the whole workgroup
     if (steps <= 1) quantize_cols<T, 2, 1, STAGE, FEW>(s, p, blk, tid, stage, scale);
     else if (steps <= 2) quantize_cols<T, 2, 2, STAGE, FEW>(s, p, blk, tid, stage, scale);
-    else if (steps <= 4) quantize_cols<T, 2, 4, STAGE, FEW>(s, p, blk, tid, stage, scale);
-    else if (FEW || steps <= 8) quantize_cols<T, 2, 8, STAGE, FEW>(s, p, blk, tid, stage, scale);
-    else if constexpr (!FEW) quantize_cols<T, 2, QC_MOST, STAGE>(s, p, blk, tid, stage, scale);
+    else if (MOST == 4 || steps <= 4) quantize_cols<T, 2, 4, STAGE, FEW>(s, p, blk, tid, stage, scale);
+    else if constexpr (MOST > 4) {
+        if (MOST == 8 || steps <= 8) quantize_cols<T, 2, 8, STAGE, FEW>(s, p, blk, tid, stage, scale);
+        else quantize_cols<T, 2, MOST, STAGE>(s, p, blk, tid, stage, scale);
+    }
 }
-template <typename T, typename A, bool FEW>
-__global__ __launch_bounds__(TFTQ_QC_WG, 2) void k_quantize_cols_two(const A args)
+template <typename T, typename A, int MOST>
+__global__ __launch_bounds__(TFTQ_QC_WG, MOST > 4 ? 2 : 4) void k_quantize_cols_two(const A args)
 {
-    quantize_cols_two<T, FEW>(args);
+    quantize_cols_two<T, MOST>(args);
 }
-template <typename T, bool FEW>
-__global__ __launch_bounds__(TFTQ_QC_WG, 2) void k_quantize_cols_two_one(TFTQ_ONE_PARAMS)
+template <typename T, int MOST>
+__global__ __launch_bounds__(TFTQ_QC_WG, MOST > 4 ? 2 : 4) void k_quantize_cols_two_one(TFTQ_ONE_PARAMS)
 {
-    quantize_cols_two<T, FEW>(one_of(TFTQ_ONE));
+    quantize_cols_two<T, MOST>(one_of(TFTQ_ONE));
 }
 
 template <typename T>
@@ -891,16 +895,20 @@ static int launch_qc(const tftq_plan *plan, const KArgs &ka, hipStream_t st)
 {
     return with_args(ka, [&](const auto &args) {
         typedef typename std::decay<decltype(args)>::type A;
-        const bool most = plan->cols_most > 4, two = most && plan->cols_two;
+        // kernels of 2 groups: for rows of up to QC_MOST steps, and for few blocks in 16 bits
+        // (the figures at k_quantize_cols_two)
         constexpr bool HALF = Elem<T>::ESZ == 2;
-        // few blocks: the figures at k_quantize_cols_two
-        const bool few = HALF && plan->cols_two && plan->cols_most <= 8 && plan->nwg[ST_QC] <= (most ? 48 : 192);
+        constexpr int FEW8 = HALF ? 8 : QC_MOST, FEW4 = HALF ? 4 : QC_MOST;
+        const int most = plan->cols_most, blocks = plan->nwg[ST_QC];
+        const bool two = plan->cols_two, few = HALF && two && blocks <= (most > 4 ? 48 : most > 2 ? 192 : 256) && most <= 8;
         if constexpr (std::is_same<A, KOne>::value)
-            return launch_kernel(few ? k_quantize_cols_two_one<T, HALF> : two ? k_quantize_cols_two_one<T, false>
-                                 : most ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
+            return launch_kernel(few && most <= 4 ? k_quantize_cols_two_one<T, FEW4> : few ? k_quantize_cols_two_one<T, FEW8>
+                                 : two && most > 4 ? k_quantize_cols_two_one<T, QC_MOST>
+                                 : most > 4 ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
         else
-            return launch_kernel(few ? k_quantize_cols_two<T, A, HALF> : two ? k_quantize_cols_two<T, A, false>
-                                 : most ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
+            return launch_kernel(few && most <= 4 ? k_quantize_cols_two<T, A, FEW4> : few ? k_quantize_cols_two<T, A, FEW8>
+                                 : two && most > 4 ? k_quantize_cols_two<T, A, QC_MOST>
+                                 : most > 4 ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
     });
 }
 
