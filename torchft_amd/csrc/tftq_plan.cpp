@@ -190,36 +190,47 @@ static uint8_t pick_reduce_kind(const Seg &s, int ws, int64_t slot_size)
 // columns, but cost the same however many rows and columns of them the tensor has (a block never
 // crosses a slot), so they lose on narrow tensors and where a slot has few rows of one.
 //
-// What either costs, in us: a kernel takes the longest of its workgroups' latencies, or BASE and the
-// work of all its tensors, whichever is more.  Fitted to kernels back to back in a graph, 2248 lists in
-// quantize and 562 in dequantize: one tensor and lists of up to 10000, 16 to 65536 rows, 17 to 16384
-// columns, 1 to 64 slots, both sizes of element.  On all but 33 of them the choice takes the faster
-// kernel or one within 5 % or 0.3 us of it.  Teams against blocks in quantize, bf16:
-// [4096, 14336] 267 against 41 us, [256, 8192] 41 against 12.3, [1024, 128] 7.0 against 4.4,
-// [100000, 32] 9.7 against 35, 10000 [32, 32] in 16 slots 26 against 644; teams against tiles in
-// dequantize: [4096, 14336] 290 against 28, [256, 256] 4.0 against 5.8, 10000 [32, 32] 18 against 22.
+// What either costs, in us: a kernel takes the longest of its workgroups' latencies, or its start and the
+// work of all its tensors, whichever is more.  Quantize was fitted to kernels back to back in a graph, 980
+// matrices alone, 16 to 600000 rows, 17 to 24000 columns, 1 to 32 slots, both sizes of element, each with the
+// teams and with every number of groups of rows that a block can have: what is chosen takes 0.6 % more than the
+// best of them in the mean, and in 41 cases more than 5 % and 0.2 us more.  Dequantize was fitted to 562
+// lists.  Teams against blocks in quantize, bf16: [4096, 14336] 267 against 41 us in a graph of one
+// matrix, [256, 8192] 41 against 12.3, [1024, 128] 7.0 against 4.4, 10000 [32, 32] in 16 slots 26 against 644;
+// teams against tiles in dequantize: [4096, 14336] 290 against 28, [256, 256] 4.0 against 5.8, 10000 [32, 32] 18
+// against 22.
 struct Cost {
     double latency, work;
+    double start = 3.5;
+    double alone() const { return std::max(latency, start + work); }
 };
-constexpr double COST_BASE = 3.5;
-constexpr double COST_HIDDEN = 4.2;  // of a latency, beside other tensors in the same launch
+constexpr double COST_HIDDEN_Q = 3.6, COST_HIDDEN_D = 4.2;  // of a latency, beside other tensors in the same launch
 // What a second launch of quantize, behind one for other tensors, saves of its own: [4096, 4096] by
 // rows and one transposed [64, 64], 9.6 us in one launch and 12.6 in two; [1024, 1024], 15.8 and 13.4.
-constexpr double COST_OVERLAP = 0.8;
+constexpr double COST_OVERLAP = 0.2;
 
 // Quantize's blocks of 2^lg groups of rows.  A block's time is a fixed part per step and the bytes it
-// moves at 6.2 TB/s, slower by SLOW where it uses a part of a line only and by more where two workgroups no
-// longer fit a compute unit (more than 4 steps); it counts padding lanes and rows as if they were real.
+// moves at 6.2 TB/s, slower by `slow`, as far as it uses a part of a line only, and by `wide`, where two
+// workgroups no longer fit a compute unit (more than 4 steps); it counts padding lanes and rows as if they
+// were real.
 static Cost cost_of_blocks(const Seg &s, int lg, int esz, int ws)
 {
-    static const double SLOW[2][6] = {{0, 1.3, 1.15, 1.05, 1.05, 1.05}, {0, 2.1, 1.45, 1.2, 1.05, 1.05}};  // 16 bits, fp32
-    const bool half = esz == 2;
-    const int rows = tftq_qc_rows(lg, esz), steps = tftq_qc_steps(s.n, lg);
+    static const struct {
+        double slow[6], wide[2], step, latency[2], per_step[2], per_column, per_column_past, start;
+    } FIT[2] = {  // [0]: 2 groups, [1]: more
+        {{0, 1.39, 1.13, 0.813, 0.656, 0.891}, {1.22, 1.5}, 5.03e-3, {3.01, 2.93}, {0.837, 1.02}, 7.79e-4, 3.68e-3, 2.77},   // 16 bits
+        {{0, 1.12, 0.962, 0.874, 0.859, 0.923}, {1.63, 1.63}, 3.43e-3, {2.52, 3.14}, {0.611, 0.515}, 3.85e-4, 3.86e-3, 2.69}};  // fp32
+    const auto &f = FIT[esz == 4];
+    const int rows = tftq_qc_rows(lg, esz), steps = tftq_qc_steps(s.n, lg), more = lg > 1;
     const int held = steps <= 2 ? steps : steps <= 4 ? 4 : steps <= 8 ? 8 : 12;
-    double bytes = (double)rows * s.n * (esz + 1) * SLOW[!half][lg] * (held > 4 ? half ? 1.4 : 1.1 : 1.0);
-    if (steps > 12) bytes *= 2.0 - 12.0 / steps;  // what is read twice
-    const double block = sqrt(4.5e-3 * held * 4.5e-3 * held + bytes / 6.2e6 * (bytes / 6.2e6));
-    return {half ? 2.9 + 1.1 * held + 0.0006 * s.n : 2.6 + 0.6 * held + 0.0011 * s.n, (double)ws * ((s.slice_rows + rows - 1) / rows) * block};
+    double bytes = (double)rows * s.n * (esz + 1) * f.slow[lg] * (held > 4 ? f.wide[more] : 1.0);
+    double latency = f.latency[more] + f.per_step[more] * held + f.per_column * s.n;
+    if (steps > 12) {  // what is read twice
+        bytes *= 2.0 - 12.0 / steps;
+        latency += f.per_column_past * (s.n - 12288);
+    }
+    const double block = hypot(f.step * held, bytes / 6.2e6);
+    return {latency, (double)ws * ((s.slice_rows + rows - 1) / rows) * block, f.start};
 }
 
 static Cost cost_of(const Seg &s, uint8_t kind, int st, int esz, int ws)
@@ -232,8 +243,9 @@ static Cost cost_of(const Seg &s, uint8_t kind, int st, int esz, int ws)
         return {4.3 + 0.006 * std::min(n, 256.0), tiles * 1.45e-3 + m * n * esz * 1.35e-7};
     }
     if (st == ST_Q)
-        return kind == K_GEN64 ? Cost{3.0 + 0.0045 * n, padded * n * (half ? 4.5e-6 : 6.0e-6)}
-                               : Cost{3.0 + (half ? 0.032 : 0.026) * n, padded * (n * 2.1e-6 + 1.2e-5)};
+        return kind == K_GEN64 ? half ? Cost{2.56 + 0.0052 * n, padded * n * 3.97e-6, 2.03} : Cost{2.41 + 0.00441 * n, padded * n * 5.51e-6, 1.5}
+               : half          ? Cost{2.22 + 0.0288 * n, padded * (n * 1.85e-6 + 5.0e-7), 2.71}
+                               : Cost{2.28 + 0.0255 * n, padded * (n * 1.94e-6 + 3.63e-6), 2.52};
     return kind == K_GEN64 ? Cost{2.9 + 0.0044 * n, m * n * 4.0e-6}
                            : Cost{3.0 + 0.021 * n, m * (n * 1.0e-6 + (half ? 1.4e-5 : 2.0e-5))};
 }
@@ -276,7 +288,7 @@ static void pick_groups(tftq_plan *p)
             }
             double best = HUGE_VAL;
             for (int lg = 1; lg <= most; lg++) {
-                const double t = std::max(cost[lg].latency, COST_BASE + least[0] - least[1] + cost[lg].work);
+                const double t = std::max(cost[lg].latency, cost[lg].start + least[0] - least[1] + cost[lg].work);
                 if (t >= best) continue;
                 best = t;
                 s.lg_groups = (uint8_t)lg;
@@ -291,7 +303,8 @@ static void pick_column_kinds(tftq_plan *p, int st, uint8_t blocks)
 {
     enum { NONE, LESS_WORK, ALL, N_WAYS };
     // per way: what is left to the teams, what goes to the blocks
-    Cost teams[N_WAYS] = {}, taken[N_WAYS] = {};
+    const Cost nothing = {0.0, 0.0, 0.0};
+    Cost teams[N_WAYS] = {nothing, nothing, nothing}, taken[N_WAYS] = {nothing, nothing, nothing};
     bool any[N_WAYS] = {}, others = false;
     for (const Seg &s : p->segs) {
         if (!stored_by_columns(s, st, p->esz)) {
@@ -302,23 +315,25 @@ static void pick_column_kinds(tftq_plan *p, int st, uint8_t blocks)
         for (int way = NONE; way < N_WAYS; way++) {
             const bool take = way == ALL || (way == LESS_WORK && b.work < t.work);
             Cost &sum = take ? taken[way] : teams[way];
-            sum.latency = std::max(sum.latency, take ? b.latency : t.latency);
-            sum.work += take ? b.work : t.work;
+            const Cost &c = take ? b : t;
+            sum = {std::max(sum.latency, c.latency), sum.work + c.work, std::max(sum.start, c.start)};
             any[way] = any[way] || take;
         }
     }
     int best = NONE;
     double least = HUGE_VAL;
     for (int way = NONE; way < N_WAYS; way++) {
-        auto launch = [&](double latency, double work) {
-            return others ? std::max(latency - COST_HIDDEN, work) : latency > 0.0 ? std::max(latency, COST_BASE + work) : 0.0;
+        auto launch = [&](const Cost &c) {
+            if (others) return std::max(c.latency - (st == ST_D ? COST_HIDDEN_D : COST_HIDDEN_Q), c.work);
+            return c.latency > 0.0 ? c.alone() : 0.0;
         };
+        const Cost &a = teams[way], &b = taken[way];
         double t;
         if (st == ST_D) {
-            t = launch(std::max(teams[way].latency, taken[way].latency), teams[way].work + taken[way].work);
+            t = launch({std::max(a.latency, b.latency), a.work + b.work});
         } else {
-            t = launch(teams[way].latency, teams[way].work);
-            if (any[way]) t += std::max(taken[way].latency, COST_BASE + taken[way].work) - (others ? COST_OVERLAP : 0.0);
+            t = launch(a);
+            if (any[way]) t += b.alone() - (others ? COST_OVERLAP : 0.0);
         }
         if (t < least) {
             least = t;
@@ -330,6 +345,34 @@ static void pick_column_kinds(tftq_plan *p, int st, uint8_t blocks)
         if (stored_by_columns(s, st, p->esz) &&
             (best == ALL || cost_of(s, blocks, st, p->esz, p->ws).work < cost_of(s, s.kind[st], st, p->esz, p->ws).work))
             s.kind[st] = blocks;
+}
+
+// Gives every block of a list 2 groups where the tensors' own choices would gain little.  Rows of more than
+// 4 steps run in a kernel of their own where all blocks of the list have 2 groups, 4 to 9 % sooner than in the
+// general one (us, 8 slots: [4096, 14336] beside [4096, 1024] in 2 and in 8 groups, bf16 64.2 and 68.8, fp32 114.6
+// and 125.3).  And a few small tensors are done sooner if none of them has blocks that live long: bf16
+// [231, 2922] and [803, 2922] 10.8 with their own, 10.2 in 2 groups, 8 slots, [251, 224], [2344, 672] and [248, 672]
+// 5.5 and 4.9, fp32 [181, 1573], [1620, 1573] and [162, 524] in one slot 8.1 and 6.7.
+static void pick_two_groups(tftq_plan *p)
+{
+    constexpr double LOSS = 0.07, LOSS_SMALL = 0.25, SMALL = 10.0;
+    double wide = 0.0;
+    int64_t blocks = 0;  // in 2 groups
+    Cost two = {0.0, 0.0, 0.0}, own = two;
+    for (const Seg &s : p->segs) {
+        if (s.kind[ST_Q] != K_COLS) continue;
+        const Cost a = cost_of_blocks(s, 1, p->esz, p->ws), b = cost_of_blocks(s, s.lg_groups, p->esz, p->ws);
+        two = {std::max(two.latency, a.latency), two.work + a.work, a.start};
+        own = {std::max(own.latency, b.latency), own.work + b.work, b.start};
+        if (s.lg_groups == 1 && tftq_qc_steps(s.n, 1) > 4) wide += a.work;
+        const int rows = tftq_qc_rows(1, p->esz);
+        blocks += (int64_t)p->ws * ((s.slice_rows + rows - 1) / rows);
+    }
+    // (in 16 bits only what the kernel for few blocks takes)
+    const bool small = p->nseg > 1 && (p->esz == 4 || blocks <= 256) && two.alone() < SMALL && two.alone() < (1.0 + LOSS_SMALL) * own.alone();
+    if (!small && (wide == 0.0 || two.work - own.work >= LOSS * wide)) return;
+    for (Seg &s : p->segs)
+        if (s.kind[ST_Q] == K_COLS) s.lg_groups = 1;
 }
 
 // Kinds for little work.  K_VECS gives a lane 8 vectors, in 2 to 8 rows one after the other, and K_COL1
@@ -605,8 +648,9 @@ extern "C" int tftq_plan_create(int dtype, int n_tensors, const int64_t *shapes,
         s.side = (uint8_t)tftq_reduce_rows_side(s.kind[ST_R], s.row_bytes / 4 - 1, s.slice_rows, p->ws);
     }
     pick_few_kinds(p);
-        pick_groups(p);
+    pick_groups(p);
     pick_column_kinds(p, ST_Q, K_COLS);
+    pick_two_groups(p);
     pick_column_kinds(p, ST_D, K_TILE);
     for (int i = 0; i < n_tensors; i++) {
         Seg &s = p->segs[(size_t)i];
