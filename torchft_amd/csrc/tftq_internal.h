@@ -79,6 +79,13 @@ TFTQ_HD static inline int tftq_qc_steps(int n, int lg_groups)
     const int step = 4 * TFTQ_QC_WG >> lg_groups;
     return (n + step - 1) / step;
 }
+// Whether blocks of 2^lg groups take rows of so many steps: the kernels have variants for these (quantize_cols_steps)
+// and pick_groups gives no others.  (Among 1.5 million lists of every size its costs chose no others where they
+// could: not 4 groups for rows of 5 to 8 of their steps, nor 32 for more than one.)
+TFTQ_HD constexpr bool tftq_qc_has(int lg_groups, int steps)
+{
+    return lg_groups == 1 || (lg_groups <= 4 && steps <= 4) || (lg_groups == 2 && steps > 8 && steps <= 12) || steps <= 1;
+}
 // K_TILE
 constexpr int TFTQ_TILE_ROWS = 64, TFTQ_TILE_COLS = 256;
 
@@ -329,6 +336,17 @@ struct tftq_plan {
     std::vector<uint8_t> blob;  // host image of the device table (nseg > TFTQ_N_INLINE)
     size_t static_bytes;        // what tftq_reduce_static writes of it: all but the index of quantize's second launch
 };
+
+// The kernel of quantize's second launch: one for any blocks, or, where all have 2 groups, one for few of them,
+// in 16 bits, or one for rows of more than 4 steps (the figures are at k_quantize_cols_two).
+enum QcKernel { QC_ANY_4, QC_ANY_12, QC_TWO_4, QC_TWO_8, QC_TWO_12 };  // and the steps that stay in registers
+static inline QcKernel tftq_qc_kernel(const tftq_plan &p)
+{
+    const int most = p.cols_most, few = most > 4 ? 48 : most > 2 ? 192 : 256;
+    if (p.cols_two && p.esz == 2 && most <= 8 && p.nwg[ST_QC] <= few) return most > 4 ? QC_TWO_8 : QC_TWO_4;
+    if (most <= 4) return QC_ANY_4;
+    return p.cols_two ? QC_TWO_12 : QC_ANY_12;
+}
 
 // ---------------------------------------------------------------------------
 // kernel arguments

@@ -259,10 +259,10 @@ static bool stored_by_columns(const Seg &s, int st, int esz)
 }
 
 // How many groups of rows a block of quantize holds (Seg::lg_groups).  More make whole lines of what it
-// reads and fewer blocks, and fewer columns per step: rows of more than 12 steps keep 2 groups, more than 4
-// groups are for rows of up to 4 steps, and more than 4 steps (a workgroup per compute unit) for tensors
-// of 192 blocks: fp32 [1797, 3500] 10.4 us in 2 groups, 14.1 in 120 blocks of 4.  A tensor takes the groups that are the least work, or, if the launch
-// has little else to do, those that are done soonest.  us in 2 / 4 / 8 / 16 / 32 groups, bf16, 8 slots:
+// reads and fewer blocks, and fewer columns per step (tftq_qc_has); more than 4 steps of more than 2
+// groups (a workgroup per compute unit) are for tensors of 192 blocks: bf16 [5682, 4287] in 16 slots, say.  A
+// tensor takes the groups that are the least work, or, if the launch has little else to do, those that are
+// done soonest.  us in 2 / 4 / 8 / 16 / 32 groups, bf16, 8 slots:
 // [2330168, 18] 920 / 458 / 232 / 126 / 65, [42799, 147] 18.5 / 11.0 / 8.0 / 7.0 / 8.1, [3495, 300] 4.7 / 4.6 / 5.8 /
 // 8.3 / -, [41943, 1000] 30.4 / 25.1 / 21.9 / - / -, [1048, 1000] 5.1 / 6.3 / 9.0 / - / -, [11983, 3500] 28.9 / 34.0 / - / -
 // / -, fp32 63.6 / 51.6.
@@ -274,7 +274,7 @@ static void pick_groups(tftq_plan *p)
             if (!stored_by_columns(s, ST_Q, p->esz)) continue;
             Cost cost[6];
             int most = 1;
-            for (int lg = 1; lg <= 5 && (lg == 1 || tftq_qc_steps(s.n, lg) <= (lg == 2 ? 12 : 4)); lg++) {
+            for (int lg = 1; lg <= 5 && tftq_qc_has(lg, tftq_qc_steps(s.n, lg)); lg++) {
                 const int rows = tftq_qc_rows(lg, p->esz);
                 if (lg > 1 && tftq_qc_steps(s.n, lg) > 4 && (int64_t)p->ws * ((s.slice_rows + rows - 1) / rows) < 192) break;
                 cost[lg] = cost_of_blocks(s, lg, p->esz, p->ws);

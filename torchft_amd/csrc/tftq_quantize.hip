@@ -791,31 +791,34 @@ DEV void quantize_cols(const Seg &s, const KCall &p, int blk, int tid, uint8_t *
 }
 
 // Steps that stay in registers: 12 for lists with rows of more than 4 steps (250 registers, two
-// wavefronts per SIMD; 14 spill), else 4 (115 registers, four).  More than 4 groups take no more than 4
-// steps (pick_groups).
+// wavefronts per SIMD; 14 spill), else 4 (115 registers, four).
 constexpr int QC_MOST = 12;
-// The stage: all packed rows of a block of up to 4 steps, or 8 (fp32, 4 groups: 12).  2 groups do without in
-// fp32 ([41943, 1000] 75 us straight from the registers and 77 through the stage) and beside rows of more than 4
-// steps (bf16 [4096, 8192], [8192, 4096] and [4096, 1024] in one list, 4 slots, 73.6 us through the stage and 70.3).
+// The stage: all packed rows of a block of up to 4 steps, in fp32 also those of 12 steps of 4 groups.  2 groups do
+// without in fp32 ([41943, 1000] 75 us straight from the registers and 77 through the stage) and beside rows of more
+// than 4 steps (bf16 [4096, 8192], [8192, 4096] and [4096, 1024] in one list, 4 slots, 73.6 us through the stage and 70.3).
 template <typename T, int NSMAX>
 struct ColsStage {
-    static constexpr int VECTORS = NSMAX == 4 ? 4 : Elem<T>::ESZ == 4 ? NSMAX : 8;
+    static constexpr int VECTORS = Elem<T>::ESZ == 4 ? NSMAX : 4;
     static constexpr int BYTES = TFTQ_QC_WG * 4 * VECTORS * Elem<T>::EPV + 32 * Elem<T>::EPV * 4 + 128;
 };
 constexpr int QC_LEAST_STAGE = 4096;  // for the maxima of up to 4 groups alone
+// The variants that tftq_qc_has names.
 template <typename T, int G, int NSMAX>
 DEV void quantize_cols_steps(const Seg &s, const KCall &p, int blk, int tid, uint8_t *stage, float *scale)
 {
-    constexpr int STAGE = ColsStage<T, NSMAX>::BYTES;
+    constexpr int STAGE = ColsStage<T, NSMAX>::BYTES, LG = __builtin_ctz(G);
     constexpr bool DIRECT = G == 2 && (Elem<T>::ESZ == 4 || NSMAX > 4);
-    const int steps = tftq_qc_steps(s.n, __builtin_ctz(G));  // same for the whole workgroup
+    const int steps = tftq_qc_steps(s.n, LG);  // same for the whole workgroup
     constexpr int SHORT = DIRECT ? QC_LEAST_STAGE : STAGE;
-    if (steps <= 1) quantize_cols<T, G, 1, SHORT>(s, p, blk, tid, stage, scale);
-    else if (steps <= 2) quantize_cols<T, G, 2, SHORT>(s, p, blk, tid, stage, scale);
-    else if (NSMAX == 4 || steps <= 4) quantize_cols<T, G, 4, SHORT>(s, p, blk, tid, stage, scale);
-    else if constexpr (NSMAX > 4) {
-        if (steps <= 8) quantize_cols<T, G, 8, SHORT>(s, p, blk, tid, stage, scale);
-        else quantize_cols<T, G, NSMAX, Elem<T>::ESZ == 4 && G == 4 ? STAGE : QC_LEAST_STAGE>(s, p, blk, tid, stage, scale);
+    if (!tftq_qc_has(LG, 2) || steps <= 1) quantize_cols<T, G, 1, SHORT>(s, p, blk, tid, stage, scale);
+    else if constexpr (tftq_qc_has(LG, 2)) {
+        if (steps <= 2) quantize_cols<T, G, 2, SHORT>(s, p, blk, tid, stage, scale);
+        else if (NSMAX == 4 || !tftq_qc_has(LG, 12) || steps <= 4) quantize_cols<T, G, 4, SHORT>(s, p, blk, tid, stage, scale);
+        else if constexpr (NSMAX > 4 && tftq_qc_has(LG, 12)) {
+            constexpr bool EIGHT = tftq_qc_has(LG, 8);
+            if (EIGHT && steps <= 8) quantize_cols<T, G, EIGHT ? 8 : NSMAX, SHORT>(s, p, blk, tid, stage, scale);
+            else quantize_cols<T, G, NSMAX, Elem<T>::ESZ == 4 && G == 4 ? STAGE : QC_LEAST_STAGE>(s, p, blk, tid, stage, scale);
+        }
     }
 }
 template <typename T, int NSMAX, typename A>
@@ -895,20 +898,28 @@ static int launch_qc(const tftq_plan *plan, const KArgs &ka, hipStream_t st)
 {
     return with_args(ka, [&](const auto &args) {
         typedef typename std::decay<decltype(args)>::type A;
-        // kernels of 2 groups: for rows of up to QC_MOST steps, and for few blocks in 16 bits
-        // (the figures at k_quantize_cols_two)
-        constexpr bool HALF = Elem<T>::ESZ == 2;
-        constexpr int FEW8 = HALF ? 8 : QC_MOST, FEW4 = HALF ? 4 : QC_MOST;
-        const int most = plan->cols_most, blocks = plan->nwg[ST_QC];
-        const bool two = plan->cols_two, few = HALF && two && blocks <= (most > 4 ? 48 : most > 2 ? 192 : 256) && most <= 8;
-        if constexpr (std::is_same<A, KOne>::value)
-            return launch_kernel(few && most <= 4 ? k_quantize_cols_two_one<T, FEW4> : few ? k_quantize_cols_two_one<T, FEW8>
-                                 : two && most > 4 ? k_quantize_cols_two_one<T, QC_MOST>
-                                 : most > 4 ? k_quantize_cols_one<T, QC_MOST> : k_quantize_cols_one<T, 4>, ka, args, 0, st, TFTQ_QC_WG);
-        else
-            return launch_kernel(few && most <= 4 ? k_quantize_cols_two<T, A, FEW4> : few ? k_quantize_cols_two<T, A, FEW8>
-                                 : two && most > 4 ? k_quantize_cols_two<T, A, QC_MOST>
-                                 : most > 4 ? k_quantize_cols<T, A, QC_MOST> : k_quantize_cols<T, A, 4>, ka, args, 0, st, TFTQ_QC_WG);
+        constexpr int FEW8 = Elem<T>::ESZ == 2 ? 8 : QC_MOST, FEW4 = Elem<T>::ESZ == 2 ? 4 : QC_MOST;  // (16 bits only)
+        if constexpr (std::is_same<A, KOne>::value) {
+            auto kernel = k_quantize_cols_one<T, 4>;
+            switch (tftq_qc_kernel(*plan)) {
+            case QC_ANY_4: break;
+            case QC_ANY_12: kernel = k_quantize_cols_one<T, QC_MOST>; break;
+            case QC_TWO_4: kernel = k_quantize_cols_two_one<T, FEW4>; break;
+            case QC_TWO_8: kernel = k_quantize_cols_two_one<T, FEW8>; break;
+            case QC_TWO_12: kernel = k_quantize_cols_two_one<T, QC_MOST>; break;
+            }
+            return launch_kernel(kernel, ka, args, 0, st, TFTQ_QC_WG);
+        } else {
+            auto kernel = k_quantize_cols<T, A, 4>;
+            switch (tftq_qc_kernel(*plan)) {
+            case QC_ANY_4: break;
+            case QC_ANY_12: kernel = k_quantize_cols<T, A, QC_MOST>; break;
+            case QC_TWO_4: kernel = k_quantize_cols_two<T, A, FEW4>; break;
+            case QC_TWO_8: kernel = k_quantize_cols_two<T, A, FEW8>; break;
+            case QC_TWO_12: kernel = k_quantize_cols_two<T, A, QC_MOST>; break;
+            }
+            return launch_kernel(kernel, ka, args, 0, st, TFTQ_QC_WG);
+        }
     });
 }
 
